@@ -109,7 +109,7 @@ template <int D, bool F32 = false, int DA = D>
 __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid_attn_bwd_dkdv_kernel(
     const bf16* __restrict__ q, Strides qs, const bf16* __restrict__ k, Strides ks, const bf16* __restrict__ vpb,
     const bf16* __restrict__ dout, Strides dos, const bf16* __restrict__ seeds, float* __restrict__ dvp, float* __restrict__ dka, int Hq, int Hkv, int T, int BH, float scale, Lo lo,
-    const bf16* __restrict__ vpbl) {
+    const bf16* __restrict__ vpbl, int nsplit, float* __restrict__ part) {
   static_assert(!F32 || D == 64 || D == 128, "fp32 inputs: head dim 64 or 128");
   constexpr int NDT = D / 32;
   constexpr int NKS = D / 16;
@@ -120,7 +120,8 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
   __shared__ __attribute__((aligned(16))) DkdvSmem<D, F32> sm;
   constexpr int NB = stage_bufs(D, F32);
   const int id = blockIdx.x;
-  const int jb = id / BH, bh = id - (id / BH) * BH;
+  const int jb = id / (BH * nsplit), rem = id - jb * (BH * nsplit);
+  const int sp = rem / BH, bh = rem - sp * BH;
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int G = Hq / Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -149,7 +150,10 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
   const int nt64 = T / 64;
   const int it_first = jb * 2;            // first query tile any wave needs
   const int ntile = nt64 - it_first;      // query tiles per query head
-  const int nsteps = G * ntile;           // step s: query head s / ntile, tile it_first + s % ntile
+  // step s of a column block: query head s / ntile, tile it_first + s % ntile; this
+  // workgroup's share is the steps s0 .. s0 + nsteps - 1
+  const int s0 = (int)((int64_t)G * ntile * sp / nsplit);
+  const int nsteps = (int)((int64_t)G * ntile * (sp + 1) / nsplit) - s0;
   const int it_w = jw / 64;               // this wave's diagonal tile
   const int kloc = jw - it_w * 64 + l32;  // this lane's key inside its diagonal tile
   int plan_q[64 * (D / 8) / 256], plan_o[64 * (D / 8) / 256];
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
   dma_plan<64, D / 8, 256, SW>(qs.t, plan_q);
   dma_plan<64, D / 8, 256, SW>(dos.t, plan_o);
   auto stage = [&](int s) {
-    const int gi = s / ntile, it = it_first + s - gi * ntile, buf = s % NB;
+    const int gi = (s0 + s) / ntile, it = it_first + s0 + s - gi * ntile, buf = s % NB;
     const int hq = h * G + gi, bhq = b * Hq + hq, i0 = it * 64;
     if (w < 2) dma_1k(seeds + ((int64_t)bhq * T + i0 + 32 * w) * 16, &sm.seed[buf][32 * w][0]);  // 2 KB of seed rows
     dma_stage<64, D / 8>(plan_q, q + b * qs.b + hq * qs.h + (int64_t)i0 * qs.t, sm.q[buf]);
@@ -169,7 +173,7 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
       dma_stage<64, D / 8>(plan_o, lo.dout + b * dos.b + hq * dos.h + (int64_t)i0 * dos.t, sm.dOl[buf]);
     }
   };
-  stage(0);
+  if (nsteps > 0) stage(0);
   if (NB == 3 && nsteps > 1) {
     stage(1);
     dma_wait_but<STAGE_OPS>();
@@ -275,7 +279,7 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
   // step s works on buffer s % NB: the loop is unrolled by NB so that it is a constant
   auto step = [&](auto bufc, const int s) __attribute__((always_inline)) {
     if (s + NB - 1 < nsteps) stage(s + NB - 1);
-    const int it = it_first + s % ntile;
+    const int it = it_first + (s0 + s) % ntile;
     if (it > it_w) tile(bufc, false);
     else if (it == it_w) tile(bufc, true);
     if (NB == 3 && s + 2 < nsteps) dma_wait_but<STAGE_OPS>();  // the step after next may stay in flight
@@ -289,8 +293,10 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
       if (s + 2 < nsteps) step(std::integral_constant<int, 2>{}, s + 2);
     }
   }
-  float* ov = dvp + ((int64_t)bh * T + jrow) * D;
-  float* ok = dka + ((int64_t)bh * T + jrow) * D;
+  // the first share of a block writes dV' and dK themselves, the others their partial sums
+  const int64_t nel = (int64_t)BH * T * D;
+  float* ov = (sp == 0 ? dvp : part + (int64_t)(2 * sp - 2) * nel) + ((int64_t)bh * T + jrow) * D;
+  float* ok = (sp == 0 ? dka : part + (int64_t)(2 * sp - 1) * nel) + ((int64_t)bh * T + jrow) * D;
 #pragma unroll
   for (int t = 0; t < NDT; ++t)
 #pragma unroll
@@ -304,6 +310,19 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
       *reinterpret_cast<f32x4*>(ov + t * 32 + 8 * qq + 4 * g) = a;
       *reinterpret_cast<f32x4*>(ok + t * 32 + 8 * qq + 4 * g) = bq;
     }
+}
+
+// dV' and dK of a split column sweep: dvp += the shares' partial dV', dka += their dK, in
+// the order of the shares (deterministic).  n4: float4 elements of one tensor.
+__global__ __launch_bounds__(256) void lucid_dkdv_sum_kernel(float* __restrict__ dvp, float* __restrict__ dka,
+                                                             const float* __restrict__ part, int nsplit, int64_t n4) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  float* dst = blockIdx.y ? dka : dvp;
+  f32x4 x = reinterpret_cast<const f32x4*>(dst)[i];
+  for (int sp = 1; sp < nsplit; ++sp)
+    x += reinterpret_cast<const f32x4*>(part)[(2 * sp - 2 + (int64_t)blockIdx.y) * n4 + i];
+  reinterpret_cast<f32x4*>(dst)[i] = x;
 }
 
 // ---------------------------------------------------------------------------

@@ -138,8 +138,25 @@ struct BwdWs {
   float* colsum; // [BH][T][D]   sum_I M_IJ^T K^_I
   int* counters; // [BH]
   bf16 *doh, *dol; // fp32 inputs only: the bf16 pair of dO ([BHq][T][D] rows)
+  float* dkdv;   // [2 (dkdv_splits - 1)][BH][T][D] partial dV' and dK of a split column sweep
   size_t bytes;
 };
+
+// Shares that the dK/dV' sweep of a 128-key column block is cut into.  The blocks of a
+// causal sweep are as long as G (T - key) / 64 steps, so a launch of at most one block per
+// resident workgroup takes as long as the longest block, twice the mean; with twice as many
+// workgroups as slots (two per CU for bf16 at 64 columns, else one), longest first, the
+// slots finish together.  A share keeps at least eight 64-row steps in the longest block, so
+// that its start and its partial sums stay small beside its sweep.  B1 Hq32 Hkv4 T16000 d64
+// (500 blocks on 512 slots): 3.92 ms in one share, 2.58 in two, 2.52 in three (with the
+// sum of the partials, 0.02), 2.48 in eight; B1 Hq32 Hkv8 T8192 d128 (512 blocks on 256 slots)
+// 1.57 ms in one, 1.58 in two, 1.72 in eight.
+int dkdv_splits(int BH, int G, int T, int D, bool f32) {
+  const int64_t jobs = (int64_t)BH * (T / 128), slots = padded_dim(D) == 64 && !f32 ? 512 : 256;
+  const int64_t want = (2 * slots + jobs - 1) / jobs, most = (int64_t)G * (T / 64) / 8;
+  const int64_t ns = want < most ? want : most;
+  return ns < 1 ? 1 : ns < 8 ? (int)ns : 8;
+}
 
 BwdWs carve_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = false) {
   D = padded_dim(D);
@@ -164,6 +181,7 @@ BwdWs carve_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = fal
     w.doh = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
     w.dol = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
   }
+  w.dkdv = reinterpret_cast<float*>(take((dkdv_splits(B * Hkv, Hq / Hkv, T, D, f32) - 1) * 2 * BH * T * D * 4));
   w.bytes = off;
   return w;
 }
@@ -322,11 +340,16 @@ int launch_attn_bwd(const void* dout, const int64_t* dos, const void* q, const i
   // registers).  DA: the active head-dim columns (zero-padded rows of a smaller head dim)
   constexpr int RW = D == 128 ? 32 : 64;
   constexpr int XWGR = D == 128 ? 128 : 256;
+  const int nsp = dkdv_splits(BH, Hq / Hkv, T, D, false);
   auto sweeps = [&](auto dac) -> int {
     constexpr int DA = decltype(dac)::value;
     LUCID_LAUNCH("lucid_attn_bwd_dkdv_kernel", (lucid::lucid_attn_bwd_dkdv_kernel<D, false, DA>),
-                 dim3((T / 128) * BH), st, (const bf16*)q, S(qs), (const bf16*)k, S(ks), f.vpb, (const bf16*)dout,
-                 S(dos), w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH, scale, lucid::Lo{}, nullptr);
+                 dim3((T / 128) * BH * nsp), st, (const bf16*)q, S(qs), (const bf16*)k, S(ks), f.vpb,
+                 (const bf16*)dout, S(dos), w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH, scale, lucid::Lo{}, nullptr, nsp,
+                 w.dkdv);
+    if (nsp > 1)
+      LUCID_LAUNCH("lucid_dkdv_sum_kernel", lucid::lucid_dkdv_sum_kernel, dim3(((int64_t)BH * T * D / 4 + 255) / 256, 2),
+                   st, w.dvp, w.dka, w.dkdv, nsp, (int64_t)BH * T * D / 4);
     LUCID_LAUNCH_B("lucid_attn_bwd_dq_kernel", (lucid::lucid_attn_bwd_dq_kernel<D, false, false, RW, 256, DA>),
                    dim3(((T + 255) / 256) * BHq), dim3(64 * (256 / RW)), st, (const bf16*)q, S(qs), (const bf16*)k,
                    S(ks), f.vpb, (const bf16*)dout, S(dos), lse, w.delta, f.mass, (bf16*)dq, S(dqs), Hq, Hkv, T, BHq,
@@ -463,6 +486,7 @@ BwdWs carve_seam_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool attn
       w.doh = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
       w.dol = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
     }
+    w.dkdv = reinterpret_cast<float*>(take((dkdv_splits(B * Hkv, Hq / Hkv, T, D, f32) - 1) * 2 * BH * T * D * 4));
   } else {
     w.dvb = reinterpret_cast<bf16*>(take(BH * T * D * 2));
     w.dvbl = reinterpret_cast<bf16*>(take(BH * T * D * 2));
@@ -648,12 +672,14 @@ int launch_attn_bwd_f32(const void* dout, const int64_t* dos, const void* o, con
   // head dim 128: four waves of 32 rows for dQ (128 rows per workgroup, one wave per SIMD),
   // so that the hi/lo operands of a wave stay in registers
   constexpr int RW = D == 128 ? 32 : 64, WGR = D == 128 ? 128 : 256;
-  const dim3 gkv((T / 128) * BH), gq(((T + WGR - 1) / WGR) * BHq), bq(64 * (WGR / RW));
+  const int nsp = dkdv_splits(BH, Hq / Hkv, T, D, true);
+  const dim3 gsum(((int64_t)BH * T * D / 4 + 255) / 256, 2), gkv((T / 128) * BH * nsp), gq(((T + WGR - 1) / WGR) * BHq), bq(64 * (WGR / RW));
   if constexpr (D == 128) {
     const int da = active_dims<D>(dn);
 #define LUCID_ATTN_BWD_NARROW(DA)                                                                                   \
   LUCID_LAUNCH("lucid_attn_bwd_dkdv_f32_kernel", (lucid::lucid_attn_bwd_dkdv_kernel<D, true, DA>), gkv, st, f.qh,  \
-               cq, f.kch, ck, f.vpb, w.doh, cq, w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH, scale, lo, f.vpbl);          \
+               cq, f.kch, ck, f.vpb, w.doh, cq, w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH, scale, lo, f.vpbl, nsp, w.dkdv); \
+  if (nsp > 1) LUCID_LAUNCH("lucid_dkdv_sum_kernel", lucid::lucid_dkdv_sum_kernel, gsum, st, w.dvp, w.dka, w.dkdv, nsp, (int64_t)BH * T * D / 4); \
   LUCID_LAUNCH_B("lucid_attn_bwd_dq_f32_kernel", (lucid::lucid_attn_bwd_dq_kernel<D, true, true, RW, WGR, DA>), gq, \
                  bq, st, f.qh, cq, f.kch, ck, f.vpb, w.doh, cq, lse, w.delta, f.mass, (float*)dq, S(dqs), Hq, Hkv, T,  \
                  BHq, scale, lo, f.vpbl)
@@ -668,7 +694,10 @@ int launch_attn_bwd_f32(const void* dout, const int64_t* dos, const void* o, con
 #undef LUCID_ATTN_BWD_NARROW
   }
   LUCID_LAUNCH("lucid_attn_bwd_dkdv_f32_kernel", (lucid::lucid_attn_bwd_dkdv_kernel<D, true>), gkv, st, f.qh, cq,
-               f.kch, ck, f.vpb, w.doh, cq, w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH, scale, lo, f.vpbl);
+               f.kch, ck, f.vpb, w.doh, cq, w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH, scale, lo, f.vpbl, nsp, w.dkdv);
+  if (nsp > 1)
+    LUCID_LAUNCH("lucid_dkdv_sum_kernel", lucid::lucid_dkdv_sum_kernel, gsum, st, w.dvp, w.dka, w.dkdv, nsp,
+                 (int64_t)BH * T * D / 4);
   LUCID_LAUNCH_B("lucid_attn_bwd_dq_f32_kernel", (lucid::lucid_attn_bwd_dq_kernel<D, true, true, RW, WGR>), gq, bq,
                  st, f.qh, cq, f.kch, ck, f.vpb, w.doh, cq, lse, w.delta, f.mass, (float*)dq, S(dqs), Hq, Hkv, T,
                  BHq, scale, lo, f.vpbl);
