@@ -339,7 +339,10 @@ __global__ __launch_bounds__(256) void lucid_dkdv_sum_kernel(float* __restrict__
 // shared key direction cancels out of dQ_i = s sum_j dS_ij K_j and the bf16 rounding of
 // dS would leave it behind; dS enters as a hi/lo pair (K is exact in bf16).  dP = dO V'^T
 // keeps the bf16 V' of the forward: delta_i = dO_i . O_i equals sum_j P_ij dP_ij only when
-// both use the same V', and that identity is what cancels the shared direction.
+// both use the same V', and that identity is what cancels the shared direction.  The exact
+// bf16 instances run waves of 32 rows: at head dim 64 that is two waves per SIMD where 64-row
+// waves took 392 registers and one (16 exact heads of T = 16000: 2.94 -> 2.35 ms, and with
+// the step loop unrolled as below 2.13).
 // ---------------------------------------------------------------------------
 template <int D>
 struct DqSmem {
@@ -359,7 +362,7 @@ struct DqSmemF32 {  // fp32 inputs: the lo tiles of K and V' beside the hi tiles
 // operands need one wave per SIMD to stay in registers)
 // DA: the head-dim columns that can be nonzero (as in lucid_attn_bwd_dkdv_kernel)
 template <int D, bool EXACT, bool F32 = false, int RW = 64, int WGR = 256, int DA = D>
-__global__ __launch_bounds__(64 * (WGR / RW)) LUCID_TWO_WAVES_IF((D == 64 || RW == 32) && !EXACT) void lucid_attn_bwd_dq_kernel(
+__global__ __launch_bounds__(64 * (WGR / RW)) LUCID_TWO_WAVES_IF(EXACT ? D == 64 && RW == 32 && !F32 : D == 64 || RW == 32) void lucid_attn_bwd_dq_kernel(
     const bf16* __restrict__ q, Strides qs, const bf16* __restrict__ k, Strides ks, const bf16* __restrict__ vpb,
     const bf16* __restrict__ dout, Strides dos, const float* __restrict__ lse,
     const float* __restrict__ delta, const float* __restrict__ mass,
@@ -529,7 +532,7 @@ __global__ __launch_bounds__(64 * (WGR / RW)) LUCID_TWO_WAVES_IF((D == 64 || RW 
     else dma_wait();
     __syncthreads();
   };
-  if constexpr (EXACT) {  // the exact instances keep the rolled loop (registers)
+  if constexpr (EXACT && (F32 || D != 64)) {  // these exact instances keep the rolled loop (registers)
     for (int jt = 0; jt < ntile; ++jt) {
       const int buf = jt % NB;
       if (jt + NB - 1 < ntile) stage(jt + NB - 1);
@@ -542,7 +545,7 @@ __global__ __launch_bounds__(64 * (WGR / RW)) LUCID_TWO_WAVES_IF((D == 64 || RW 
       __syncthreads();
     }
   } else {
-    static_assert(EXACT || NB == 3, "the bf16 instances stage three deep");
+    static_assert(NB == 3, "the unrolled instances stage three deep");
     for (int jt = 0; jt < ntile; jt += 3) {
       step(std::integral_constant<int, 0>{}, jt);
       if (jt + 1 < ntile) step(std::integral_constant<int, 1>{}, jt + 1);
@@ -1359,7 +1362,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void l
 // EXACT (heads whose row mass exceeds kExactMass; each instance returns at once for the
 // other heads): the exponents come from raw K tiles times fp32 factors r_I r_J, and
 // G = V' dV^T and M K are split into hi*hi + hi*lo + lo*hi with the lo parts of V'
-// (staged beside V') and dV (held beside dV); one workgroup per CU.
+// (staged beside V') and dV (held beside dV); one 32-row n-tile per wave, which at head dim
+// 64 fits two workgroups per CU (2 exact heads of T = 16000: 0.79 ms with two n-tiles and one
+// workgroup, 0.55 ms).
 // ---------------------------------------------------------------------------
 template <int D, bool EXACT, bool F32 = false>
 struct ProwSmem {
@@ -1379,7 +1384,7 @@ struct ProwSmem<D, true, F32> {
 // NT: 32-row n-tiles per wave (2: 256 rows per workgroup; 1: 128 rows, for the fp32 instance
 // at head dim 128, whose hi/lo row operands of two n-tiles do not fit the registers)
 template <int D, bool EXACT, bool F32 = false, int NT = 2>
-__global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void lucid_precond_bwd_row_kernel(
+__global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && (!EXACT || (NT == 1 && !F32))) void lucid_precond_bwd_row_kernel(
     const bf16* __restrict__ k, Strides ks, int Hkv, int T, int BH, const float* __restrict__ rinv,
     const bf16* __restrict__ khat, float scale, float dn, const bf16* __restrict__ vpb,
     const bf16* __restrict__ vpbl, const bf16* __restrict__ dvb,

@@ -336,8 +336,8 @@ int launch_attn_bwd(const void* dout, const int64_t* dos, const void* q, const i
                S(dos), (const bf16*)o, S(os), f.olo, f.mass, Hq, Hkv, T, w.delta, w.counters, BH, lucid::Lo{}, lse,
                cinv, w.seeds);
   // dQ: four waves of 64 rows at head dim 64, eight waves of 32 rows at 128; the exact
-  // instance at 128: 128 rows per workgroup, one wave per SIMD (its hi/lo operands need the
-  // registers).  DA: the active head-dim columns (zero-padded rows of a smaller head dim)
+  // instances: waves of 32 rows (at 128, 128 rows per workgroup, one wave per SIMD: its hi/lo
+  // operands need the registers).  DA: the active head-dim columns (zero-padded rows of a smaller head dim)
   constexpr int RW = D == 128 ? 32 : 64;
   constexpr int XWGR = D == 128 ? 128 : 256;
   const int nsp = dkdv_splits(BH, Hq / Hkv, T, D, false);
@@ -354,8 +354,8 @@ int launch_attn_bwd(const void* dout, const int64_t* dos, const void* q, const i
                    dim3(((T + 255) / 256) * BHq), dim3(64 * (256 / RW)), st, (const bf16*)q, S(qs), (const bf16*)k,
                    S(ks), f.vpb, (const bf16*)dout, S(dos), lse, w.delta, f.mass, (bf16*)dq, S(dqs), Hq, Hkv, T, BHq,
                    scale, lucid::Lo{}, nullptr);
-    LUCID_LAUNCH_B("lucid_attn_bwd_dq_exact_kernel", (lucid::lucid_attn_bwd_dq_kernel<D, true, false, RW, XWGR, DA>),
-                   dim3(((T + XWGR - 1) / XWGR) * BHq), dim3(64 * (XWGR / RW)), st, (const bf16*)q, S(qs),
+    LUCID_LAUNCH_B("lucid_attn_bwd_dq_exact_kernel", (lucid::lucid_attn_bwd_dq_kernel<D, true, false, 32, XWGR, DA>),
+                   dim3(((T + XWGR - 1) / XWGR) * BHq), dim3(64 * (XWGR / 32)), st, (const bf16*)q, S(qs),
                    (const bf16*)k, S(ks), f.vpb, (const bf16*)dout, S(dos), lse, w.delta, f.mass, (bf16*)dq, S(dqs),
                    Hq, Hkv, T, BHq, scale, lucid::Lo{}, nullptr);
     return LUCID_OK;
@@ -410,9 +410,9 @@ int launch_precond_bwd(const void* k, const int64_t* ks, const FwdWs& f, void* d
   LUCID_LAUNCH("lucid_precond_bwd_row_kernel", (lucid::lucid_precond_bwd_row_kernel<D, false>),
                dim3(((T + 255) / 256) * BH), st, (const bf16*)k, S(ks), Hkv, T, BH, f.rinv, f.khat, scale, dn,
                f.vpb, f.vpbl, w.dvb, w.dvbl, f.mass, w.colsum, dka, (bf16*)dk, S(dks), lucid::Lo{});
-  // the exact instance at head dim 128: one n-tile per wave (128 rows per workgroup), so that
-  // its hi/lo row operands stay in registers
-  constexpr int XNT = D == 128 ? 1 : 2;
+  // the exact instance: one n-tile per wave (128 rows per workgroup), so that its hi/lo row
+  // operands stay in registers
+  constexpr int XNT = 1;
   LUCID_LAUNCH("lucid_precond_bwd_row_exact_kernel", (lucid::lucid_precond_bwd_row_kernel<D, true, false, XNT>),
                dim3(((T + 128 * XNT - 1) / (128 * XNT)) * BH), st, (const bf16*)k, S(ks), Hkv, T, BH, f.rinv, f.khat,
                scale, dn, f.vpb, f.vpbl, w.dvb, w.dvbl, f.mass, w.colsum, dka, (bf16*)dk, S(dks), lucid::Lo{});
