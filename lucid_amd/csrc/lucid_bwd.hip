@@ -579,7 +579,7 @@ __global__ __launch_bounds__(64 * (WGR / RW)) LUCID_TWO_WAVES_IF(EXACT ? D == 64
 // ---------------------------------------------------------------------------
 // Chained transposed solve dV = P^-T dV' (Lucid_Tril_Solver.backward :328-334)
 // and the column sums C_J = sum_{I >= J} M_IJ^T K^_I, M = (dV V'^T) * P.
-// Workgroup = 128 columns: sub-blocks A = J0..J0+63 and B = J0+64..J0+127.
+// Workgroup = 128 columns J0 .. J0+127 (block p).
 // id -> (p = NP-1 - id/BH, bh = id % BH): ids grow as p falls, so a workgroup
 // waits only on later blocks held by lower ids.  counters[bh] = n means the
 // last n 64-blocks of dV are published.
@@ -594,55 +594,49 @@ __global__ __launch_bounds__(64 * (WGR / RW)) LUCID_TWO_WAVES_IF(EXACT ? D == 64
 // (acc starts at -dV'^T).  Only the swept rows' K^ is rounded to bf16: its rounding
 // differs from row to row, so it does not add up over the sums over I, while the
 // column's own key stays exact (scaled by r_J in fp32).  The EXACT instance stages raw
-// K rows and 1/rms instead and scales by r_I r_J in fp32.  Then dV_B = X_B^T R_B, dV_A = X_A^T (R_A - P_BA^T dV_B),
-// R = dV' - acc, and the diagonal-block terms of C.  The chain's critical path
-// is the work after the last tile becomes visible, so dV' and both inverses
-// are loaded earlier.  At
+// K rows and 1/rms instead and scales by r_I r_J in fp32.  Then, with R = dV' - acc,
+//   dV_p = X^T R + link dV_{p+1}  (X^T, link = -X^T P_{p+1,p}^T: lucid_link_kernel),
+// X^T and R as 3-term splits.  Between the next block's publish and this one's stand the wait,
+// staging 16 KB of dV, one 128-deep product, the store and the counter.  Block p + 2's rows enter R by P^T dV
+// alone, their P taken while they are being solved; the column-sum terms of blocks p + 1 and
+// p + 2 and of the block itself follow the publish.  2 heads of T = 16000 at d = 64: 1.24 ms
+// with every later tile swept and the two sub-blocks solved in turn (10 us a hand-off), 0.63
+// with links, 0.50 with block p + 2 taken apart (4 us); exact 1.59 -> 1.02 ms; 8 heads of
+// T = 8192 at d = 128 1.05 -> 0.57 ms.  At
 // d = 64 two workgroups share a CU (LDS <= 80 KB, <= 256 registers per lane).
 //
 // EXACT (heads whose row mass exceeds kExactMass; each instance returns at once for the
 // other heads): dV is also kept as its bf16 residual (dvbl), the staged row tiles carry
 // it, V'_J's residual (vpbl) is held beside V'_J, and every product that sums over rows
 // is split into hi*hi + hi*lo + lo*hi: P^T dV, G = dV V'^T, M^T K (K is exact in bf16,
-// so two terms) and the in-block P_BA^T dV_B.  One workgroup per CU.
+// so two terms) and link dV_{p+1}.  One workgroup per CU.
 // F32 (fp32 inputs, exact, head dim 64): K also comes as hi + lo (the lo row tiles staged
 // beside the others, K_J's lo part in registers, K^T's lo copy ktl), so every product with
 // K takes three terms as well (four for the K.K of P); dV is written in fp32.
 // ---------------------------------------------------------------------------
 template <int D, bool EXACT, bool F32 = false>
-struct PcolSmem;
-template <int D>
-struct PcolSmem<D, false, false> {
-  union {
-    struct {
-      bf16 k[3][64 * D];   // swizzled tiles (chunk c of row r at c ^ (r & 7))
-      bf16 dv[3][64 * D];
-      float r[3][64];
-    } st;
-    struct {
-      float Rt[D][132];     // R^T for the 128 columns (0..63 = A, 64..127 = B), reductions
-      float Xt[64][68];     // Xt[c][r] = (P_diag^-1)[r][c] of the sub-block being solved
-      bf16 vT[D][128 + 8];  // dV^T of the block (bf16, T-perm within 16-groups)
-    } fin;
-  } u;
-};
-template <int D, bool F32>
-struct PcolSmem<D, true, F32> {
+struct PcolSmem {
   static constexpr int NB = stage_bufs(D, F32);
   union {
     struct {
-      bf16 k[NB][64 * D];
+      bf16 k[NB][64 * D];   // swizzled tiles (chunk c of row r at c ^ (r & 7))
       bf16 dv[NB][64 * D];
-      bf16 dvl[NB][64 * D];  // lo part of dV
-      bf16 kl[F32 ? NB : 1][F32 ? 64 * D : 8];  // lo part of K (fp32 inputs)
-      float r[NB][64];
+      bf16 dvl[EXACT ? NB : 1][EXACT ? 64 * D : 8];  // lo part of dV
+      bf16 kl[F32 ? NB : 1][F32 ? 64 * D : 8];       // lo part of K (fp32 inputs)
+      float r[NB][EXACT ? 64 : 4];
     } st;
-    struct {
-      float Rt[D][132];
-      float Xt[64][68];
-      bf16 vT[D][128 + 8];
-      bf16 vTl[D][128 + 8];  // lo part of dV^T of the block
+    struct {  // the block's finish
+      bf16 nx[2][64 * D];                              // dV rows of the next block (two row tiles)
+      bf16 nxl[EXACT ? 2 : 1][EXACT ? 64 * D : 8];     // their lo part
+      bf16 rh[128 * D], rl[128 * D];                   // R rows hi / lo (swizzled), then dV of the block (rl: its lo)
     } fin;
+    struct {  // the column sums of the next block's rows
+      bf16 nx[2][64 * D];
+      bf16 nxl[EXACT ? 2 : 1][EXACT ? 64 * D : 8];
+      bf16 k[2][64 * D];                               // their K rows
+      bf16 kl[F32 ? 2 : 1][F32 ? 64 * D : 8];
+      float r[2][EXACT ? 64 : 4];
+    } cs;
   } u;
 };
 
@@ -653,8 +647,8 @@ template <int D, bool EXACT, bool F32 = false, int DA = D>
 __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void lucid_precond_bwd_col_kernel(
     const bf16* __restrict__ k, Strides ks, int Hkv, int T, int BH, const float* __restrict__ rinv,
     const bf16* __restrict__ khat, float scale, const bf16* __restrict__ kt, const bf16* __restrict__ vpb,
-    const bf16* __restrict__ vpbl, const float* __restrict__ pinv, const float* __restrict__ mass,
-    const float* __restrict__ dvp,
+    const bf16* __restrict__ vpbl, const bf16* __restrict__ xt, const bf16* __restrict__ link,
+    const float* __restrict__ mass, const float* __restrict__ dvp,
     bf16* __restrict__ dvb, bf16* __restrict__ dvbl, std::conditional_t<F32, float, bf16>* __restrict__ dv_out,
     Strides dvs, float* __restrict__ colsum, int* __restrict__ counters, Lo lo) {
   static_assert(!F32 || EXACT, "fp32 inputs: exact instance");
@@ -718,13 +712,15 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void luc
     }
   }
 
-  // ---- sweep over the later 64-row tiles, far (published first) to near ----
-  const int first = NT - 1, last = 2 * p + 2;  // tiles first, first-1, ..., last
+  // ---- sweep over the later 64-row tiles, far (published first) to near, but for the next
+  // two blocks' (p + 1 enters dV through the link, p + 2 by its P^T dV alone; both enter the
+  // column sums after the publish) ----
+  const int first = NT - 1, last = 2 * p + 6;  // tiles first, first-1, ..., last
   int ready = 0;
   // step k of the sweep stages tile first - k into buffer k % NB; the newest
   // STAGE_OPS vector memory operations of a wave are the tiles of a step
   constexpr int STAGE_OPS = (F32 ? 4 : EXACT ? 3 : 2) * (64 * (D / 8) / 256);
-  const int nsteps = first - last + 1;
+  const int nsteps = max(first - last + 1, 0);
   int plan_k[64 * (D / 8) / 256], plan_d[64 * (D / 8) / 256];
   dma_plan<64, D / 8>(ks.t, plan_k);
   dma_plan<64, D / 8>(D, plan_d);
@@ -759,27 +755,6 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void luc
       }
     }
   };
-  // the two inverses X_A, X_B (2 x 64 x 64 fp32) into stg[0..7]: chunk u -> sub-block u >> 2
-  const float* pinv_blk = pinv + ((int64_t)bh * NT + 2 * p) * 4096;
-  f32x4 xr[8];
-  auto xload = [&]() {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int idx = tid + 256 * u;
-      const int sb = idx >> 10, r = (idx >> 4) & 63, c4 = (idx & 15) * 4;
-      xr[u] = *reinterpret_cast<const f32x4*>(pinv_blk + sb * 4096 + r * 64 + c4);
-    }
-  };
-  auto xstore_t = [&](int sb) {
-#pragma unroll
-    for (int u = 4 * sb; u < 4 * sb + 4; ++u) {
-      const int idx = tid + 256 * u;
-      const int r = (idx >> 4) & 63, c4 = (idx & 15) * 4;
-      const f32x4 x = xr[u];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sm.u.fin.Xt[c4 + e][r] = x[e];
-    }
-  };
   if (nsteps > 0) {
     ready = wait_counter_gt(cnt, NT - 1 - first);
     stage(0);
@@ -787,22 +762,24 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void luc
     if (NB == 3) try_issue(1);
     if (issued > 1) dma_wait_but<STAGE_OPS>();
     else dma_wait();
-  } else {
-    xload();
   }
   __syncthreads();
 
-  auto sweep_tile = [&](int buf) {
+  // one staged 64-row tile (K rows tk / tkl, dV rows tdv / tdvl, 1/rms tr); SOLVE: P^T dV as
+  // well as the column sums
+  auto sweep_tile = [&](const bf16* tk, const bf16* tkl, const bf16* tdv, const bf16* tdvl, const float* tr,
+                        auto solvec) __attribute__((always_inline)) {
+    constexpr bool SOLVE = decltype(solvec)::value;
 #pragma unroll
     for (int rh = 0; rh < 2; ++rh) {
       bf16x8 ka[NKS], da[NKS];
 #pragma unroll
       for (int st = 0; st < NKS_A; ++st) {
-        ka[st] = ld8(swz<D / 8>(sm.u.st.k[buf], rh * 32 + l32, 2 * st + g));
-        da[st] = ld8(swz<D / 8>(sm.u.st.dv[buf], rh * 32 + l32, 2 * st + g));
+        ka[st] = ld8(swz<D / 8>(tk, rh * 32 + l32, 2 * st + g));
+        da[st] = ld8(swz<D / 8>(tdv, rh * 32 + l32, 2 * st + g));
       }
       float rI[16];
-      if constexpr (EXACT) lds_rows16(&sm.u.st.r[buf][rh * 32], g, rI);
+      if constexpr (EXACT) lds_rows16(tr + rh * 32, g, rI);
       f32x16 sc = zero16(), gg = zero16();
 #pragma unroll
       for (int st = 0; st < NKS_A; ++st) {
@@ -813,13 +790,13 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void luc
 #pragma unroll
         for (int st = 0; st < NKS_A; ++st) {
           gg = mfma32(da[st], vbJl[st], gg);
-          gg = mfma32(ld8(swz<D / 8>(sm.u.st.dvl[buf], rh * 32 + l32, 2 * st + g)), vbJ[st], gg);
+          gg = mfma32(ld8(swz<D / 8>(tdvl, rh * 32 + l32, 2 * st + g)), vbJ[st], gg);
         }
       }
       if constexpr (F32) {
 #pragma unroll
         for (int st = 0; st < NKS_A; ++st) {
-          const bf16x8 kal = ld8(swz<D / 8>(sm.u.st.kl[buf], rh * 32 + l32, 2 * st + g));
+          const bf16x8 kal = ld8(swz<D / 8>(tkl, rh * 32 + l32, 2 * st + g));
           sc = mfma32(ka[st], kbJl[st], sc);
           sc = mfma32(kal, kbJ[st], sc);
           sc = mfma32(kal, kbJl[st], sc);
@@ -831,46 +808,55 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void luc
         sc[e] = pe;
         gg[e] = EXACT ? gg[e] * pe * rI[e] : gg[e] * pe;
       }
-      const bf16x8 pb0 = pack_b(sc, 0), pb1 = pack_b(sc, 1);
       const bf16x8 mb0 = pack_b(gg, 0), mb1 = pack_b(gg, 1);
-      bf16x8 pl0, pl1, ml0, ml1;  // lo parts (EXACT)
+      bf16x8 pb0, pb1, pl0, pl1, ml0, ml1;  // (lo parts: EXACT)
+      if constexpr (SOLVE) {
+        pb0 = pack_b(sc, 0);
+        pb1 = pack_b(sc, 1);
+      }
       if constexpr (EXACT) {
-        pl0 = pack_lo(sc, 0, pb0);
-        pl1 = pack_lo(sc, 1, pb1);
+        if constexpr (SOLVE) {
+          pl0 = pack_lo(sc, 0, pb0);
+          pl1 = pack_lo(sc, 1, pb1);
+        }
         ml0 = pack_lo(gg, 0, mb0);
         ml1 = pack_lo(gg, 1, mb1);
       }
 #pragma unroll
       for (int t = 0; t < NDT_A; ++t) {
-        const bf16x8 a0 = lds_tr_a<D / 8>(sm.u.st.dv[buf], rh * 32, t * 32);
-        const bf16x8 a1 = lds_tr_a<D / 8>(sm.u.st.dv[buf], rh * 32 + 16, t * 32);
-        const bf16x8 k0 = lds_tr_a<D / 8>(sm.u.st.k[buf], rh * 32, t * 32);
-        const bf16x8 k1 = lds_tr_a<D / 8>(sm.u.st.k[buf], rh * 32 + 16, t * 32);
-        adv[t] = mfma32(a0, pb0, adv[t]);
-        adv[t] = mfma32(a1, pb1, adv[t]);
+        const bf16x8 k0 = lds_tr_a<D / 8>(tk, rh * 32, t * 32);
+        const bf16x8 k1 = lds_tr_a<D / 8>(tk, rh * 32 + 16, t * 32);
+        if constexpr (SOLVE) {
+          const bf16x8 a0 = lds_tr_a<D / 8>(tdv, rh * 32, t * 32);
+          const bf16x8 a1 = lds_tr_a<D / 8>(tdv, rh * 32 + 16, t * 32);
+          adv[t] = mfma32(a0, pb0, adv[t]);
+          adv[t] = mfma32(a1, pb1, adv[t]);
+          if constexpr (EXACT) {
+            adv[t] = mfma32(a0, pl0, adv[t]);
+            adv[t] = mfma32(a1, pl1, adv[t]);
+            adv[t] = mfma32(lds_tr_a<D / 8>(tdvl, rh * 32, t * 32), pb0, adv[t]);
+            adv[t] = mfma32(lds_tr_a<D / 8>(tdvl, rh * 32 + 16, t * 32), pb1, adv[t]);
+          }
+        }
         acs[t] = mfma32(k0, mb0, acs[t]);
         acs[t] = mfma32(k1, mb1, acs[t]);
         if constexpr (EXACT) {
-          adv[t] = mfma32(a0, pl0, adv[t]);
-          adv[t] = mfma32(a1, pl1, adv[t]);
-          adv[t] = mfma32(lds_tr_a<D / 8>(sm.u.st.dvl[buf], rh * 32, t * 32), pb0, adv[t]);
-          adv[t] = mfma32(lds_tr_a<D / 8>(sm.u.st.dvl[buf], rh * 32 + 16, t * 32), pb1, adv[t]);
           acs[t] = mfma32(k0, ml0, acs[t]);
           acs[t] = mfma32(k1, ml1, acs[t]);
         }
         if constexpr (F32) {
-          acs[t] = mfma32(lds_tr_a<D / 8>(sm.u.st.kl[buf], rh * 32, t * 32), mb0, acs[t]);
-          acs[t] = mfma32(lds_tr_a<D / 8>(sm.u.st.kl[buf], rh * 32 + 16, t * 32), mb1, acs[t]);
+          acs[t] = mfma32(lds_tr_a<D / 8>(tkl, rh * 32, t * 32), mb0, acs[t]);
+          acs[t] = mfma32(lds_tr_a<D / 8>(tkl, rh * 32 + 16, t * 32), mb1, acs[t]);
         }
       }
     }
   };
-  // all steps but the last; the last one is peeled so that the inverses it
-  // prefetches do not hold registers through the loop
-  for (int ks_ = 0; ks_ + 1 < nsteps; ++ks_) {
+  for (int ks_ = 0; ks_ < nsteps; ++ks_) {
+    const int buf = ks_ % NB;
     try_issue(ks_ + NB - 1);
-    sweep_tile(ks_ % NB);
-    if (issued == ks_ + 1) {  // the next tile was not published yet: wait for it
+    sweep_tile(sm.u.st.k[buf], sm.u.st.kl[F32 ? buf : 0], sm.u.st.dv[buf], sm.u.st.dvl[EXACT ? buf : 0],
+               sm.u.st.r[buf], std::true_type{});
+    if (ks_ + 1 < nsteps && issued == ks_ + 1) {  // the next tile was not published yet: wait for it
       ready = wait_counter_gt(cnt, NT - 1 - (first - issued));
       stage(issued);
       ++issued;
@@ -879,133 +865,217 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void luc
     else dma_wait();
     __syncthreads();
   }
-  if (nsteps > 0) {
-    xload();  // fetch the inverses while the last tile is processed
-    sweep_tile((nsteps - 1) % NB);
+
+  // ---- the rows of block p + 2: P while their dV is still being solved, then P^T dV ----
+  const bool hasnx = p + 1 < NP, hasn2 = p + 2 < NP;
+  // K rows (and 1/rms) of block p + d into the column-sum staging
+  auto stage_near = [&](int d) {
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb) {
+      const int i1 = J0 + 128 * d + 64 * hb;
+      if constexpr (EXACT) {
+        if (w == 0) dma_f32x64(rv + i1, sm.u.cs.r[hb]);
+        dma_stage<64, D / 8>(plan_k, kh + (int64_t)i1 * ks.t, sm.u.cs.k[hb]);
+      } else {
+        dma_stage<64, D / 8>(plan_d, khh + (int64_t)i1 * D, sm.u.cs.k[hb]);
+      }
+      if constexpr (F32) dma_stage<64, D / 8>(plan_k, klh + (int64_t)i1 * ks.t, sm.u.cs.kl[hb]);
+    }
+  };
+  auto stage_near_dv = [&](int d) {
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb) {
+      const int64_t o1 = (int64_t)(J0 + 128 * d + 64 * hb) * D;
+      dma_stage<64, D / 8>(plan_d, dvbh + o1, sm.u.cs.nx[hb]);
+      if constexpr (EXACT) dma_stage<64, D / 8>(plan_d, dvblh + o1, sm.u.cs.nxl[hb]);
+    }
+  };
+  if (hasn2) {
+    stage_near(2);
     dma_wait();
     __syncthreads();
+    bf16x8 pn[4][2], pnl[EXACT ? 4 : 1][2];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // 32-row quarter q of the block
+      const bf16* tk = sm.u.cs.k[q >> 1];
+      const bf16* tkl = sm.u.cs.kl[F32 ? q >> 1 : 0];
+      const int rh = q & 1;
+      f32x16 sc = zero16();
+#pragma unroll
+      for (int st = 0; st < NKS_A; ++st) {
+        const bf16x8 ka = ld8(swz<D / 8>(tk, rh * 32 + l32, 2 * st + g));
+        sc = mfma32(ka, kbJ[st], sc);
+        if constexpr (F32) {
+          const bf16x8 kal = ld8(swz<D / 8>(tkl, rh * 32 + l32, 2 * st + g));
+          sc = mfma32(ka, kbJl[st], sc);
+          sc = mfma32(kal, kbJ[st], sc);
+          sc = mfma32(kal, kbJl[st], sc);
+        }
+      }
+      float rI[16];
+      if constexpr (EXACT) lds_rows16(sm.u.cs.r[q >> 1] + rh * 32, g, rI);
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        sc[e] = __builtin_amdgcn_exp2f(EXACT ? fmaf(sc[e] * aJ, rI[e], -c0) : sc[e] * aJ);
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        pn[q][hh] = pack_b(sc, hh);
+        if constexpr (EXACT) pnl[q][hh] = pack_lo(sc, hh, pn[q][hh]);
+      }
+    }
+    const int need = NT - 2 * p - 5;  // block p + 2 is published once the counter exceeds this
+    if (need >= ready) ready = wait_counter_gt(cnt, need);
+    stage_near_dv(2);
+    dma_wait();
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int t = 0; t < NDT_A; ++t)
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          const bf16x8 a = lds_tr_a<D / 8>(sm.u.cs.nx[q >> 1], (q & 1) * 32 + 16 * hh, t * 32);
+          adv[t] = mfma32(a, pn[q][hh], adv[t]);
+          if constexpr (EXACT) {
+            adv[t] = mfma32(a, pnl[q][hh], adv[t]);
+            adv[t] = mfma32(lds_tr_a<D / 8>(sm.u.cs.nxl[q >> 1], (q & 1) * 32 + 16 * hh, t * 32), pn[q][hh], adv[t]);
+          }
+        }
   }
 
-  if constexpr (!EXACT) {  // the sweep's factor 1/C
-    const float Cf = __builtin_amdgcn_exp2f(-c0);
+  // ---- the block: dV_p = X^T R + link dV_{p+1}, R = dV' - acc = -adv (X^T, link: xt and
+  // link planes); wave -> its 32 columns ----
+  const float Cf = EXACT ? 1.f : __builtin_amdgcn_exp2f(-c0);  // the sweep's factor 1/C
+  auto& fin = sm.u.fin;
+  const int wu = __builtin_amdgcn_readfirstlane(w);
+  const int crow = cw + l32;  // this lane's column in the block
+  const int64_t prow = ((int64_t)bh * NP + p) * 32768 + crow * 128 + 8 * g;
+  bf16x8 zh[8], zl[8];  // this wave's rows of X^T (k-steps 2w ..), then of the link
 #pragma unroll
-    for (int t = 0; t < NDT; ++t)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        adv[t][e] *= Cf;
-        acs[t][e] *= Cf;
-      }
+  for (int st = 0; st < 8; ++st) {
+    if (st < 2 * wu) continue;
+    zh[st] = ld8(xt + prow + 16 * st);
+    zl[st] = ld8(xt + prow + 16384 + 16 * st);
   }
-  // ---- R = dV' - acc = -adv for this wave's columns; X^T of sub-block B ----
-  float(*Rt)[132] = sm.u.fin.Rt;
 #pragma unroll
   for (int t = 0; t < NDT; ++t)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) Rt[t * 32 + drow(e, g)][cw + l32] = -adv[t][e];
-  xstore_t(1);
+    for (int qq = 0; qq < 4; ++qq) {
+      const int d0 = t * 32 + 8 * qq + 4 * g;
+      bf16x4 rh, rl;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float x = -Cf * adv[t][4 * qq + u];
+        rh[u] = (bf16)x;
+        rl[u] = (bf16)(x - (float)rh[u]);
+      }
+      const int off = swz_off<D / 8>(crow, d0 >> 3) + (d0 & 7);
+      *reinterpret_cast<bf16x4*>(fin.rh + off) = rh;
+      *reinterpret_cast<bf16x4*>(fin.rl + off) = rl;
+    }
   __syncthreads();
-
-  // dV^T[d][c] = sum_r R^T[d][r] X[r][c] for sub-block sb (X lower: r >= c)
-  auto diag_solve = [&](int sb) {
-    for (int tile = w; tile < NDT * 2; tile += 4) {
-      const int dt = tile >> 1, chh = tile & 1;
-      f32x16 o = zero16();
-      for (int st = chh ? 2 : 0; st < 4; ++st) {
-        bf16x8 ah, al, bh8, bl;
-        split8(&Rt[dt * 32 + l32][sb * 64 + 16 * st + 8 * g], ah, al);
-        split8(&sm.u.fin.Xt[chh * 32 + l32][16 * st + 8 * g], bh8, bl);
-        o = mfma32(ah, bh8, o);
-        o = mfma32(ah, bl, o);
-        o = mfma32(al, bh8, o);
-      }
-      const int cl = chh * 32 + l32;
-      const int r = J0 + sb * 64 + cl;
-      const int lslot = sb * 64 + ((cl & ~15) | jmap(cl & 15));
-      bf16* ob = dvb + ((int64_t)bh * T + r) * D;
-      auto* ou = dv_out + b * dvs.b + h * dvs.h + (int64_t)r * dvs.t;
+  f32x16 o[NDT];
 #pragma unroll
-      for (int qq = 0; qq < 4; ++qq) {
-        const int d0 = dt * 32 + 8 * qq + 4 * g;
-        bf16x4 bb, bl;
+  for (int t = 0; t < NDT; ++t) o[t] = zero16();
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          bb[u] = (bf16)o[4 * qq + u];
-          sm.u.fin.vT[d0 + u][lslot] = bb[u];
-          if constexpr (EXACT) {
-            bl[u] = (bf16)(o[4 * qq + u] - (float)bb[u]);
-            sm.u.fin.vTl[d0 + u][lslot] = bl[u];
-          }
-        }
-        *reinterpret_cast<bf16x4*>(ob + d0) = bb;
-        if constexpr (F32) {
-          f32x4 x;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) x[u] = o[4 * qq + u];
-          *reinterpret_cast<f32x4*>(ou + d0) = x;
-        } else {
-          *reinterpret_cast<bf16x4*>(ou + d0) = bb;
-        }
-        if constexpr (EXACT) *reinterpret_cast<bf16x4*>(dvbl + ((int64_t)bh * T + r) * D + d0) = bl;
-      }
-    }
-  };
-  diag_solve(1);
-  publish_counter(cnt, NT - (2 * p + 1));
-
-  // ---- R_A -= P_BA^T dV_B: wave -> (A columns half na, B rows half kb) ----
-  {
-    const int na = w & 1, kb = w >> 1;
-    const int colA = J0 + na * 32 + l32;
-    f32x16 sc = zero16();
-#pragma unroll
-    for (int st = 0; st < NKS; ++st) {
-      const int64_t om = (int64_t)(J0 + 64 + kb * 32 + l32) * ks.t + 16 * st + 8 * g;
-      const int64_t on = (int64_t)colA * ks.t + 16 * st + 8 * g;
-      sc = mfma32(ld8(kh + om), ld8(kh + on), sc);
-      if constexpr (F32) {
-        sc = mfma32(ld8(kh + om), ld8(klh + on), sc);
-        sc = mfma32(ld8(klh + om), ld8(kh + on), sc);
-      }
-    }
-    const float aA = sl2 * rv[colA];
-    float rB[16];
-    load_rows16(rv + J0 + 64 + kb * 32, g, rB);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) sc[e] = __builtin_amdgcn_exp2f(fmaf(sc[e] * aA, rB[e], -c0));
-    const bf16x8 p0 = pack_b(sc, 0), p1 = pack_b(sc, 1);
-    f32x16 cr[NDT];
+  for (int st = 0; st < 8; ++st) {
+    if (st < 2 * wu) continue;
 #pragma unroll
     for (int t = 0; t < NDT; ++t) {
-      const bf16x8 v0 = ld8(&sm.u.fin.vT[t * 32 + l32][64 + kb * 32 + 8 * g]);
-      const bf16x8 v1 = ld8(&sm.u.fin.vT[t * 32 + l32][64 + kb * 32 + 16 + 8 * g]);
-      cr[t] = mfma32(v0, p0, zero16());
-      cr[t] = mfma32(v1, p1, cr[t]);
-      if constexpr (EXACT) {
-        cr[t] = mfma32(v0, pack_lo(sc, 0, p0), cr[t]);
-        cr[t] = mfma32(v1, pack_lo(sc, 1, p1), cr[t]);
-        cr[t] = mfma32(ld8(&sm.u.fin.vTl[t * 32 + l32][64 + kb * 32 + 8 * g]), p0, cr[t]);
-        cr[t] = mfma32(ld8(&sm.u.fin.vTl[t * 32 + l32][64 + kb * 32 + 16 + 8 * g]), p1, cr[t]);
+      const bf16x8 ah = lds_tr_a<D / 8>(fin.rh, 16 * st, t * 32);
+      const bf16x8 al = lds_tr_a<D / 8>(fin.rl, 16 * st, t * 32);
+      o[t] = mfma32(ah, zh[st], o[t]);
+      o[t] = mfma32(ah, zl[st], o[t]);
+      o[t] = mfma32(al, zh[st], o[t]);
+    }
+  }
+  if (hasnx) {
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      zh[st] = ld8(link + prow + 16 * st);
+      if constexpr (EXACT) zl[st] = ld8(link + prow + 16384 + 16 * st);
+    }
+    const int need = NT - 2 * p - 3;  // the next block is published once the counter exceeds this
+    if (need >= ready) wait_counter_gt(cnt, need);
+    stage_near_dv(1);
+    dma_wait();
+    __syncthreads();  // (every wave is done with R too)
+#pragma unroll
+    for (int st = 0; st < 8; ++st)
+#pragma unroll
+      for (int t = 0; t < NDT; ++t) {
+        const bf16x8 va = lds_tr_a<D / 8>(fin.nx[st >> 2], 16 * (st & 3), t * 32);
+        o[t] = mfma32(va, zh[st], o[t]);
+        if constexpr (EXACT) {
+          o[t] = mfma32(va, zl[st], o[t]);
+          o[t] = mfma32(lds_tr_a<D / 8>(fin.nxl[st >> 2], 16 * (st & 3), t * 32), zh[st], o[t]);
+        }
       }
-    }
-    const int col = na * 32 + l32;
-    if (kb == 1) {
-#pragma unroll
-      for (int t = 0; t < NDT; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) Rt[t * 32 + drow(e, g)][col] -= cr[t][e];
-    }
-    xstore_t(0);
-    __syncthreads();
-    if (kb == 0) {
-#pragma unroll
-      for (int t = 0; t < NDT; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) Rt[t * 32 + drow(e, g)][col] -= cr[t][e];
-    }
+  } else {
     __syncthreads();
   }
-  diag_solve(0);
-  publish_counter(cnt, NT - 2 * p);
+  // dV rows through this wave's own rows of rh / rl, published, then to the caller's dV
+#pragma unroll
+  for (int t = 0; t < NDT; ++t)
+#pragma unroll
+    for (int qq = 0; qq < 4; ++qq) {
+      const int d0 = t * 32 + 8 * qq + 4 * g;
+      bf16x4 bb, bl;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        bb[u] = (bf16)o[t][4 * qq + u];
+        bl[u] = (bf16)(o[t][4 * qq + u] - (float)bb[u]);
+      }
+      const int off = swz_off<D / 8>(crow, d0 >> 3) + (d0 & 7);
+      *reinterpret_cast<bf16x4*>(fin.rh + off) = bb;
+      if constexpr (EXACT) *reinterpret_cast<bf16x4*>(fin.rl + off) = bl;
+    }
+  __builtin_amdgcn_wave_barrier();
+  {
+    const __amdgpu_buffer_rsrc_t ph = pub_base(dvb + (int64_t)bh * T * D);
+    const __amdgpu_buffer_rsrc_t pl = pub_base(EXACT ? dvbl + (int64_t)bh * T * D : nullptr);
+#pragma unroll
+    for (int u = 0; u < D / 16; ++u) {  // 32 rows of D / 8 chunks
+      const int idx = lane + 64 * u, row = cw + idx / (D / 8), ch = idx % (D / 8);
+      const unsigned off = 2u * ((unsigned)(J0 + row) * (unsigned)D + 8u * ch);
+      const bf16x8 x = ld8(swz<D / 8>(fin.rh, row, ch));
+      st_pub16(ph, off, x);
+      if constexpr (EXACT) st_pub16(pl, off, ld8(swz<D / 8>(fin.rl, row, ch)));
+      if constexpr (!F32)
+        *reinterpret_cast<bf16x8*>(dv_out + b * dvs.b + h * dvs.h + (int64_t)(J0 + row) * dvs.t + 8 * ch) = x;
+    }
+  }
+  publish_stored(cnt, NT - 2 * p);
+  if constexpr (F32) {
+    float* ou = dv_out + b * dvs.b + h * dvs.h + (int64_t)(J0 + crow) * dvs.t;
+#pragma unroll
+    for (int t = 0; t < NDT; ++t)
+#pragma unroll
+      for (int qq = 0; qq < 4; ++qq)
+        *reinterpret_cast<f32x4*>(ou + t * 32 + 8 * qq + 4 * g) =
+            f32x4{o[t][4 * qq], o[t][4 * qq + 1], o[t][4 * qq + 2], o[t][4 * qq + 3]};
+  }
+
+  // ---- the next two blocks' rows in the column sums (block p + 1's dV is still staged) ----
+#pragma unroll 1
+  for (int d = 1; d <= 2; ++d) {
+    if (p + d >= NP) break;
+    stage_near(d);
+    if (d == 2) stage_near_dv(2);
+    dma_wait();
+    __syncthreads();
+#pragma unroll 1
+    for (int hb = 0; hb < 2; ++hb)
+      sweep_tile(sm.u.cs.k[hb], sm.u.cs.kl[F32 ? hb : 0], sm.u.cs.nx[hb], sm.u.cs.nxl[EXACT ? hb : 0], sm.u.cs.r[hb],
+                 std::false_type{});
+    __syncthreads();
+  }
+  if constexpr (!EXACT) {
+#pragma unroll
+    for (int t = 0; t < NDT; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acs[t][e] *= Cf;
+  }
 
   // ---- diagonal-block terms of the column sums (rows r >= columns c inside the workgroup) ----
   // wave w: its 32 columns (sub-block w >> 1) against rows of sub-blocks rb = w >> 1 .. 1
@@ -1088,11 +1158,11 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void luc
 }
 
 // ---------------------------------------------------------------------------
-// The column chain with 256 columns per workgroup (head dim 64, bf16 chains; the default
-// when T is a multiple of 256): eight waves, wave w owns columns J0 + 32w .. +32 of the
+// The column chain with 256 columns per workgroup (head dim 64, bf16 chains, many long
+// heads; linked_bwd64 in lucid_capi.hip): eight waves, wave w owns columns J0 + 32w .. +32 of the
 // four 64-column sub-blocks A..D (w >> 1), so every staged row tile (K^ rows, dV rows)
 // serves twice the columns of lucid_precond_bwd_col_kernel and a head's tiles are
-// fetched half as often.  The sweep body is that kernel's.  After the sweep over the
+// fetched half as often.  The sweep body is that kernel's.  After the sweep over all
 // rows below the block, the sub-blocks are solved from the last (D) to the first (A):
 //   dV_s = X_s^T R_s  (R_s = dV'_s - acc_s, X_s = P_ss^-1), published as the head's next
 //   64-row block; its dV rows (bf16, from the solve) and K^ rows are put in LDS in the

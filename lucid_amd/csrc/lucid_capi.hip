@@ -23,8 +23,9 @@ thread_local std::string g_last_error;
 // Per calling thread: a mode set on one thread never changes how another thread's calls run.
 thread_local int g_precision = LUCID_PRECISION_AUTO;
 
-// Forward schedule (lucid_set_fused_forward): the fused chain + attention kernel at head
-// dim 64 with one query head per kv head, or the two-kernel sequence.  Per calling thread.
+// Forward schedule (lucid_set_fused_forward): on, the fused chain + attention kernel at head
+// dim 64 with one query head per kv head where it is the faster one (linked_fwd64); off, always
+// the two-kernel sequence.  Per calling thread.
 thread_local bool g_fused_fwd = true;
 
 int fail(const std::string& msg) {
@@ -68,6 +69,8 @@ struct FwdWs {
   bf16* vpt;     // [BH][D][T]  V'^T, T-perm
   float* pinv;   // [BH][T/64][64][64]  inverses of the diagonal blocks of P
   float* zx;     // [BH][T/128][64][64] -(X_B P_BA) per 128-row block, columns T-perm
+  float* y;      // [BH][T/128][64][64] zx X_A: the inverse of the 128-row block below X_A
+  bf16* link;    // [BH][T/128][2][128][128] -X_i P_{i,i-1}, hi / lo planes, columns T-perm (lucid_link_kernel)
   bf16* vpbl;    // [BH][T][D]  lo part of V' (exact heads)
   bf16* vptl;    // [BH][D][T]  lo part of V'^T, T-perm (exact heads)
   float* mass;   // [BH]        largest row mass sum_{j<i} P_ij^2 (sampled; selects the chain precision)
@@ -105,6 +108,8 @@ FwdWs carve_fwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = fal
   w.vpt = reinterpret_cast<bf16*>(take(BH * D * T * 2));
   w.pinv = reinterpret_cast<float*>(take(BH * (T / 64) * 4096 * 4));
   w.zx = reinterpret_cast<float*>(take(BH * (T / 128) * 4096 * 4));
+  w.y = reinterpret_cast<float*>(take(BH * (T / 128) * 4096 * 4));
+  w.link = reinterpret_cast<bf16*>(take(BH * (T / 128) * 32768 * 2));
   w.vpbl = reinterpret_cast<bf16*>(take(BH * T * D * 2));
   w.vptl = reinterpret_cast<bf16*>(take(BH * D * T * 2));
   w.mass = reinterpret_cast<float*>(take(BH * 4));
@@ -136,6 +141,8 @@ struct BwdWs {
   bf16* dvb;     // [BH][T][D]   dV bf16
   bf16* dvbl;    // [BH][T][D]   lo part of dV (exact heads)
   float* colsum; // [BH][T][D]   sum_I M_IJ^T K^_I
+  bf16* xt;      // [BH][T/128][2][128][128] X_p^T, hi / lo planes, columns T-perm (lucid_link_kernel)
+  bf16* link;    // [BH][T/128][2][128][128] -X_p^T P_{p+1,p}^T, likewise
   int* counters; // [BH]
   bf16 *doh, *dol; // fp32 inputs only: the bf16 pair of dO ([BHq][T][D] rows)
   float* dkdv;   // [2 (dkdv_splits - 1)][BH][T][D] partial dV' and dK of a split column sweep
@@ -176,6 +183,8 @@ BwdWs carve_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = fal
   w.dvb = reinterpret_cast<bf16*>(take(BH * T * D * 2));
   w.dvbl = reinterpret_cast<bf16*>(take(BH * T * D * 2));
   w.colsum = reinterpret_cast<float*>(take(BH * T * D * 4));
+  w.xt = reinterpret_cast<bf16*>(take(BH * (T / 128) * 32768 * 2));
+  w.link = reinterpret_cast<bf16*>(take(BH * (T / 128) * 32768 * 2));
   w.counters = reinterpret_cast<int*>(take(BH * 4));
   if (f32) {
     w.doh = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
@@ -216,6 +225,25 @@ lucid::Strides S(const int64_t* s) { return lucid::Strides{s[0], s[1], s[2]}; }
 #define LUCID_LAUNCH_B(NAME, KERNEL, GRID, BLOCK, ST, ...) \
   LUCID_TIMED_LAUNCH_B(hip_status, NAME, KERNEL, GRID, BLOCK, ST, __VA_ARGS__)
 
+// Which chain kernels run the bf16 chains of BH heads.  The 128-row linked chains take about
+// 4.2 us a hand-off (fp32 / exact 5.5) and stage a key tile per 128 rows; the fused forward
+// 10.4 us (its hand-off carries the attention's last pair) but shares its operand reads between
+// the chain and the attention, and the 256-row chains 20-25 us per 256 rows but stage a tile
+// per 256.  So the links win where a head has few others beside it, up to a length where the
+// sweeps outweigh the hand-offs.  Measured on one MI355X, us, links against the other (BH, T):
+//   forward at head dim 64, against the fused kernel: (4, 1024) 101/96, (4, 2048) 151/157, (8, 8192) 477/557,
+//     (8, 32768) 2660/3021, (16, 1024) 112/102, (16, 4096) 298/320, (16, 8192) 592/610, (16, 16384) 1494/1444,
+//     (16, 24576) 3003/3161, (16, 32768) 5094/5334, (32, 4096) 391/383, (32, 16384) 2974/2880, (64, 2048) 277/253
+//   forward at 128, against 256 rows: (8, 8192) 925/1230, (8, 32768) 10691/11285, (8, 49152) 24239/24258,
+//     (8, 65536) 41823/40999, (32, 4096) 541/629, (32, 8192) 1545/1541, (32, 16384) 5468/4985
+//   backward at 64, against 256 columns: (16, 1024) 166/188, (32, 4096) 701/843, (16, 16384) 3921/4031,
+//     (16, 32768) 14535/14460, (32, 32768) 30392/29882, (8, 65536) 29477/29962
+bool linked_fwd64(int64_t BH, int64_t T) {
+  return T >= 2048 && (BH <= 8 || (BH <= 16 && T <= 8192) || T >= 1536 * BH);
+}
+bool linked_fwd128(int64_t BH, int64_t T) { return T % 256 != 0 || BH * T <= 8 * 49152; }
+bool linked_bwd64(int64_t BH, int64_t T) { return T % 256 != 0 || BH < 16 || BH * T < 16 * 32768; }
+
 template <int D>
 int launch_precond_fwd(const void* k, const int64_t* ks, const void* v, const int64_t* vs, float* vprime,
                        const FwdWs& w, int B, int Hkv, int T, float scale, float eps, float dn, hipStream_t st) {
@@ -228,27 +256,30 @@ int launch_precond_fwd(const void* k, const int64_t* ks, const void* v, const in
   // the in-block coupling of every 128-row chain block and (AUTO) the heads' row masses
   LUCID_LAUNCH("lucid_zx_kernel", lucid::lucid_zx_kernel<D>, dim3(T / 128, BH), st, (const bf16*)k, S(ks), Hkv, T,
                w.rinv, scale, w.pinv, w.zx, lucid::Lo{}, g_precision == LUCID_PRECISION_AUTO ? w.mass : nullptr);
+  // the 256-row chain keeps its own in-block coupling; only the exact heads read links then
+  const bool wide = D == 128 && !linked_fwd128(BH, T);
+  LUCID_LAUNCH("lucid_link_kernel", (lucid::lucid_link_kernel<D, false, false>), dim3(T / 128, BH), st,
+               (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, nullptr, w.link, w.mass, wide,
+               lucid::Lo{});
   // both instances of the chain: each solves the heads of its precision and returns at
   // once for the others
   if (g_precision != LUCID_PRECISION_EXACT) {
-    if (D == 128 && T % 256 == 0)  // 256 rows per workgroup: each staged pair serves twice the rows
+    if (wide) {  // 256 rows per workgroup: each staged pair serves twice the rows
       LUCID_LAUNCH_B("lucid_precond_fwd_wide_kernel", (lucid::lucid_precond_fwd_wide_kernel<128>),
                      dim3((T / 256) * BH), dim3(512), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH,
                      w.rinv, w.khat, scale, vprime, w.vpb, w.vpt, w.pinv, w.zx, w.mass, w.counters);
-    else if (D == 128)  // eight waves (two per SIMD) at head dim 128
-      LUCID_LAUNCH_B("lucid_precond_fwd_kernel", (lucid::lucid_precond_fwd_kernel<128, false, false, 8>),
-                     dim3((T / 128) * BH), dim3(512), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH,
-                     w.rinv, w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.zx, w.mass, w.counters,
-                     lucid::Lo{});
-    else
-      LUCID_LAUNCH("lucid_precond_fwd_kernel", (lucid::lucid_precond_fwd_kernel<D, false>), dim3((T / 128) * BH),
-                   st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH, w.rinv, w.khat, scale, vprime,
-                   w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.zx, w.mass, w.counters, lucid::Lo{});
+    } else {
+      constexpr int NW = D == 128 ? 8 : 4;  // eight waves (two per SIMD) at head dim 128
+      LUCID_LAUNCH_B("lucid_precond_fwd_kernel", (lucid::lucid_precond_fwd_kernel<D, false, false, NW>),
+                     dim3((T / 128) * BH), dim3(64 * NW), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T,
+                     BH, w.rinv, w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.link, w.mass,
+                     w.counters, lucid::Lo{});
+    }
   }
   if (g_precision != LUCID_PRECISION_FAST)
     LUCID_LAUNCH("lucid_precond_fwd_exact_kernel", (lucid::lucid_precond_fwd_kernel<D, true>),
                  dim3((T / 128) * BH), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH, w.rinv, w.khat,
-                 scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.zx, w.mass, w.counters, lucid::Lo{});
+                 scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.link, w.mass, w.counters, lucid::Lo{});
   return LUCID_OK;
 }
 
@@ -294,8 +325,8 @@ int launch_fwd(const void* q, const int64_t* qs, const void* k, const int64_t* k
                void* o, const int64_t* os, float* vprime, float* lse, const FwdWs& w, int B, int Hq, int Hkv, int T,
                float scale, float eps, float dn, hipStream_t st) {
   if constexpr (D == 64) {
-    if (Hq == Hkv && g_fused_fwd) {
-      const int BH = B * Hkv;
+    const int BH = B * Hkv;
+    if (Hq == Hkv && g_fused_fwd && !linked_fwd64(BH, T)) {
       const float mass_init = g_precision == LUCID_PRECISION_EXACT ? 1e30f : 0.f;
       LUCID_LAUNCH("lucid_prep_kernel", lucid::lucid_prep_kernel<D>, dim3(T / 64, BH), st, (const bf16*)k, S(ks),
                    Hkv, T, eps, dn, scale, w.rinv, w.kt, w.pinv, w.counters, w.mass, mass_init, lucid::Lo{}, nullptr,
@@ -308,9 +339,12 @@ int launch_fwd(const void* q, const int64_t* qs, const void* k, const int64_t* k
                      vprime, w.vpb, w.vpt, w.pinv, w.zx, w.mass, w.counters, (bf16*)o, S(os), lse);
       if (g_precision != LUCID_PRECISION_FAST) {
         // heads of the exact chains: their chain, then their attention (skip_fast)
+        LUCID_LAUNCH("lucid_link_kernel", (lucid::lucid_link_kernel<D, false, false>), dim3(T / 128, BH), st,
+                     (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, nullptr, w.link, w.mass, 1,
+                     lucid::Lo{});
         LUCID_LAUNCH("lucid_precond_fwd_exact_kernel", (lucid::lucid_precond_fwd_kernel<D, true>),
                      dim3((T / 128) * BH), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH, w.rinv,
-                     w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.zx, w.mass, w.counters,
+                     w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.link, w.mass, w.counters,
                      lucid::Lo{});
         LUCID_LAUNCH("lucid_attn_fwd_exact_kernel", lucid::lucid_attn_fwd_kernel<D>, dim3(((T + 255) / 256) * B * Hq),
                      st, (const bf16*)q, S(qs), (const bf16*)k, S(ks), w.vpt, (bf16*)o, S(os), lse, w.mass, w.olo,
@@ -377,8 +411,11 @@ int launch_precond_bwd(const void* k, const int64_t* ks, const FwdWs& f, void* d
   const int BH = B * Hkv;
   // each chain kernel in two instances (bf16 and exact), selected per head by the forward's
   // row mass; the precision forced at the forward call is recorded there
-  // bf16 chains at head dim 64: 256 columns per workgroup when T allows it
-  if (D == 64 && T % 256 == 0) {
+  // bf16 chains at head dim 64: 256 columns per workgroup for many long heads
+  const bool wide = D == 64 && !linked_bwd64(BH, T);
+  LUCID_LAUNCH("lucid_link_bwd_kernel", (lucid::lucid_link_kernel<D, false, true>), dim3(T / 128, BH), st, (const bf16*)k,
+               S(ks), Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, w.xt, w.link, f.mass, wide, lucid::Lo{});
+  if (wide) {
     LUCID_LAUNCH_B("lucid_precond_bwd_col_wide_kernel", lucid::lucid_precond_bwd_col_wide_kernel<64>,
                    dim3((T / 256) * BH), dim3(512), st, (const bf16*)k, S(ks), Hkv, T, BH, f.rinv, f.khat, scale,
                    f.vpb, f.pinv, f.mass, w.dvp, w.dvb, (bf16*)dv, S(dvs), w.colsum, w.counters);
@@ -387,14 +424,14 @@ int launch_precond_bwd(const void* k, const int64_t* ks, const FwdWs& f, void* d
   // active head-dim columns
   auto col_chains = [&](auto dac) -> int {
     constexpr int DA = decltype(dac)::value;
-    if (!(D == 64 && T % 256 == 0))
+    if (!wide)
       LUCID_LAUNCH("lucid_precond_bwd_col_kernel", (lucid::lucid_precond_bwd_col_kernel<D, false, false, DA>),
                    dim3((T / 128) * BH), st, (const bf16*)k, S(ks), Hkv, T, BH, f.rinv, f.khat, scale, f.kt, f.vpb,
-                   f.vpbl, f.pinv, f.mass, w.dvp, w.dvb, w.dvbl, (bf16*)dv, S(dvs), w.colsum, w.counters,
+                   f.vpbl, w.xt, w.link, f.mass, w.dvp, w.dvb, w.dvbl, (bf16*)dv, S(dvs), w.colsum, w.counters,
                    lucid::Lo{});
     LUCID_LAUNCH("lucid_precond_bwd_col_exact_kernel", (lucid::lucid_precond_bwd_col_kernel<D, true, false, DA>),
                  dim3((T / 128) * BH), st, (const bf16*)k, S(ks), Hkv, T, BH, f.rinv, f.khat, scale, f.kt, f.vpb,
-                 f.vpbl, f.pinv, f.mass, w.dvp, w.dvb, w.dvbl, (bf16*)dv, S(dvs), w.colsum, w.counters, lucid::Lo{});
+                 f.vpbl, w.xt, w.link, f.mass, w.dvp, w.dvb, w.dvbl, (bf16*)dv, S(dvs), w.colsum, w.counters, lucid::Lo{});
     return LUCID_OK;
   };
   int rc_col;
@@ -491,6 +528,8 @@ BwdWs carve_seam_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool attn
     w.dvb = reinterpret_cast<bf16*>(take(BH * T * D * 2));
     w.dvbl = reinterpret_cast<bf16*>(take(BH * T * D * 2));
     w.colsum = reinterpret_cast<float*>(take(BH * T * D * 4));
+    w.xt = reinterpret_cast<bf16*>(take(BH * (T / 128) * 32768 * 2));
+    w.link = reinterpret_cast<bf16*>(take(BH * (T / 128) * 32768 * 2));
   }
   w.counters = reinterpret_cast<int*>(take(BH * 4));
   w.bytes = off;
@@ -597,10 +636,12 @@ int launch_precond_fwd_f32(const void* k, const int64_t* ks, const void* v, cons
                T, eps, dn, scale, w.rinv, w.kt, w.pinv, w.counters, w.mass, kForceExact, lo, w.ktl, nullptr);
   LUCID_LAUNCH("lucid_zx_f32_kernel", (lucid::lucid_zx_kernel<D, true>), dim3(T / 128, BH), st, w.kh, ck, Hkv, T,
                w.rinv, scale, w.pinv, w.zx, lo);
+  LUCID_LAUNCH("lucid_link_f32_kernel", (lucid::lucid_link_kernel<D, true, false>), dim3(T / 128, BH), st, w.kh, ck,
+               Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, nullptr, w.link, w.mass, 0, lo);
   // the chain reads V as fp32 through lo.v with V's own strides (its bf16 operand is unused)
   LUCID_LAUNCH("lucid_precond_fwd_f32_kernel", (lucid::lucid_precond_fwd_kernel<D, true, true>),
                dim3((T / 128) * BH), st, w.kh, ck, (const bf16*)v, S(vs), Hkv, T, BH, w.rinv, nullptr, scale, vprime,
-               w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.zx, w.mass, w.counters, lo);
+               w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.link, w.mass, w.counters, lo);
   return LUCID_OK;
 }
 
@@ -715,10 +756,12 @@ int launch_precond_bwd_f32(const FwdWs& f, void* dk, const int64_t* dks, void* d
   lucid::Lo lo{};
   lo.k = f.kl;
   lo.kt = f.ktl;
+  LUCID_LAUNCH("lucid_link_bwd_f32_kernel", (lucid::lucid_link_kernel<D, true, true>), dim3(T / 128, BH), st, f.kh, ck,
+               Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, w.xt, w.link, f.mass, 0, lo);
   auto col_chain = [&](auto dac) -> int {  // over the active head-dim columns
     LUCID_LAUNCH("lucid_precond_bwd_col_f32_kernel",
                  (lucid::lucid_precond_bwd_col_kernel<D, true, true, decltype(dac)::value>), dim3((T / 128) * BH), st,
-                 f.kh, ck, Hkv, T, BH, f.rinv, nullptr, scale, f.kt, f.vpb, f.vpbl, f.pinv, f.mass, w.dvp, w.dvb,
+                 f.kh, ck, Hkv, T, BH, f.rinv, nullptr, scale, f.kt, f.vpb, f.vpbl, w.xt, w.link, f.mass, w.dvp, w.dvb,
                  w.dvbl, (float*)dv, S(dvs), w.colsum, w.counters, lo);
     return LUCID_OK;
   };

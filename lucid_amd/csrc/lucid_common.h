@@ -145,6 +145,30 @@ __device__ __forceinline__ void publish_counter(int* cnt, int val) {
   }
 }
 
+// Published stores: 16 bytes a lane written through this XCD's L2 (sc1) to the level that
+// every XCD reads, so that no L2 write-back has to precede the counter store.  base: the
+// head's buffer (wave-uniform), off: byte offset below 4 GiB.
+__device__ __forceinline__ void st_pub16(__amdgpu_buffer_rsrc_t base, unsigned off, const bf16x8& v) {
+  constexpr int kSc1 = 16;
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), base, (int)off, 0, kSc1);
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pub_base(void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, -1, 0x00027000);
+}
+
+// Advance the head's chain counter to val once every thread's st_pub16 stores have
+// completed: each wave waits for its own, the barrier orders that before the counter store.
+// Only operands written with st_pub16 are published.  16 KB handed from workgroup to
+// workgroup this way take 1.5-1.7 us a hop; with plain stores and an agent-scope release,
+// which writes back the whole L2, 1.6-2.2 us on an idle chip and more where the L2 holds
+// other kernels' dirty lines.  Every thread must call it.
+__device__ __forceinline__ void publish_stored(int* cnt, int val) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(cnt, val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // 16 consecutive-in-D-layout fp32 values of a per-row vector: rows drow(e, g) + base
 __device__ __forceinline__ void load_rows16(const float* __restrict__ p, int g, float out[16]) {
 #pragma unroll

@@ -10,6 +10,7 @@
 //                            inverses of the 64x64 diagonal blocks of P, zero chain counters
 //   lucid_zx_kernel          the in-block coupling -X_B P_BA of every 128-row chain block and
 //                            (precision "auto") the heads' row masses, lucid_mass_kernel's work
+//   lucid_link_kernel        the coupling of neighbouring 128-row chain blocks (both chains)
 //   lucid_precond_fwd_kernel chained solve, one workgroup per (128-row block, kv head);
 //                            it waits on a per-head progress counter for V'_j, j < i and
 //                            sweeps the earlier keys 128 at a time
@@ -479,71 +480,278 @@ __global__ __launch_bounds__(256) void lucid_zx_kernel(const bf16* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Chained preconditioner solve, 128 rows per workgroup made of two 64-row
-// sub-blocks A (rows i0..i0+63) and B (i0+64..i0+127).
+// Links of the 128-row chains: what couples neighbouring 128-row blocks, precomputed so that
+// a chain's hand-off is one product.  X = the inverse of the block's 128x128 diagonal block of
+// P (fp32: X_A, X_B of lucid_prep_kernel and Y = zx X_A below the diagonal).
+//   forward (BWD = false), block i and its predecessor:  link = -X P_{i,i-1}, so that
+//     V'_i = X R_i + link V'_{i-1}, R_i = V_i - sum over the blocks before i - 1;
+//     y[bh][i] = Y (fp32 64x64, the chain's X_B row needs it)
+//   backward, block i and its successor:  link = -X^T P_{i+1,i}^T, so that
+//     dV_i = X^T R_i + link dV_{i+1}; xt = X^T
+// Both are out[n][m] = -sum_k Xop[n][k] E(k, m), k in block i, m in the other block, with
+// E(k, m) = exp(s r_k r_m K_k.K_m - 1/s) (fp32 inputs: all four hi/lo terms).  link and xt are
+// bf16 hi / lo planes [2][128 rows][128 columns in T-perm order] (the lo plane of a link only
+// for exact heads).  The products of exact heads are fp32
+// MFMAs (bf16 chains: 3-term bf16 splits): along a shared key direction X takes differences of nearly equal rows of E, which
+// 16-bit operands would leave only part of (largest V' error of the fp32 path at T = 1024: 9.9e-4
+// with the splits, 6.2e-4 with fp32 products, 6.5e-4 in a chain without links).  Bound by its
+// traffic (80 KB written per block forward, 96 backward): 64 heads of T = 4096 83 / 98 us
+// with both link planes.  Wave w owns the 32 m's of m-tile w, whose E it holds over all k (a D tile's
+// 16 values are the operands of 16 two-deep steps); Xop is shared through LDS.  exact_only: heads of the bf16 chains return at once
+// (their chain does not read the links).  grid (T/128, B*Hkv)
+// ---------------------------------------------------------------------------
+template <int D, bool F32, bool BWD>
+__global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_link_kernel(
+    const bf16* __restrict__ k, Strides ks, int Hkv, int T, const float* __restrict__ rinv, float scale,
+    const float* __restrict__ pinv, const float* __restrict__ zx, float* __restrict__ y, bf16* __restrict__ xt,
+    bf16* __restrict__ link, const float* __restrict__ mass, int exact_only, Lo lo) {
+  constexpr int NKS = D / 16;
+  __shared__ __attribute__((aligned(16))) union {
+    float XAt[64][68];  // XAt[c][slot of a] = X_A[a][c]
+    float x[128][132];  // Xop rows n, columns k
+  } sm;
+  const int blk = blockIdx.x, bh = blockIdx.y, nblk = T / 128;
+  if (exact_only && !(mass[bh] > kExactMass)) return;
+  const int b = bh / Hkv, h = bh - b * Hkv;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int g = lane >> 5, l32 = lane & 31;
+  const float* pb = pinv + ((int64_t)bh * (T / 64) + 2 * blk) * 4096;  // X_A, then X_B
+  const int64_t ob = ((int64_t)bh * nblk + blk) * 32768;               // this block's planes in link / xt
+
+  // every load up front: the kernel is a few microseconds of work behind one memory latency
+  f32x4 xab[8];  // X_A, X_B: chunk u of 256 threads -> X_A (u < 4) or X_B
+#pragma unroll
+  for (int u = 0; u < 8; ++u) xab[u] = *reinterpret_cast<const f32x4*>(pb + (u >> 2) * 4096 + 4 * (tid + 256 * (u & 3)));
+  const int th = w & 1, tr = w >> 1;
+  f32x4 zq[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    zq[q] = *reinterpret_cast<const f32x4*>(zx + ((int64_t)bh * nblk + blk) * 4096 + (tr * 32 + l32) * 64 + 8 * q + 4 * g);
+  const int oblk = BWD ? blk + 1 : blk - 1;
+  const bool linked = oblk >= 0 && oblk < nblk;
+  const bf16* kp = k + b * ks.b + h * ks.h;
+  const bf16* klp = F32 ? lo.k + b * ks.b + h * ks.h : nullptr;
+  const float* rv = rinv + (int64_t)bh * T;
+  const int orow = (linked ? oblk : blk) * 128 + 32 * w + l32;
+  bf16x8 km[NKS], kk[F32 || D > 64 ? 1 : 4][NKS];
+#pragma unroll
+  for (int st = 0; st < NKS; ++st) {
+    km[st] = ld8(kp + (int64_t)orow * ks.t + 16 * st + 8 * g);
+    if constexpr (!F32 && D == 64) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) kk[kt][st] = ld8(kp + (int64_t)(blk * 128 + 32 * kt + l32) * ks.t + 16 * st + 8 * g);
+    }
+  }
+  const float am = scale * LOG2E_F * rv[orow];
+
+  // ---- Y = zx X_A: wave -> 32x32 quadrant (column half th, row half tr) ----
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int f = 4 * (tid + 256 * u), a = f >> 6, c4 = f & 63;
+    const f32x4 x = xab[u];
+    const int slot = (a & ~15) | jmap(a & 15);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sm.XAt[c4 + e][slot] = x[e];
+  }
+  __syncthreads();
+  f32x16 yq = zero16();  // BWD: D[m = row][n = column]; else D[m = column][n = row]
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(&sm.XAt[th * 32 + l32][8 * q + 4 * g]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) yq = BWD ? mfma32_f32(zq[q][e], x[e], yq) : mfma32_f32(x[e], zq[q][e], yq);
+  }
+  if constexpr (!BWD) {
+    float* yo = y + ((int64_t)bh * nblk + blk) * 4096 + (tr * 32 + l32) * 64 + th * 32 + 4 * g;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<f32x4*>(yo + 8 * q) = f32x4{yq[4 * q], yq[4 * q + 1], yq[4 * q + 2], yq[4 * q + 3]};
+  }
+  __syncthreads();  // XAt is done with
+  // ---- Xop ----
+#pragma unroll
+  for (int q = 0; q < 4; ++q)  // Y's quadrant
+    *reinterpret_cast<f32x4*>(BWD ? &sm.x[th * 32 + l32][64 + tr * 32 + 8 * q + 4 * g]
+                                  : &sm.x[64 + tr * 32 + l32][th * 32 + 8 * q + 4 * g]) =
+        f32x4{yq[4 * q], yq[4 * q + 1], yq[4 * q + 2], yq[4 * q + 3]};
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {  // X_A and X_B
+    const int f = 4 * (tid + 256 * (u & 3)), sb = u >> 2, r = f >> 6, c4 = f & 63;
+    const f32x4 x = xab[u];
+    if constexpr (BWD) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sm.x[64 * sb + c4 + e][64 * sb + r] = x[e];
+    } else {
+      *reinterpret_cast<f32x4*>(&sm.x[64 * sb + r][64 * sb + c4]) = x;
+    }
+  }
+  __syncthreads();
+  if constexpr (BWD) {
+    for (int c = tid; c < 2048; c += 256) {
+      const int r = c >> 4, q = c & 15;
+      if (r >= 64 && q < 8) continue;  // (the zero part of X^T: the chain skips those k-steps)
+      const float* src = &sm.x[r][16 * (q >> 1) + 4 * (q & 1)];  // slots 8q .. 8q+7: positions +0..3, +8..11
+      bf16x8 xh, xl;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = src[(e & 3) + 8 * (e >> 2)];
+        xh[e] = (bf16)v;
+        xl[e] = (bf16)(v - (float)xh[e]);
+      }
+      *reinterpret_cast<bf16x8*>(xt + ob + r * 128 + 8 * q) = xh;
+      *reinterpret_cast<bf16x8*>(xt + ob + 16384 + r * 128 + 8 * q) = xl;
+    }
+  }
+  // ---- E(k, m) of this wave's m-tile over all k ----
+  if (!linked) return;
+  const float c0 = LOG2E_F / scale;
+  f32x16 em[4];
+  {
+    bf16x8 kml[F32 ? NKS : 1];
+    if constexpr (F32) {
+#pragma unroll
+      for (int st = 0; st < NKS; ++st) kml[st] = ld8(klp + (int64_t)orow * ks.t + 16 * st + 8 * g);
+    }
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      const int64_t krow = (int64_t)(blk * 128 + 32 * kt + l32) * ks.t + 8 * g;
+      f32x16 sc = zero16();
+#pragma unroll
+      for (int st = 0; st < NKS; ++st) {
+        bf16x8 ka;
+        if constexpr (!F32 && D == 64) ka = kk[kt][st];
+        else ka = ld8(kp + krow + 16 * st);
+        sc = mfma32(ka, km[st], sc);
+        if constexpr (F32) {
+          const bf16x8 kal = ld8(klp + krow + 16 * st);
+          sc = mfma32(ka, kml[st], sc);
+          sc = mfma32(kal, km[st], sc);
+          sc = mfma32(kal, kml[st], sc);
+        }
+      }
+      float rk[16];
+      load_rows16(rv + blk * 128 + 32 * kt, g, rk);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) em[kt][e] = __builtin_amdgcn_exp2f(fmaf(sc[e] * am, rk[e], -c0));
+    }
+  }
+  // ---- out = -Xop E ----
+  const bool exact = F32 || mass[bh] > kExactMass;
+#pragma unroll 1
+  for (int nt = 0; nt < 4; ++nt) {  // (rolled: run once per workgroup, straight-line code waits for its fetch)
+    f32x16 o = zero16();
+    const float* xrow = &sm.x[32 * nt + l32][4 * g];
+    if (exact) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (BWD ? kt < nt : kt > nt) continue;
+          const f32x4 x = *reinterpret_cast<const f32x4*>(xrow + 32 * kt + 8 * q);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o = mfma32_f32(em[kt][4 * q + e], x[e], o);
+        }
+    } else {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          if (BWD ? kt < nt : kt > nt) continue;
+          const f32x4 x0 = *reinterpret_cast<const f32x4*>(xrow + 32 * kt + 16 * hh);
+          const f32x4 x1 = *reinterpret_cast<const f32x4*>(xrow + 32 * kt + 16 * hh + 8);
+          bf16x8 xh, xl;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float x = e < 4 ? x0[e & 3] : x1[e & 3];
+            xh[e] = (bf16)x;
+            xl[e] = (bf16)(x - (float)xh[e]);
+          }
+          const bf16x8 eh = pack_b(em[kt], hh);
+          o = mfma32(eh, xh, o);
+          o = mfma32(eh, xl, o);
+          o = mfma32(pack_lo(em[kt], hh, eh), xh, o);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[e] = -o[e];
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      bf16* dst = link + ob + (32 * nt + l32) * 128 + 32 * w + 16 * hh + 8 * g;
+      const bf16x8 oh = pack_b(o, hh);
+      *reinterpret_cast<bf16x8*>(dst) = oh;
+      if (exact) *reinterpret_cast<bf16x8*>(dst + 16384) = pack_lo(o, hh, oh);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Chained preconditioner solve, 128 rows per workgroup (two 64-row sub-blocks A and B).
 // Workgroup id -> (i2 = id / BH, bh = id % BH): ids grow with i2, so every
 // wait is on a lower id (in-order dispatch keeps the chain deadlock free) and
 // the blocks of one head share an XCD when BH % 8 == 0.  counters[bh] = number
 // of 64-row blocks of V' already published (whole 128-row blocks at a time).
 //
-// The earlier keys are swept in pairs of 64-key tiles (128 keys per barrier):
-// K^ rows (bf16, the bf16 chains; raw K rows and 1/rms, the exact ones) and V'^T (T-perm)
-// of the pair are staged once per workgroup in LDS by direct global->LDS loads (double
-// buffered, swizzled, no registers).
+// The earlier keys but for the previous block are swept in pairs of 64-key tiles (128 keys
+// per barrier): K^ rows (bf16, the bf16 chains; raw K rows and 1/rms, the exact ones) and
+// V'^T (T-perm) of the pair are staged once per workgroup in LDS by direct global->LDS loads
+// (double buffered, swizzled, no registers).
 // wave w: ih = w & 1 -> rows i0 + 64*ih .. +64 (two 32-row n-tiles, lane <-> row)
 //         kh = w >> 1 -> the 64-key tile 2*pair + kh of every staged pair
 //   acc^T[d][i] += V'^T[d][j] P^T[j][i],  P^T[j][i] = exp(s r_i r_j K_j.K_i - 1/s)
-// (the kh = 0 accumulators start at -V^T).  Then V'_A = X_A R_A and
-// V'_B = X_B R_B + Z V'_A with Z = -(X_B P_BA), R = V - acc, X = P_diag^-1 (fp32, both
-// from lucid_prep_kernel) applied through a 3-term bf16 split (hi*hi + hi*lo + lo*hi),
-// Z through a 2-term split against bf16 V'_A.  The chain's critical path is the work
-// after the last pair becomes visible, so everything that does not depend on it (V,
-// the two inverses, Z) is loaded earlier.  At d = 64 two workgroups share a CU (LDS <= 80 KB,
-// <= 256 registers per lane) so that one's MFMA work overlaps the other's exp.  At d = 128
-// the bf16 chain runs NW = 8 waves (two per SIMD, 220 registers): wave w owns the 32 rows
-// i0 + 32 (w % 4) .. of key half w / 4 (one n-tile instead of two), one solve tile each.
+// (the kh = 0 accumulators start at -V^T).  Then, with R = V - acc,
+//   V'_i = X R + link V'_{i-1},  X = [X_A 0; Y X_B] the inverse of P's diagonal block,
+//   link = -X P_{i,i-1} (lucid_link_kernel),
+// X and R as 3-term bf16 splits (hi*hi + hi*lo + lo*hi), the link in bf16 like the sweep's P
+// (exact: hi and lo).  A chain is bound by its hand-offs where few heads run, so as little as
+// possible stands between the previous block's publish and this one's: the wait, staging 16 KB
+// of V'^T, one 128-deep product, the store and the counter (about 3 us); X R, which
+// needs block i-2, runs beside the previous block's own step, its P taken while block i-2 is
+// being solved.  2 heads of T = 16000 at d = 64: 0.92 ms with the previous block swept like
+// the others and the two sub-blocks solved one after the other (7.3 us a hand-off), 0.57 with
+// links, 0.52 with the last swept pair's P taken ahead (4.2 us); exact 1.24 -> 0.67 ms; 8
+// heads of T = 8192 at d = 128: 0.66 ms (256-row blocks) -> 0.38.  At d = 64 two workgroups
+// share a CU (LDS <= 80 KB, <= 256 registers per lane) so that one's MFMA work overlaps the
+// other's exp.  At d = 128 the bf16 chain runs NW = 8 waves (two per SIMD): wave w owns the 32
+// rows i0 + 32 (w % 4) .. of key half w / 4 (one n-tile instead of two).
 //
 // EXACT (heads whose row mass exceeds kExactMass; the other instance returns at once for
 // them and vice versa): V' is also kept as its bf16 residual lo = bf16(V' - bf16(V'))
 // (vpbl row-major, vptl T-perm), the staged pairs carry the lo tile too, and every
-// off-diagonal product is split: P V' ~= Ph Vh + Pl Vh + Ph Vl, as is Z V'_A.  The
+// off-diagonal product is split: P V' ~= Ph Vh + Pl Vh + Ph Vl, as is link V'_{i-1}.  The
 // extra tile and registers allow one workgroup per CU; at d = 128 the staged pairs are
 // single-buffered (three 32 KB tiles), each pair staged after the previous one's sweep.
 // ---------------------------------------------------------------------------
-template <int D, bool EXACT, bool F32 = false>
-struct PfwdSmem;
-template <int D>
-struct PfwdSmem<D, false, false> {
+// LDS of the block's finish (the bytes of the staging buffers): the cross-wave sum of R, the
+// previous block's V'^T over it, R as hi / lo row tiles and V'^T of the block over them.
+template <int D, bool EXACT>
+struct PfwdFin {
+  union {
+    float Rt[D][132];  // the kh = 1 waves' part of R^T
+    struct {
+      bf16 v[D * 128], vl[EXACT ? D * 128 : 8];  // V'^T of the previous block (swizzled)
+    } p;
+  } a;
   union {
     struct {
-      bf16 k[2][128 * D];  // swizzled tiles (chunk c of row r at c ^ (r & 7))
-      bf16 v[2][D * 128];
-      float r[2][128];
-    } st;
+      bf16 h[128 * D], l[128 * D];  // rows of R (swizzled)
+    } r;
     struct {
-      float Rt[D][132];     // R^T for the 128 rows (cols 0..63 = A, 64..127 = B)
-      float X[64][68];      // inverse of the diagonal block being solved
-      bf16 vT[D][128 + 8];  // V'^T of the block (bf16, T-perm within 16-groups)
-    } fin;
-  } u;
+      bf16 v[D][128 + 8], vl[EXACT ? D : 1][128 + 8];  // V'^T of the block (T-perm within 16-groups)
+    } t;
+  } b;
 };
-template <int D, bool F32>
-struct PfwdSmem<D, true, F32> {
-  static constexpr int NBUF = D == 128 ? 1 : 2;
+template <int D, bool EXACT, bool F32 = false>
+struct PfwdSmem {
+  static constexpr int NBUF = EXACT && D == 128 ? 1 : 2;
   union {
     struct {
-      bf16 k[NBUF][128 * D];
+      bf16 k[NBUF][128 * D];  // swizzled tiles (chunk c of row r at c ^ (r & 7))
       bf16 kl[F32 ? NBUF : 1][F32 ? 128 * D : 8];  // lo part of K (fp32 inputs)
       bf16 v[NBUF][D * 128];
-      bf16 vl[NBUF][D * 128];  // lo part of V'^T
-      float r[NBUF][128];
+      bf16 vl[EXACT ? NBUF : 1][EXACT ? D * 128 : 8];  // lo part of V'^T
+      float r[NBUF][EXACT ? 128 : 4];
     } st;
-    struct {
-      float Rt[D][132];
-      float X[64][68];
-      bf16 vT[D][128 + 8];
-      bf16 vTl[D][128 + 8];  // lo part of V'^T of the block
-    } fin;
+    PfwdFin<D, EXACT> fin;
   } u;
 };
 
@@ -552,8 +760,9 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
     const bf16* __restrict__ k, Strides ks, const bf16* __restrict__ v, Strides vs, int Hkv, int T, int BH,
     const float* __restrict__ rinv, const bf16* __restrict__ khat, float scale, float* __restrict__ vp32,
     bf16* __restrict__ vpb,
-    bf16* __restrict__ vpt, bf16* __restrict__ vpbl, bf16* __restrict__ vptl, float* __restrict__ pinv,
-    const float* __restrict__ zx, const float* __restrict__ mass, int* __restrict__ counters, Lo lo) {
+    bf16* __restrict__ vpt, bf16* __restrict__ vpbl, bf16* __restrict__ vptl, const float* __restrict__ pinv,
+    const float* __restrict__ y, const bf16* __restrict__ link, const float* __restrict__ mass,
+    int* __restrict__ counters, Lo lo) {
   static_assert(EXACT || !F32, "fp32 inputs run the exact chains");
   static_assert(NW == 4 || (NW == 8 && D == 128 && !EXACT), "eight waves: the bf16 chain at head dim 128");
   constexpr int NDT = D / 32;
@@ -630,15 +839,16 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
       }
   }
 
-  // ---- off-diagonal sweep over the i2 earlier pairs of 64-key tiles ----
+  // ---- off-diagonal sweep over the earlier pairs of 64-key tiles, but for the last one
+  // (the previous block), which enters through its link ----
   // pair pp (keys 128pp .. 128pp+127) is complete once the counter exceeds 2pp+1;
   // it is staged into buffer pp & 1 by direct global->LDS loads
-  const int npair = i2;
+  const int npair = i2 > 0 ? i2 - 1 : 0;
   int ready = 0;
   int plan_k[128 * (D / 8) / NTHR], plan_v[D * 16 / NTHR];
   dma_plan<128, D / 8, NTHR>(EXACT ? ks.t : (int64_t)D, plan_k);
   dma_plan<D, 16, NTHR>(T, plan_v);
-  auto stage = [&](int pp) {
+  auto stage_k = [&](int pp) {  // the pair's keys: no part of the chain
     const int buf = SINGLE ? 0 : pp & 1;
     if constexpr (EXACT) {
       if (w < 2) dma_f32x64(rv + pp * 128 + 64 * w, &sm.u.st.r[buf][64 * w]);
@@ -647,38 +857,28 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
       dma_stage<128, D / 8, NTHR>(plan_k, khh + (int64_t)pp * 128 * D, sm.u.st.k[buf]);
     }
     if constexpr (F32) dma_stage<128, D / 8, NTHR>(plan_k, klh + (int64_t)pp * 128 * ks.t, sm.u.st.kl[buf]);
+  };
+  auto stage_v = [&](int pp) {  // its V'^T, once published
+    const int buf = SINGLE ? 0 : pp & 1;
     dma_stage<D, 16, NTHR>(plan_v, vpth + pp * 128, sm.u.st.v[buf]);
     if constexpr (EXACT) dma_stage<D, 16, NTHR>(plan_v, vptlh + pp * 128, sm.u.st.vl[buf]);
   };
-  // the two inverses X_A, X_B (2 x 64 x 64 fp32): chunk u -> sub-block u / XH
-  constexpr int XPER = 2048 / NTHR, XH = XPER / 2;  // 16-byte chunks per thread, per sub-block
-  f32x4 xr[XPER];
-  auto xload = [&]() {
-#pragma unroll
-    for (int u = 0; u < XPER; ++u) {
-      const int idx = tid + NTHR * u;
-      const int sb = idx >> 10, r = (idx >> 4) & 63, c4 = (idx & 15) * 4;
-      xr[u] = *reinterpret_cast<const f32x4*>(pinv_blk + sb * 4096 + r * 64 + c4);
-    }
+  auto stage = [&](int pp) {
+    stage_k(pp);
+    stage_v(pp);
   };
-  auto xstore = [&](int sb) {
-#pragma unroll
-    for (int u = XH * sb; u < XH * sb + XH; ++u) {
-      const int idx = tid + NTHR * u;
-      const int r = (idx >> 4) & 63, c4 = (idx & 15) * 4;
-      *reinterpret_cast<f32x4*>(&sm.u.fin.X[r][c4]) = xr[u];
-    }
+  // P^T of 32 keys (mt) of the wave's key half, as operands of P V'
+  struct PB {
+    bf16x8 hi[NTW][2], lo[EXACT ? NTW : 1][2];
   };
-  auto sweep_pair = [&](int buf) {
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
+  auto scores = [&](int buf, int mt, PB& pbs) __attribute__((always_inline)) {
+    {
       const int key0 = kh * 64 + mt * 32;
       bf16x8 ka[NKS];
 #pragma unroll
       for (int st = 0; st < NKS; ++st) ka[st] = ld8(swz<D / 8>(sm.u.st.k[buf], key0 + l32, 2 * st + g));
       float rj[16];
       if constexpr (EXACT) lds_rows16(&sm.u.st.r[buf][key0], g, rj);
-      bf16x8 pb[NTW][2], pbl[NTW][2];
 #pragma unroll
       for (int nt = 0; nt < NTW; ++nt) {
         f32x16 sc = zero16();
@@ -696,66 +896,89 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
 #pragma unroll
         for (int e = 0; e < 16; ++e)
           sc[e] = __builtin_amdgcn_exp2f(EXACT ? fmaf(sc[e] * ai[nt], rj[e], -c0) : sc[e]);
-        pb[nt][0] = pack_b(sc, 0);
-        pb[nt][1] = pack_b(sc, 1);
+        pbs.hi[nt][0] = pack_b(sc, 0);
+        pbs.hi[nt][1] = pack_b(sc, 1);
         if constexpr (EXACT) {
-          pbl[nt][0] = pack_lo(sc, 0, pb[nt][0]);
-          pbl[nt][1] = pack_lo(sc, 1, pb[nt][1]);
+          pbs.lo[nt][0] = pack_lo(sc, 0, pbs.hi[nt][0]);
+          pbs.lo[nt][1] = pack_lo(sc, 1, pbs.hi[nt][1]);
         }
       }
+    }
+  };
+  auto pv = [&](int buf, int mt, const PB& pbs) __attribute__((always_inline)) {
+    {
+      const int key0 = kh * 64 + mt * 32;
 #pragma unroll
       for (int t = 0; t < NDT; ++t) {
         const bf16x8 va0 = ld8(swz<16>(sm.u.st.v[buf], t * 32 + l32, key0 / 8 + g));
         const bf16x8 va1 = ld8(swz<16>(sm.u.st.v[buf], t * 32 + l32, key0 / 8 + 2 + g));
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt) {
-          acc[t][nt] = mfma32(va0, pb[nt][0], acc[t][nt]);
-          acc[t][nt] = mfma32(va1, pb[nt][1], acc[t][nt]);
+          acc[t][nt] = mfma32(va0, pbs.hi[nt][0], acc[t][nt]);
+          acc[t][nt] = mfma32(va1, pbs.hi[nt][1], acc[t][nt]);
         }
         if constexpr (EXACT) {
           const bf16x8 vl0 = ld8(swz<16>(sm.u.st.vl[buf], t * 32 + l32, key0 / 8 + g));
           const bf16x8 vl1 = ld8(swz<16>(sm.u.st.vl[buf], t * 32 + l32, key0 / 8 + 2 + g));
 #pragma unroll
           for (int nt = 0; nt < NTW; ++nt) {
-            acc[t][nt] = mfma32(va0, pbl[nt][0], acc[t][nt]);
-            acc[t][nt] = mfma32(va1, pbl[nt][1], acc[t][nt]);
-            acc[t][nt] = mfma32(vl0, pb[nt][0], acc[t][nt]);
-            acc[t][nt] = mfma32(vl1, pb[nt][1], acc[t][nt]);
+            acc[t][nt] = mfma32(va0, pbs.lo[nt][0], acc[t][nt]);
+            acc[t][nt] = mfma32(va1, pbs.lo[nt][1], acc[t][nt]);
+            acc[t][nt] = mfma32(vl0, pbs.hi[nt][0], acc[t][nt]);
+            acc[t][nt] = mfma32(vl1, pbs.hi[nt][1], acc[t][nt]);
           }
         }
       }
     }
   };
+  auto sweep_pair = [&](int buf) {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      PB pbs;
+      scores(buf, mt, pbs);
+      pv(buf, mt, pbs);
+    }
+  };
+  // the last swept pair's keys are staged and its P^T taken while its V' is still being
+  // solved, so that only P V' follows its publish
+  const int lastp = npair - 1;
   if (npair > 0) {
-    ready = wait_counter_gt(cnt, 1);
-    stage(0);
+    if (npair > 1) ready = wait_counter_gt(cnt, 1);
+    stage_k(0);
+    if (npair > 1) stage_v(0);
     dma_wait();
-  } else {
-    xload();
   }
   __syncthreads();
-  // all pairs but the last; the last one is peeled so that the inverses it
-  // prefetches do not hold registers through the loop
-  for (int pp = 0; pp + 1 < npair; ++pp) {
+  for (int pp = 0; pp < lastp; ++pp) {
+    const bool tolast = pp + 1 == lastp;
     const int need = 2 * pp + 3;  // pair pp + 1 is complete once the counter exceeds this
     if constexpr (SINGLE) {
       sweep_pair(0);
       __syncthreads();  // every wave is done with the buffer
-      if (need >= ready) ready = wait_counter_gt(cnt, need);
-      stage(pp + 1);
+      if (tolast) {
+        stage_k(pp + 1);
+      } else {
+        if (need >= ready) ready = wait_counter_gt(cnt, need);
+        stage(pp + 1);
+      }
       dma_wait();
       __syncthreads();
       continue;
     }
-    if (need >= ready) {
-      const int seen = poll_counter(cnt);
-      if (seen > need) {
-        chain_acquire();
-        ready = seen;
+    bool early = tolast;
+    if (tolast) {
+      stage_k(pp + 1);
+    } else {
+      if (need >= ready) {
+        const int seen = poll_counter(cnt);
+        if (seen > need) {
+          chain_acquire();
+          ready = seen;
+        }
       }
+      early = need < ready;
+      if (early) stage(pp + 1);
     }
-    const bool early = need < ready;
-    if (early) stage(pp + 1);
     sweep_pair(pp & 1);
     if (!early) {
       ready = wait_counter_gt(cnt, need);
@@ -764,118 +987,164 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
     dma_wait();
     __syncthreads();
   }
+
+  // ---- the block: V'_i = X R + link V'_{i-1}, X = [X_A 0; Y X_B] ----
+  // wave -> 32 rows (wr) and DW 32-column tiles of V'^T from dt0
+  auto& fin = sm.u.fin;
+  const int wu = __builtin_amdgcn_readfirstlane(w);
+  const int wr = wu & 3;
+  constexpr int DW = NDT * 4 / NW;
+  const int dt0 = (wu >> 2) * DW;
+  // this wave's rows of X as hi / lo, k-steps 0 .. 2 wr + 1; slots 8g .. 8g+7 of a 16-group
+  // hold columns 4g .. +3 and 8 + 4g .. +3
+  bf16x8 xh[8], xl[8];
+#pragma unroll
+  for (int st = 0; st < 8; ++st) {
+    if (st >= 2 * wr + 2) continue;
+    const int rl = (wr & 1) * 32 + l32;
+    const float* src = (wr < 2 ? pinv_blk + rl * 64 + 16 * st
+                        : st < 4 ? y + ((int64_t)bh * (T / 128) + i2) * 4096 + rl * 64 + 16 * st
+                                 : pinv_blk + 4096 + rl * 64 + 16 * (st - 4)) + 4 * g;
+    f32x4 xr[2];
+    xr[0] = *reinterpret_cast<const f32x4*>(src);
+    xr[1] = *reinterpret_cast<const f32x4*>(src + 8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = xr[e >> 2][e & 3];
+      xh[st][e] = (bf16)x;
+      xl[st][e] = (bf16)(x - (float)xh[st][e]);
+    }
+  }
   if (npair > 0) {
-    xload();  // fetch the inverses while the last pair is processed
-    sweep_pair(SINGLE ? 0 : (npair - 1) & 1);
+    const int buf = SINGLE ? 0 : lastp & 1;
+    PB pbs[2];
+    scores(buf, 0, pbs[0]);
+    scores(buf, 1, pbs[1]);
+    if (2 * npair - 1 >= ready) ready = wait_counter_gt(cnt, 2 * npair - 1);
+    stage_v(lastp);
+    dma_wait();
+    __syncthreads();
+    pv(buf, 0, pbs[0]);
+    pv(buf, 1, pbs[1]);
     __syncthreads();
   }
-
-  // ---- reduce the key halves: R^T = -(acc_0 + acc_1) (Rt columns = rows of this workgroup) ----
-  float(*Rt)[132] = sm.u.fin.Rt;
+  // R = -(acc_0 + acc_1), split into hi / lo row tiles
   if (kh == 1) {
 #pragma unroll
     for (int t = 0; t < NDT; ++t)
 #pragma unroll
       for (int nt = 0; nt < NTW; ++nt)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) Rt[t * 32 + drow(e, g)][ih * 32 * NTW + nt * 32 + l32] = acc[t][nt][e];
+        for (int e = 0; e < 16; ++e) fin.a.Rt[t * 32 + drow(e, g)][ih * 32 * NTW + nt * 32 + l32] = acc[t][nt][e];
   }
-  xstore(0);
   __syncthreads();
   if (kh == 0) {
 #pragma unroll
-    for (int t = 0; t < NDT; ++t)
+    for (int nt = 0; nt < NTW; ++nt) {
+      const int row = ih * 32 * NTW + nt * 32 + l32;
 #pragma unroll
-      for (int nt = 0; nt < NTW; ++nt)
+      for (int t = 0; t < NDT; ++t)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          float& x = Rt[t * 32 + drow(e, g)][ih * 32 * NTW + nt * 32 + l32];
-          x = -Cf * (acc[t][nt][e] + x);
+        for (int qd = 0; qd < 4; ++qd) {
+          const int d0 = t * 32 + 8 * qd + 4 * g;
+          bf16x4 rh, rl;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const float x = -Cf * (acc[t][nt][4 * qd + u] + fin.a.Rt[d0 + u][row]);
+            rh[u] = (bf16)x;
+            rl[u] = (bf16)(x - (float)rh[u]);
+          }
+          const int off = swz_off<D / 8>(row, d0 >> 3) + (d0 & 7);
+          *reinterpret_cast<bf16x4*>(fin.b.r.h + off) = rh;
+          *reinterpret_cast<bf16x4*>(fin.b.r.l + off) = rl;
         }
+    }
   }
-  // Z rows of this wave's B output tiles (row half rh = w & 1), 8 columns per lane half and
-  // 16-column step, fetched while sub-block A is solved
-  f32x4 zr[4][2];
+  __syncthreads();
+  f32x16 o[DW];
+#pragma unroll
+  for (int t = 0; t < DW; ++t) o[t] = zero16();
+#pragma unroll
+  for (int st = 0; st < 8; ++st) {
+    if (st >= 2 * wr + 2) continue;
+#pragma unroll
+    for (int t = 0; t < DW; ++t) {
+      const bf16x8 ah = lds_tr_a<D / 8>(fin.b.r.h, 16 * st, (dt0 + t) * 32);
+      const bf16x8 al = lds_tr_a<D / 8>(fin.b.r.l, 16 * st, (dt0 + t) * 32);
+      o[t] = mfma32(ah, xh[st], o[t]);
+      o[t] = mfma32(ah, xl[st], o[t]);
+      o[t] = mfma32(al, xh[st], o[t]);
+    }
+  }
+  if (i2 > 0) {  // the link's rows before the wait, V'^T of the previous block after it
+    const bf16* lrow = link + ((int64_t)bh * (T / 128) + i2) * 32768 + (32 * wr + l32) * 128 + 8 * g;
+    bf16x8 zh[8], zl[8];
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      zh[st] = ld8(lrow + 16 * st);
+      if constexpr (EXACT) zl[st] = ld8(lrow + 16384 + 16 * st);
+    }
+    if (2 * i2 - 1 >= ready) wait_counter_gt(cnt, 2 * i2 - 1);
+    dma_stage<D, 16, NTHR>(plan_v, vpth + (i2 - 1) * 128, fin.a.p.v);
+    if constexpr (EXACT) dma_stage<D, 16, NTHR>(plan_v, vptlh + (i2 - 1) * 128, fin.a.p.vl);
+    dma_wait();
+    __syncthreads();  // (every wave is done with R too)
+#pragma unroll
+    for (int st = 0; st < 8; ++st)
+#pragma unroll
+      for (int t = 0; t < DW; ++t) {
+        const bf16x8 va = ld8(swz<16>(fin.a.p.v, (dt0 + t) * 32 + l32, 2 * st + g));
+        o[t] = mfma32(va, zh[st], o[t]);
+        if constexpr (EXACT) {
+          o[t] = mfma32(va, zl[st], o[t]);
+          o[t] = mfma32(ld8(swz<16>(fin.a.p.vl, (dt0 + t) * 32 + l32, 2 * st + g)), zh[st], o[t]);
+        }
+      }
+  } else {
+    __syncthreads();
+  }
+  // V'^T to the T-perm operand copy through this wave's own columns of fin.b.t, then published
+  const int lslot = 32 * wr + ((l32 & ~15) | jmap(l32 & 15));
+#pragma unroll
+  for (int t = 0; t < DW; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const bf16 hi = (bf16)o[t][e];
+      fin.b.t.v[(dt0 + t) * 32 + drow(e, g)][lslot] = hi;
+      if constexpr (EXACT) fin.b.t.vl[(dt0 + t) * 32 + drow(e, g)][lslot] = (bf16)(o[t][e] - (float)hi);
+    }
+  __builtin_amdgcn_wave_barrier();
   {
-    const float* zrow = zx + ((int64_t)bh * (T / 128) + i2) * 4096 + ((w & 1) * 32 + l32) * 64 + 8 * g;
+    const __amdgpu_buffer_rsrc_t ph = pub_base(vpt + (int64_t)bh * D * T);
+    const __amdgpu_buffer_rsrc_t pl = pub_base(EXACT ? vptl + (int64_t)bh * D * T : nullptr);
 #pragma unroll
-    for (int st = 0; st < 4; ++st) {
-      zr[st][0] = *reinterpret_cast<const f32x4*>(zrow + 16 * st);
-      zr[st][1] = *reinterpret_cast<const f32x4*>(zrow + 16 * st + 4);
+    for (int u = 0; u < 2 * DW; ++u) {
+      const int idx = lane + 64 * u, dd = dt0 * 32 + (idx >> 2), s8 = 32 * wr + (idx & 3) * 8;
+      const unsigned off = 2u * ((unsigned)dd * (unsigned)T + (unsigned)(i0 + s8));
+      st_pub16(ph, off, ld8(&fin.b.t.v[dd][s8]));
+      if constexpr (EXACT) st_pub16(pl, off, ld8(&fin.b.t.vl[dd][s8]));
     }
   }
-  __syncthreads();
-
-  // V'^T[d][r] = sum_c R^T[d][c] X[r][c] for sub-block sb (X lower triangular)
-  auto diag_solve = [&](int sb) {
-    for (int tile = w; tile < NDT * 2; tile += NW) {
-      const int dt = tile >> 1, rh = tile & 1;
-      f32x16 o = zero16();
-      const int kmax = rh ? 4 : 2;
-      for (int st = 0; st < kmax; ++st) {
-        bf16x8 ah, al, bh8, bl;
-        split8(&Rt[dt * 32 + l32][sb * 64 + 16 * st + 8 * g], ah, al);
-        split8(&sm.u.fin.X[rh * 32 + l32][16 * st + 8 * g], bh8, bl);
-        o = mfma32(ah, bh8, o);
-        o = mfma32(ah, bl, o);
-        o = mfma32(al, bh8, o);
+  publish_stored(cnt, 2 * i2 + 2);
+  // the rows of V' (fp32 and bf16): nothing in this kernel waits for them
+  const int64_t orow = ((int64_t)bh * T + i0 + 32 * wr + l32) * D;
+#pragma unroll
+  for (int t = 0; t < DW; ++t)
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) {
+      const int d0 = (dt0 + t) * 32 + 8 * qd + 4 * g;
+      f32x4 f;
+      bf16x4 bb, bl;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        f[u] = o[t][4 * qd + u];
+        bb[u] = (bf16)f[u];
+        bl[u] = (bf16)(f[u] - (float)bb[u]);
       }
-      if (sb == 1) {  // + Z V'_A: V'_A^T from the bf16 T-perm tile, Z split into hi + lo
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          bf16x8 zh, zl;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float x = zr[st][e >> 2][e & 3];
-            zh[e] = (bf16)x;
-            zl[e] = (bf16)(x - (float)zh[e]);
-          }
-          const bf16x8 va = ld8(&sm.u.fin.vT[dt * 32 + l32][16 * st + 8 * g]);
-          o = mfma32(va, zh, o);
-          o = mfma32(va, zl, o);
-          if constexpr (EXACT) o = mfma32(ld8(&sm.u.fin.vTl[dt * 32 + l32][16 * st + 8 * g]), zh, o);
-        }
-      }
-      const int rl = rh * 32 + l32;
-      const int r = i0 + sb * 64 + rl;
-      const int lslot = sb * 64 + ((rl & ~15) | jmap(rl & 15));
-      float* out32 = vp32 + ((int64_t)bh * T + r) * D;
-      bf16* outb = vpb + ((int64_t)bh * T + r) * D;
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const int d0 = dt * 32 + 8 * qd + 4 * g;
-        f32x4 f;
-        bf16x4 bb, bl;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          f[u] = o[4 * qd + u];
-          bb[u] = (bf16)o[4 * qd + u];
-          sm.u.fin.vT[d0 + u][lslot] = bb[u];
-          if constexpr (EXACT) {
-            bl[u] = (bf16)(o[4 * qd + u] - (float)bb[u]);
-            sm.u.fin.vTl[d0 + u][lslot] = bl[u];
-          }
-        }
-        *reinterpret_cast<f32x4*>(out32 + d0) = f;
-        *reinterpret_cast<bf16x4*>(outb + d0) = bb;
-        if constexpr (EXACT) *reinterpret_cast<bf16x4*>(vpbl + ((int64_t)bh * T + r) * D + d0) = bl;
-      }
+      *reinterpret_cast<f32x4*>(vp32 + orow + d0) = f;
+      *reinterpret_cast<bf16x4*>(vpb + orow + d0) = bb;
+      if constexpr (EXACT) *reinterpret_cast<bf16x4*>(vpbl + orow + d0) = bl;
     }
-  };
-  diag_solve(0);
-  __syncthreads();
-  xstore(1);
-  __syncthreads();
-  diag_solve(1);
-  __syncthreads();
-  // V'^T of the whole block to the T-perm operand copy: 16-byte stores
-  for (int c = tid; c < D * 16; c += NTHR) {
-    const int dd = c >> 4, s8 = (c & 15) * 8;
-    *reinterpret_cast<bf16x8*>(vpt + ((int64_t)bh * D + dd) * T + i0 + s8) = ld8(&sm.u.fin.vT[dd][s8]);
-    if constexpr (EXACT)
-      *reinterpret_cast<bf16x8*>(vptl + ((int64_t)bh * D + dd) * T + i0 + s8) = ld8(&sm.u.fin.vTl[dd][s8]);
-  }
-  publish_counter(cnt, 2 * i2 + 2);
 }
 
 // ---------------------------------------------------------------------------
@@ -1475,7 +1744,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void l
 // Fused forward at head dim 64 (bf16, one query head per kv head): the chained
 // preconditioner solve of one 128-row block and the causal attention of the same 128
 // query rows in one workgroup, so that every staged key tile and every LDS operand read
-// feeds both.  The chain (ids, counters, staging, finalisation) is lucid_precond_fwd_kernel's;
+// feeds both.  The chain (ids, counters, staging) is lucid_precond_fwd_kernel's, but sweeps the
+// previous block too and solves sub-block A, then B: V'_A = X_A R_A, V'_B = X_B R_B + zx V'_A;
 // the attention is lucid_attn_fwd_kernel's online softmax.  Wave w owns rows
 // i0 + 32w .. +32 (lane <-> row) of both and sweeps all 128 keys of each staged pair as
 // four 32-key sub-tiles mt:
@@ -1489,6 +1759,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void l
 // attention kernel with skip_fast cover them).
 // ---------------------------------------------------------------------------
 template <int D>
+struct FusedSmem {
+  union {
+    struct {
+      bf16 k[2][128 * D];  // swizzled tiles (chunk c of row r at c ^ (r & 7))
+      bf16 v[2][D * 128];
+      float r[2][128];
+    } st;
+    struct {
+      float Rt[D][132];     // R^T for the 128 rows (cols 0..63 = A, 64..127 = B)
+      float X[64][68];      // inverse of the diagonal block being solved
+      bf16 vT[D][128 + 8];  // V'^T of the block (bf16, T-perm within 16-groups)
+    } fin;
+  } u;
+};
+template <int D>
 __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_fused_fwd_kernel(
     const bf16* __restrict__ q, Strides qs, const bf16* __restrict__ k, Strides ks, const bf16* __restrict__ v,
     Strides vs, int Hkv, int T, int BH, const float* __restrict__ rinv, float scale, float* __restrict__ vp32,
@@ -1498,7 +1783,7 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_fused_fwd_
   static_assert(D == 64, "fused forward: head dim 64");
   constexpr int NDT = D / 32;
   constexpr int NKS = D / 16;
-  __shared__ __attribute__((aligned(16))) PfwdSmem<D, false, false> sm;
+  __shared__ __attribute__((aligned(16))) FusedSmem<D> sm;
 
   const int id = blockIdx.x;
   const int i2 = id / BH, bh = id - (id / BH) * BH;
