@@ -69,12 +69,11 @@ struct FwdWs {
   bf16* vpt;     // [BH][D][T]  V'^T, T-perm
   float* pinv;   // [BH][T/64][64][64]  inverses of the diagonal blocks of P
   float* zx;     // [BH][T/128][64][64] -(X_B P_BA) per 128-row block, columns T-perm
-  float* y;      // [BH][T/128][64][64] zx X_A: the inverse of the 128-row block below X_A
-  bf16* link;    // [BH][T/128][2][128][128] -X_i P_{i,i-1}, hi / lo planes, columns T-perm (lucid_link_kernel)
   bf16* vpbl;    // [BH][T][D]  lo part of V' (exact heads)
   bf16* vptl;    // [BH][D][T]  lo part of V'^T, T-perm (exact heads)
   float* mass;   // [BH]        largest row mass sum_{j<i} P_ij^2 (sampled; selects the chain precision)
   bf16* olo;     // [BHq][T][D] lo part of O (exact heads)
+  float* y;      // olo's bytes until the attention: zx X_A per 128-row block (lucid_link_kernel)
   int* counters; // [BH]
   // fp32 inputs only: the bf16 pairs of Q and K ([BH][T][D] rows), K^T's lo part, the
   // mean key of each head (fp32 [BH][D]) and the pair of K - mean (the attention's keys)
@@ -108,12 +107,11 @@ FwdWs carve_fwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = fal
   w.vpt = reinterpret_cast<bf16*>(take(BH * D * T * 2));
   w.pinv = reinterpret_cast<float*>(take(BH * (T / 64) * 4096 * 4));
   w.zx = reinterpret_cast<float*>(take(BH * (T / 128) * 4096 * 4));
-  w.y = reinterpret_cast<float*>(take(BH * (T / 128) * 4096 * 4));
-  w.link = reinterpret_cast<bf16*>(take(BH * (T / 128) * 32768 * 2));
   w.vpbl = reinterpret_cast<bf16*>(take(BH * T * D * 2));
   w.vptl = reinterpret_cast<bf16*>(take(BH * D * T * 2));
   w.mass = reinterpret_cast<float*>(take(BH * 4));
   w.olo = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
+  w.y = reinterpret_cast<float*>(w.olo);  // 128 bytes a row and kv head: at most olo's
   w.counters = reinterpret_cast<int*>(take(BH * 4));
   if (f32) {
     if (with_q) {
@@ -259,7 +257,8 @@ int launch_precond_fwd(const void* k, const int64_t* ks, const void* v, const in
   // the 256-row chain keeps its own in-block coupling; only the exact heads read links then
   const bool wide = D == 128 && !linked_fwd128(BH, T);
   LUCID_LAUNCH("lucid_link_kernel", (lucid::lucid_link_kernel<D, false, false>), dim3(T / 128, BH), st,
-               (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, nullptr, w.link, w.mass, wide,
+               (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, vprime, w.vpbl, w.khat,
+               nullptr, nullptr, w.mass, wide,
                lucid::Lo{});
   // both instances of the chain: each solves the heads of its precision and returns at
   // once for the others
@@ -272,14 +271,14 @@ int launch_precond_fwd(const void* k, const int64_t* ks, const void* v, const in
       constexpr int NW = D == 128 ? 8 : 4;  // eight waves (two per SIMD) at head dim 128
       LUCID_LAUNCH_B("lucid_precond_fwd_kernel", (lucid::lucid_precond_fwd_kernel<D, false, false, NW>),
                      dim3((T / 128) * BH), dim3(64 * NW), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T,
-                     BH, w.rinv, w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.link, w.mass,
+                     BH, w.rinv, w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.mass,
                      w.counters, lucid::Lo{});
     }
   }
   if (g_precision != LUCID_PRECISION_FAST)
     LUCID_LAUNCH("lucid_precond_fwd_exact_kernel", (lucid::lucid_precond_fwd_kernel<D, true>),
                  dim3((T / 128) * BH), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH, w.rinv, w.khat,
-                 scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.link, w.mass, w.counters, lucid::Lo{});
+                 scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.mass, w.counters, lucid::Lo{});
   return LUCID_OK;
 }
 
@@ -340,11 +339,12 @@ int launch_fwd(const void* q, const int64_t* qs, const void* k, const int64_t* k
       if (g_precision != LUCID_PRECISION_FAST) {
         // heads of the exact chains: their chain, then their attention (skip_fast)
         LUCID_LAUNCH("lucid_link_kernel", (lucid::lucid_link_kernel<D, false, false>), dim3(T / 128, BH), st,
-                     (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, nullptr, w.link, w.mass, 1,
+                     (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, vprime, w.vpbl, w.khat,
+                     nullptr, nullptr, w.mass, 1,
                      lucid::Lo{});
         LUCID_LAUNCH("lucid_precond_fwd_exact_kernel", (lucid::lucid_precond_fwd_kernel<D, true>),
                      dim3((T / 128) * BH), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH, w.rinv,
-                     w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.link, w.mass, w.counters,
+                     w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.mass, w.counters,
                      lucid::Lo{});
         LUCID_LAUNCH("lucid_attn_fwd_exact_kernel", lucid::lucid_attn_fwd_kernel<D>, dim3(((T + 255) / 256) * B * Hq),
                      st, (const bf16*)q, S(qs), (const bf16*)k, S(ks), w.vpt, (bf16*)o, S(os), lse, w.mass, w.olo,
@@ -414,7 +414,8 @@ int launch_precond_bwd(const void* k, const int64_t* ks, const FwdWs& f, void* d
   // bf16 chains at head dim 64: 256 columns per workgroup for many long heads
   const bool wide = D == 64 && !linked_bwd64(BH, T);
   LUCID_LAUNCH("lucid_link_bwd_kernel", (lucid::lucid_link_kernel<D, false, true>), dim3(T / 128, BH), st, (const bf16*)k,
-               S(ks), Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, w.xt, w.link, f.mass, wide, lucid::Lo{});
+               S(ks), Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, nullptr, nullptr,
+               nullptr, w.xt, w.link, f.mass, wide, lucid::Lo{});
   if (wide) {
     LUCID_LAUNCH_B("lucid_precond_bwd_col_wide_kernel", lucid::lucid_precond_bwd_col_wide_kernel<64>,
                    dim3((T / 256) * BH), dim3(512), st, (const bf16*)k, S(ks), Hkv, T, BH, f.rinv, f.khat, scale,
@@ -637,11 +638,12 @@ int launch_precond_fwd_f32(const void* k, const int64_t* ks, const void* v, cons
   LUCID_LAUNCH("lucid_zx_f32_kernel", (lucid::lucid_zx_kernel<D, true>), dim3(T / 128, BH), st, w.kh, ck, Hkv, T,
                w.rinv, scale, w.pinv, w.zx, lo);
   LUCID_LAUNCH("lucid_link_f32_kernel", (lucid::lucid_link_kernel<D, true, false>), dim3(T / 128, BH), st, w.kh, ck,
-               Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, nullptr, w.link, w.mass, 0, lo);
+               Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, vprime, w.vpbl, w.khat,
+               nullptr, nullptr, w.mass, 0, lo);
   // the chain reads V as fp32 through lo.v with V's own strides (its bf16 operand is unused)
   LUCID_LAUNCH("lucid_precond_fwd_f32_kernel", (lucid::lucid_precond_fwd_kernel<D, true, true>),
-               dim3((T / 128) * BH), st, w.kh, ck, (const bf16*)v, S(vs), Hkv, T, BH, w.rinv, nullptr, scale, vprime,
-               w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.link, w.mass, w.counters, lo);
+               dim3((T / 128) * BH), st, w.kh, ck, (const bf16*)v, S(vs), Hkv, T, BH, w.rinv, w.khat, scale, vprime,
+               w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.mass, w.counters, lo);
   return LUCID_OK;
 }
 
@@ -757,7 +759,8 @@ int launch_precond_bwd_f32(const FwdWs& f, void* dk, const int64_t* dks, void* d
   lo.k = f.kl;
   lo.kt = f.ktl;
   LUCID_LAUNCH("lucid_link_bwd_f32_kernel", (lucid::lucid_link_kernel<D, true, true>), dim3(T / 128, BH), st, f.kh, ck,
-               Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, w.xt, w.link, f.mass, 0, lo);
+               Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, nullptr, nullptr, nullptr, w.xt,
+               w.link, f.mass, 0, lo);
   auto col_chain = [&](auto dac) -> int {  // over the active head-dim columns
     LUCID_LAUNCH("lucid_precond_bwd_col_f32_kernel",
                  (lucid::lucid_precond_bwd_col_kernel<D, true, true, decltype(dac)::value>), dim3((T / 128) * BH), st,

@@ -490,8 +490,11 @@ __global__ __launch_bounds__(256) void lucid_zx_kernel(const bf16* __restrict__ 
 //     dV_i = X^T R_i + link dV_{i+1}; xt = X^T
 // Both are out[n][m] = -sum_k Xop[n][k] E(k, m), k in block i, m in the other block, with
 // E(k, m) = exp(s r_k r_m K_k.K_m - 1/s) (fp32 inputs: all four hi/lo terms).  link and xt are
-// bf16 hi / lo planes [2][128 rows][128 columns in T-perm order] (the lo plane of a link only
-// for exact heads).  The products of exact heads are fp32
+// bf16 hi / lo planes [128 rows][128 columns in T-perm order] (the lo plane of a link only for
+// exact heads).  The forward's links take no workspace of their own: row n of block i's hi
+// plane lies in V' row n of the block (vp32), the halves of its lo row in rows n of vpbl and of
+// khat (which the exact chains do not read), and y in olo; block i's workgroup reads them before
+// it, alone, writes V' and its lo part there, and the attention writes olo later still.  The products of exact heads are fp32
 // MFMAs (bf16 chains: 3-term bf16 splits): along a shared key direction X takes differences of nearly equal rows of E, which
 // 16-bit operands would leave only part of (largest V' error of the fp32 path at T = 1024: 9.9e-4
 // with the splits, 6.2e-4 with fp32 products, 6.5e-4 in a chain without links).  Bound by its
@@ -503,8 +506,9 @@ __global__ __launch_bounds__(256) void lucid_zx_kernel(const bf16* __restrict__ 
 template <int D, bool F32, bool BWD>
 __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_link_kernel(
     const bf16* __restrict__ k, Strides ks, int Hkv, int T, const float* __restrict__ rinv, float scale,
-    const float* __restrict__ pinv, const float* __restrict__ zx, float* __restrict__ y, bf16* __restrict__ xt,
-    bf16* __restrict__ link, const float* __restrict__ mass, int exact_only, Lo lo) {
+    const float* __restrict__ pinv, const float* __restrict__ zx, float* __restrict__ y, float* __restrict__ vp32,
+    bf16* __restrict__ vpbl, bf16* __restrict__ khat, bf16* __restrict__ xt, bf16* __restrict__ link,
+    const float* __restrict__ mass, int exact_only, Lo lo) {
   constexpr int NKS = D / 16;
   __shared__ __attribute__((aligned(16))) union {
     float XAt[64][68];  // XAt[c][slot of a] = X_A[a][c]
@@ -676,10 +680,15 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_link_kerne
     for (int e = 0; e < 16; ++e) o[e] = -o[e];
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
-      bf16* dst = link + ob + (32 * nt + l32) * 128 + 32 * w + 16 * hh + 8 * g;
+      const int n = 32 * nt + l32, m = 32 * w + 16 * hh + 8 * g;
+      const int64_t row = (int64_t)bh * T + blk * 128 + n;
       const bf16x8 oh = pack_b(o, hh);
-      *reinterpret_cast<bf16x8*>(dst) = oh;
-      if (exact) *reinterpret_cast<bf16x8*>(dst + 16384) = pack_lo(o, hh, oh);
+      bf16* dh = BWD ? link + ob + n * 128 + m : reinterpret_cast<bf16*>(vp32 + row * D) + m;
+      *reinterpret_cast<bf16x8*>(dh) = oh;
+      if (exact) {
+        bf16* dl = BWD ? dh + 16384 : (m < 64 ? vpbl : khat) + row * D + (m & 63);
+        *reinterpret_cast<bf16x8*>(dl) = pack_lo(o, hh, oh);
+      }
     }
   }
 }
@@ -761,8 +770,7 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
     const float* __restrict__ rinv, const bf16* __restrict__ khat, float scale, float* __restrict__ vp32,
     bf16* __restrict__ vpb,
     bf16* __restrict__ vpt, bf16* __restrict__ vpbl, bf16* __restrict__ vptl, const float* __restrict__ pinv,
-    const float* __restrict__ y, const bf16* __restrict__ link, const float* __restrict__ mass,
-    int* __restrict__ counters, Lo lo) {
+    const float* __restrict__ y, const float* __restrict__ mass, int* __restrict__ counters, Lo lo) {
   static_assert(EXACT || !F32, "fp32 inputs run the exact chains");
   static_assert(NW == 4 || (NW == 8 && D == 128 && !EXACT), "eight waves: the bf16 chain at head dim 128");
   constexpr int NDT = D / 32;
@@ -1077,12 +1085,13 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
     }
   }
   if (i2 > 0) {  // the link's rows before the wait, V'^T of the previous block after it
-    const bf16* lrow = link + ((int64_t)bh * (T / 128) + i2) * 32768 + (32 * wr + l32) * 128 + 8 * g;
+    const int64_t lrow = ((int64_t)bh * T + i0 + 32 * wr + l32) * D;
+    const bf16* lhi = reinterpret_cast<const bf16*>(vp32 + lrow) + 8 * g;
     bf16x8 zh[8], zl[8];
 #pragma unroll
     for (int st = 0; st < 8; ++st) {
-      zh[st] = ld8(lrow + 16 * st);
-      if constexpr (EXACT) zl[st] = ld8(lrow + 16384 + 16 * st);
+      zh[st] = ld8(lhi + 16 * st);
+      if constexpr (EXACT) zl[st] = ld8((st < 4 ? vpbl : khat) + lrow + 16 * (st & 3) + 8 * g);
     }
     if (2 * i2 - 1 >= ready) wait_counter_gt(cnt, 2 * i2 - 1);
     dma_stage<D, 16, NTHR>(plan_v, vpth + (i2 - 1) * 128, fin.a.p.v);
