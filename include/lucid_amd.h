@@ -339,6 +339,14 @@ int lucid_causal_lm_loss_fwd(const void* logits, int64_t row_stride, const int64
 int lucid_causal_lm_loss_bwd(const void* logits, int64_t row_stride, const int64_t* labels, int R, int T, int V,
                              const float* lse, const float* valid, const float* scale, void* dlogits, void* stream);
 
+/* Zero-pad n (1 to 3) tensors [B, H[i], T, d] of one dtype (LUCID_DTYPE_BF16 or
+ * LUCID_DTYPE_F32), element strides strides[3 i ..] of their first three axes, unit stride on
+ * the last, into contiguous [B, H[i], Tp, dp] tensors (dst 16-byte aligned, dp a multiple of 8):
+ * the operands of the entry points above from ragged T or other head dims, in one launch (the
+ * reference pads with torch ops, run_clm_chunk.py:517-610). */
+int lucid_pad_rows(int n, const void* const* src, const int64_t* strides, const int* H, void* const* dst, int B, int T,
+                   int Tp, int d, int dp, int dtype, void* stream);
+
 /* One AdamW step (decoupled weight decay) over n parameter tensors, the update of
  * torch.optim.AdamW, the default optimizer of the HF Trainer that the reference's training
  * script builds (run_clm_chunk.py:776; no counterpart in modeling_lucid.py):

@@ -1607,6 +1607,37 @@ int lucid_causal_lm_loss_bwd(const void* logits, int64_t row_stride, const int64
   return LUCID_OK;
 }
 
+int lucid_pad_rows(int n, const void* const* src, const int64_t* strides, const int* H, void* const* dst, int B, int T,
+                   int Tp, int d, int dp, int dtype, void* stream) {
+  g_last_error.clear();
+  if (n < 1 || n > 3 || (dtype != LUCID_DTYPE_BF16 && dtype != LUCID_DTYPE_F32))
+    return fail("lucid_pad_rows: 1 to 3 tensors, dtype LUCID_DTYPE_BF16 or LUCID_DTYPE_F32");
+  if (B <= 0 || T <= 0 || Tp < T || d <= 0 || dp < d || dp % 8)
+    return fail("lucid_pad_rows: B, T, d positive, Tp >= T, dp >= d and a multiple of 8");
+  const int es = dtype == LUCID_DTYPE_F32 ? 4 : 2;
+  lucid::PadTensors p{};
+  int most = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!src[i] || !dst[i] || H[i] <= 0) return fail("lucid_pad_rows: null tensor or no heads");
+    if (reinterpret_cast<uintptr_t>(src[i]) % es || reinterpret_cast<uintptr_t>(dst[i]) % 16)
+      return fail("lucid_pad_rows: src must be element aligned, dst 16-byte aligned");
+    p.src[i] = src[i];
+    p.dst[i] = dst[i];
+    p.st[i] = S(strides + 3 * i);
+    p.H[i] = H[i];
+    most = H[i] > most ? H[i] : most;
+  }
+  const int64_t blocks = ((int64_t)B * most * Tp * (dp * es / 16) + 255) / 256;
+  if (blocks > (int64_t)0x7fffffff) return fail("grid too large");
+  const dim3 grid((unsigned)blocks, n);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (es == 2)
+    LUCID_LAUNCH("lucid_pad_kernel", lucid::lucid_pad_kernel<uint16_t>, grid, st, p, B, T, Tp, d, dp);
+  else
+    LUCID_LAUNCH("lucid_pad_kernel", lucid::lucid_pad_kernel<uint32_t>, grid, st, p, B, T, Tp, d, dp);
+  return LUCID_OK;
+}
+
 int lucid_adamw_step(int n, void* const* params, const void* const* grads, void* const* exp_avgs,
                      void* const* exp_avg_sqs, const int64_t* numels, int dtype, float lr, float beta1, float beta2,
                      float eps, float weight_decay, int64_t step, void* stream) {

@@ -130,6 +130,54 @@ __global__ __launch_bounds__(256) void lucid_prep_kernel(const bf16* __restrict_
 }
 
 // ---------------------------------------------------------------------------
+// Zero-padding of up to three [B, H_i, T, d] tensors (any strides, unit stride on d) into
+// contiguous [B, H_i, Tp, dp] ones, one launch for a call's operands: 16-byte chunks of the
+// output, from 16- or 8-byte loads where the source's address allows, element by element
+// otherwise (and at the last columns).  HBM bound; a small call's launch count is what it
+// saves (a fill and a copy per tensor before: 24 us of the 250 of B2 H8 T333 d64 forward and
+// backward).  grid (chunks of the largest tensor / 256, tensors)
+// ---------------------------------------------------------------------------
+struct PadTensors {
+  const void* src[3];
+  void* dst[3];
+  Strides st[3];
+  int H[3];
+};
+template <typename E>  // uint16_t (bf16) or uint32_t (fp32)
+__global__ __launch_bounds__(256) void lucid_pad_kernel(PadTensors p, int B, int T, int Tp, int d, int dp) {
+  constexpr int PER = 16 / sizeof(E);
+  typedef E chunk __attribute__((ext_vector_type(PER)));
+  typedef E half __attribute__((ext_vector_type(PER / 2)));
+  const int i = blockIdx.y, H = p.H[i], cpr = dp / PER;
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = c / cpr;
+  if (row >= (int64_t)B * H * Tp) return;
+  const int col = (int)(c - row * cpr) * PER;
+  const int t = (int)(row % Tp), bh = (int)(row / Tp);
+  chunk x = {};
+  if (t < T && col < d) {
+    const E* src = static_cast<const E*>(p.src[i]) + (int64_t)(bh / H) * p.st[i].b + (int64_t)(bh % H) * p.st[i].h +
+                   (int64_t)t * p.st[i].t + col;
+    const uintptr_t at = reinterpret_cast<uintptr_t>(src);
+    if (col + PER <= d && at % 16 == 0) {
+      x = *reinterpret_cast<const chunk*>(src);
+    } else if (col + PER <= d && at % 8 == 0) {
+      const half lo = *reinterpret_cast<const half*>(src), hi = *reinterpret_cast<const half*>(src + PER / 2);
+#pragma unroll
+      for (int e = 0; e < PER / 2; ++e) {
+        x[e] = lo[e];
+        x[PER / 2 + e] = hi[e];
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < PER; ++e)
+        if (col + e < d) x[e] = src[e];
+    }
+  }
+  reinterpret_cast<chunk*>(p.dst[i])[c] = x;
+}
+
+// ---------------------------------------------------------------------------
 // Operands of the attention on a caller's V' (eager_lucid_attention_forward): V' rows
 // (bf16 or fp32, strided) to the bf16 row-major copy vpb and the T-perm copy vpt the
 // attention kernels read, 1/rms of K for the row-mass pass, and the head's row mass

@@ -22,6 +22,7 @@ leaves every dot product unchanged; the RMS of k_norm divides by the true d.
 from __future__ import annotations
 
 import contextlib
+import ctypes
 
 import torch
 import torch.nn.functional as F
@@ -67,10 +68,27 @@ def _check_inputs(q, k, v, f32_ok=False):
             raise ValueError("lucid_amd: number of query heads must be a multiple of key/value heads")
 
 
+def _pad_rows(ts, tp: int, dp: int) -> list[torch.Tensor]:
+    """Up to three non-empty GPU tensors [B, H_i, T, d] of one dtype zero-padded to contiguous
+    [B, H_i, tp, dp], one launch."""
+    lib = _lib.load()
+    ts = [t if t.stride(-1) == 1 else t.contiguous() for t in ts]
+    B, _, T, d = ts[0].shape
+    n, dev = len(ts), ts[0].device
+    outs = [torch.empty(B, t.shape[1], tp, dp, dtype=t.dtype, device=dev) for t in ts]
+    rc = lib.lucid_pad_rows(n, (ctypes.c_void_p * n)(*(t.data_ptr() for t in ts)),
+                            (ctypes.c_int64 * (3 * n))(*(s for t in ts for s in t.stride()[:3])),
+                            (ctypes.c_int * n)(*(t.shape[1] for t in ts)),
+                            (ctypes.c_void_p * n)(*(t.data_ptr() for t in outs)), B, T, tp, d, dp,
+                            1 if ts[0].dtype == torch.float32 else 0, _lib.stream_handle(dev))
+    _lib.check(lib, rc, "lucid_pad_rows")
+    return outs
+
+
 def _prep(t: torch.Tensor, tp: int) -> torch.Tensor:
     """Pad the time axis (dim 2) to ``tp`` and make the last axis contiguous with 8-aligned strides."""
     if t.shape[2] != tp:
-        t = F.pad(t, (0, 0, 0, tp - t.shape[2]))
+        return _pad_rows((t,), tp, t.shape[3])[0]
     if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:3]) or t.data_ptr() % 16:
         t = t.contiguous()
     return t
@@ -166,6 +184,18 @@ def _bwd(do, q, k, o, lse, ws, scale, eps, dn, layouts=(False, False, False)):
     return dq, dk, dv
 
 
+def _prep_do(do: torch.Tensor, dtype: torch.dtype, tp: int, dp: int) -> torch.Tensor:
+    """dO [B, T, H, d] in ``dtype`` as the kernels read it: padded to [B, tp, H, dp], unit stride on
+    the last axis, 8-element strides, 16-byte aligned."""
+    if do.dtype != dtype:
+        do = do.to(dtype)
+    if do.shape[1] != tp or do.shape[3] != dp:
+        return _pad_rows((do.transpose(1, 2),), tp, dp)[0].transpose(1, 2)
+    if do.stride(-1) != 1 or any(s % 8 for s in do.stride()) or do.data_ptr() % 16:
+        do = do.contiguous()
+    return do
+
+
 class LucidAttentionFunction(torch.autograd.Function):
     """O = softmax(s Q K^T, causal) (P^-1 V) with HIP forward and backward kernels.
 
@@ -182,8 +212,11 @@ class LucidAttentionFunction(torch.autograd.Function):
             B, Hq, _, D = q.shape
             return (q.new_empty(B, t, Hq, D),
                     torch.empty(B, k.shape[1], t, D, dtype=torch.float32, device=q.device))
-        tp = _padded_len(t)
-        qp, kp, vp_ = _prep(q, tp), _prep(k, tp), _prep(v, tp)
+        tp, dp = _padded_len(t), _padded_dim(dn)
+        if t != tp or dn != dp:
+            qp, kp, vp_ = _pad_rows((q, k, v), tp, dp)
+        else:
+            qp, kp, vp_ = _prep(q, tp), _prep(k, tp), _prep(v, tp)
         ctx.f32 = q.dtype == torch.float32
         o, vprime, lse, ws = (_fwd_f32 if ctx.f32 else _fwd)(qp, kp, vp_, scale, eps, dn)
         ctx.save_for_backward(qp, kp, o, lse, ws)
@@ -194,7 +227,7 @@ class LucidAttentionFunction(torch.autograd.Function):
         # no zero-filled gradient for the V' output, which the backward ignores (a T x d fp32
         # fill per call otherwise)
         ctx.set_materialize_grads(False)
-        return o[:, :t], vprime[:, :, :t]
+        return o[:, :t, :, :dn], vprime[:, :, :t, :dn]
 
     @staticmethod
     def backward(ctx, do, _dvprime):
@@ -204,19 +237,13 @@ class LucidAttentionFunction(torch.autograd.Function):
             return (do.new_zeros(ctx.shapes[0]), do.new_zeros(ctx.shapes[1]), do.new_zeros(ctx.shapes[1]),
                     None, None, None)
         qp, kp, o, lse, ws = ctx.saved_tensors
-        t, tp = ctx.t, qp.shape[2]
-        dt = torch.float32 if ctx.f32 else torch.bfloat16
-        if do.dtype != dt:
-            do = do.to(dt)
-        if t != tp:
-            do = F.pad(do, (0, 0, 0, 0, 0, tp - t))
-        if do.stride(-1) != 1 or any(s % 8 for s in do.stride()) or do.data_ptr() % 16:
-            do = do.contiguous()
+        t, tp, dn, dp = ctx.t, qp.shape[2], ctx.dn, qp.shape[3]
+        do = _prep_do(do, torch.float32 if ctx.f32 else torch.bfloat16, tp, dp)
         if ctx.f32:
             dq, dk, dv = _bwd_f32(do, qp, kp, o, lse, ws, ctx.scale, ctx.dn, ctx.layouts)
         else:
             dq, dk, dv = _bwd(do, qp, kp, o, lse, ws, ctx.scale, ctx.eps, ctx.dn, ctx.layouts)
-        return dq[:, :, :t], dk[:, :, :t], dv[:, :, :t], None, None, None
+        return dq[:, :, :t, :dn], dk[:, :, :t, :dn], dv[:, :, :t, :dn], None, None, None
 
 
 _PRECISIONS = {"auto": 0, "fast": 1, "exact": 2}
@@ -301,11 +328,7 @@ def lucid_attention(query, key, value, scaling=None, eps=1e-5, return_vprime=Fal
     _check_inputs(query, key, value, f32_ok=True)
     d = query.shape[-1]
     scale = d ** -0.5 if scaling is None else float(scaling)
-    dp = _padded_dim(d)
-    q, k, v = (_pad_d(t, dp) for t in (query, key, value))
-    o, vprime = LucidAttentionFunction.apply(q, k, v, scale, eps, d)
-    if dp != d:
-        o, vprime = o[..., :d], vprime[..., :d]
+    o, vprime = LucidAttentionFunction.apply(query, key, value, scale, eps, d)
     return (o, vprime) if return_vprime else o
 
 
@@ -453,13 +476,7 @@ class AttentionOnVPrimeFunction(torch.autograd.Function):
         lib = _lib.load()
         B, Hq, tp, D = qp.shape
         Hkv, t, dn = kp.shape[1], ctx.t, ctx.dn
-        dt = torch.float32 if ctx.f32in else torch.bfloat16
-        if do.dtype != dt:
-            do = do.to(dt)
-        if t != tp:
-            do = F.pad(do, (0, 0, 0, 0, 0, tp - t))
-        if do.stride(-1) != 1 or any(s % 8 for s in do.stride()) or do.data_ptr() % 16:
-            do = do.contiguous()
+        do = _prep_do(do, torch.float32 if ctx.f32in else torch.bfloat16, tp, D)
         dev = qp.device
         if ctx.f32in:
             dq = torch.empty(B, Hq, tp, D, dtype=torch.float32, device=dev)
@@ -595,7 +612,7 @@ def lucid_decode(query, key, value, key_cache, vprime_cache, cache_len, scaling=
     cap = key_cache.shape[2]
     if L == 0:
         return (query.new_empty(B, 0, Hq, d), torch.empty(B, Hkv, 0, d, dtype=torch.float32, device=query.device))
-    q, k, v = (_prep(_pad_d(t, D), L) for t in (query, key, value))
+    q, k, v = _pad_rows((query, key, value), L, D) if d != D else (_prep(t, L) for t in (query, key, value))
     o = torch.empty(B, L, Hq, D, dtype=torch.bfloat16, device=q.device)
     vp_new = torch.empty(B, Hkv, L, D, dtype=torch.float32, device=q.device)
     ws = torch.empty(max(lib.lucid_decode_tokens_workspace_bytes(B, Hq, Hkv, L, cap, d), 256), dtype=torch.uint8,
