@@ -835,17 +835,19 @@ int launch_precond_only_bwd_f32(const void* dvp, const int64_t* dvps, const FwdW
 
 // Decoding: split the cached sequence so that one resident round of split workgroups
 // runs (at least 64 keys per split): the split kernel holds two workgroups per CU at
-// head dim 128 (66 KB of LDS each) and four at 64, on 256 CUs.  Monotone in Tp, so the
-// workspace sized for the capacity covers every call.
-int decode_splits(int BH, int Tp, int D) {
+// head dim 128 (66 KB of LDS each) and four at 64, half as many with two column tiles, on
+// 256 CUs.  Monotone in Tp, so the workspace sized for the capacity covers every call.
+int decode_splits(int BH, int Tp, int D, int NCT) {
   if (Tp <= 0) return 0;
-  const int wgs = padded_dim(D) == 128 ? 512 : 1024;
+  const int wgs = (padded_dim(D) == 128 ? 512 : 1024) / NCT;
   const int want = (wgs + BH - 1) / BH, most = (Tp + 63) / 64;
   return want < most ? want : most;
 }
 
-// Tokens per split/combine pass: the L (G + 1) columns of one 32-column score tile.
-int decode_pass_tokens(int G) { return 32 / (G + 1); }
+// Tokens per split/combine pass: the L (G + 1) columns of one 32-column score tile, or of two
+// (the instances for groups of 4 and 8) where L needs them.
+int decode_col_tiles(int G, int L) { return (G == 4 || G == 8) && L > 32 / (G + 1) ? 2 : 1; }
+int decode_pass_tokens(int G, int L) { return 32 * decode_col_tiles(G, L) / (G + 1); }
 
 // Query heads per kv head are decoded in chunks of at most 31 (a chunk's query columns and
 // the preconditioner row of each token share one 32-column score tile): G <= 31 is one
@@ -882,16 +884,16 @@ lucid::DecodePartials carve_decode(void* base, int BH, int G, int L, int nsplit,
 // chunk of query heads at a time: the chunks run in turn on the same partials).
 size_t decode_ws_bytes(int BH, int G, int L, int T_end, int D) {
   const int Gs = decode_groups(G).gs;
-  const int Lp = L < decode_pass_tokens(Gs) ? L : decode_pass_tokens(Gs);
+  const int Lp = L < decode_pass_tokens(Gs, L) ? L : decode_pass_tokens(Gs, L);
   size_t n = 0;
-  carve_decode(nullptr, BH, Gs, Lp, decode_splits(BH, T_end, D), D, &n);
+  carve_decode(nullptr, BH, Gs, Lp, decode_splits(BH, T_end, D, decode_col_tiles(Gs, L)), D, &n);
   return n;
 }
 
 // L new tokens in passes of LM tokens: each pass reads the cache once (split kernel) and
 // appends its tokens (combine kernel), so the next pass sees them.  The Gs query heads
 // g0 .. g0+Gs-1 of each kv head's Gt; G > 0: the instance for Gs = G.
-template <int D, int G>
+template <int D, int G, int NCT>
 int launch_decode(const void* q, const int64_t* qs, const void* k, const int64_t* ks, const void* v,
                   const int64_t* vs, void* kc, const int64_t* kcs, void* vc, const int64_t* vcs, void* o,
                   const int64_t* os, float* vp_new, void* ws, int B, int Hkv, int L, int Tp, float scale, float eps,
@@ -899,18 +901,18 @@ int launch_decode(const void* q, const int64_t* qs, const void* k, const int64_t
   const int BH = B * Hkv;
   for (int t0 = 0; t0 < L; t0 += LM) {
     const int Lc = L - t0 < LM ? L - t0 : LM, Tc = Tp + t0;
-    const int ns = decode_splits(BH, Tc, D);
+    const int ns = decode_splits(BH, Tc, D, NCT);
     const lucid::DecodePartials part = carve_decode(ws, BH, Gs, Lc, ns, D, nullptr);
     const bf16* qc = (const bf16*)q + t0 * qs[2];
     const bf16* kn = (const bf16*)k + t0 * ks[2];
     const bf16* vn = (const bf16*)v + t0 * vs[2];
     if (ns > 0) {
       const int KS = (Tc + ns - 1) / ns;
-      LUCID_LAUNCH("lucid_decode_split_kernel", (lucid::lucid_decode_split_kernel<D, G>), dim3(ns, BH), st, qc,
+      LUCID_LAUNCH("lucid_decode_split_kernel", (lucid::lucid_decode_split_kernel<D, G, NCT>), dim3(ns, BH), st, qc,
                    S(qs), kn, S(ks), (const bf16*)kc, S(kcs), (const bf16*)vc, S(vcs), Hkv, Tc, KS, Lc, scale, eps,
                    dn, part, Gs, Gt, g0);
     }
-    LUCID_LAUNCH("lucid_decode_combine_kernel", (lucid::lucid_decode_combine_kernel<D, G>), dim3(BH, Gs), st, ns,
+    LUCID_LAUNCH("lucid_decode_combine_kernel", (lucid::lucid_decode_combine_kernel<D, G, NCT>), dim3(BH, Gs), st, ns,
                  Lc, qc, S(qs), kn, S(ks), vn, S(vs), (bf16*)kc, S(kcs), (bf16*)vc, S(vcs),
                  (bf16*)o + t0 * os[2], S(os), vp_new + (size_t)t0 * D, L, Hkv, Tc, scale, eps, dn, part, Gs, Gt, g0,
                  write_cache);
@@ -923,23 +925,24 @@ int decode_dispatch_g(int G, const void* q, const int64_t* qs, const void* k, co
                       const int64_t* vs, void* kc, const int64_t* kcs, void* vc, const int64_t* vcs, void* o,
                       const int64_t* os, float* vp_new, void* ws, int B, int Hkv, int L, int Tp, float scale,
                       float eps, float dn, hipStream_t st) {
-#define LUCID_DECODE_G(GI) \
-  launch_decode<D, GI>(q, qs, k, ks, v, vs, kc, kcs, vc, vcs, o, os, vp_new, ws, B, Hkv, L, Tp, scale, eps, dn, st, G, G, 0, \
-                       decode_pass_tokens(G), 1)
+#define LUCID_DECODE_G(GI, NCT)                                                                                          \
+  launch_decode<D, GI, NCT>(q, qs, k, ks, v, vs, kc, kcs, vc, vcs, o, os, vp_new, ws, B, Hkv, L, Tp, scale, eps, dn, st, \
+                            G, G, 0, decode_pass_tokens(G, L), 1)
+  const bool two = decode_col_tiles(G, L) == 2;
   switch (G) {  // the common groupings as their own instances
-    case 1: return LUCID_DECODE_G(1);
-    case 2: return LUCID_DECODE_G(2);
-    case 4: return LUCID_DECODE_G(4);
-    case 8: return LUCID_DECODE_G(8);
+    case 1: return LUCID_DECODE_G(1, 1);
+    case 2: return LUCID_DECODE_G(2, 1);
+    case 4: return two ? LUCID_DECODE_G(4, 2) : LUCID_DECODE_G(4, 1);
+    case 8: return two ? LUCID_DECODE_G(8, 2) : LUCID_DECODE_G(8, 1);
     default: break;
   }
 #undef LUCID_DECODE_G
   // any other group: the generic instance, in chunks of query heads above 31
   const DecodeGroups dg = decode_groups(G);
-  const int LM = decode_pass_tokens(dg.gs);
+  const int LM = decode_pass_tokens(dg.gs, 1);
   for (int c = 0; c < dg.chunks; ++c) {
     const int g0 = c * dg.gs, gs = G - g0 < dg.gs ? G - g0 : dg.gs;
-    if (int rc = launch_decode<D, 0>(q, qs, k, ks, v, vs, kc, kcs, vc, vcs, o, os, vp_new, ws, B, Hkv, L, Tp, scale,
+    if (int rc = launch_decode<D, 0, 1>(q, qs, k, ks, v, vs, kc, kcs, vc, vcs, o, os, vp_new, ws, B, Hkv, L, Tp, scale,
                                      eps, dn, st, gs, G, g0, LM, c == 0))
       return rc;
   }

@@ -23,12 +23,16 @@ namespace lucid {
 
 constexpr float DEC_NEG = -1e30f;  // finite "minus infinity" for empty softmax states
 
-// Tokens of one pass: the L (G + 1) columns of a 32-column score tile.  G = 0 is the
+// Tokens of one pass: the L (G + 1) columns of NCT 32-column score tiles.  G = 0 is the
 // generic instance (the group size Gs a runtime argument, 3 <= Gs <= 31): its per-token
-// arrays hold the 8 tokens of its smallest group.
-template <int G>
+// arrays hold the 8 tokens of its smallest group.  NCT = 2 (groups of 4 and 8, calls of more
+// tokens than one tile takes): one read of the cache and one combine for twice the tokens, at
+// one wave per SIMD at head dim 128 (B8 Hq32 Hkv4 d68, 2900 rows, 5 tokens: two passes of
+// 24 + 13 us, 74.8 us a call; one pass 28 + 13, 44.6; Hq32 Hkv8 d128, 128K rows, 12 tokens
+// 311 -> 217 us).
+template <int G, int NCT>
 constexpr int decode_tokens_per_pass() {
-  return G > 0 ? 32 / (G + 1) : 8;
+  return G > 0 ? 32 * NCT / (G + 1) : 8;
 }
 
 struct DecodePartials {
@@ -51,61 +55,72 @@ struct DecodePartials {
 // The columns hold the Gs query heads g0 .. g0+Gs-1 of the kv head's Gt (query head
 // h Gt + g0 + i); G > 0 fixes Gs = G at compile time, G = 0 takes Gs at run time.  A key
 // column's partials do not depend on the other columns of the tile.
-template <int D, int G>
+template <int D>
 struct DecodeMfmaSmem {
   union {
     bf16 v[4][2][32 * D];  // per wave, double buffered, swizzled (chunk c of row r at c ^ (r & 7))
     struct {
-      float so[4][32][D];  // per wave: the columns of O^T
+      float so[4][32][D + 1];  // per wave: the columns of O^T (of one column tile at a time)
       float m[4][32], l[4][32];
     } fin;
   } u;
   float nn[4][32];  // per wave: squared norms of the tile's keys
 };
 
-template <int D, int G>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void lucid_decode_split_kernel(
+template <int D, int G, int NCT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((D == 64 ? 4 : 2) / NCT))) void lucid_decode_split_kernel(
     const bf16* __restrict__ q, Strides qs, const bf16* __restrict__ kn, Strides kns,
     const bf16* __restrict__ kc, Strides kcs, const bf16* __restrict__ vc, Strides vcs, int Hkv, int Tp, int KS,
     int L, float scale, float eps, float dn, DecodePartials part, int Gs, int Gt, int g0) {
   constexpr int NKS = D / 16, NDT = D / 32, CPR = D / 8, NST = 32 * CPR / 64;  // NST: staging loads per tile
   static_assert(G + 1 <= 32, "query heads + the preconditioner row must fit one 32-column tile");
   const int GG = G > 0 ? G : Gs;  // query columns per token (GG + 1 <= 32, checked by the host)
-  __shared__ __attribute__((aligned(16))) DecodeMfmaSmem<D, G> sm;
+  __shared__ __attribute__((aligned(16))) DecodeMfmaSmem<D> sm;
   const int s = blockIdx.x, bh = blockIdx.y, BH = gridDim.y;
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 5, l32 = lane & 31;
-  const int col = l32;  // score / output column of this lane
-  const int tok = col / (GG + 1), hi = col - tok * (GG + 1);
-  const bool valid = tok < L, isq = valid && hi < GG, isk = valid && hi == GG;
   const int j0 = s * KS, j1 = min(Tp, j0 + KS);
+  const float sl2 = scale * LOG2E_F, c0 = LOG2E_F / scale;
 
-  // B operand: column col of X^T (k = d), zero for the padding columns
-  bf16x8 xb[NKS];
-  float nt = 0.f;
+  // B operand: column col = 32 ct + l32 of X^T (k = d), zero for the padding columns
+  bool valid[NCT], isq[NCT];
+  bf16x8 xb[NCT][NKS];
+  float c1[NCT];
 #pragma unroll
-  for (int st = 0; st < NKS; ++st) {
-    bf16x8 x;
-    if (isq) {
-      x = ld8(q + b * qs.b + (h * Gt + g0 + hi) * qs.h + (int64_t)tok * qs.t + 16 * st + 8 * g);
-    } else if (isk) {
-      x = ld8(kn + b * kns.b + h * kns.h + (int64_t)tok * kns.t + 16 * st + 8 * g);
+  for (int ct = 0; ct < NCT; ++ct) {
+    const int col = 32 * ct + l32, tok = col / (GG + 1), hi = col - tok * (GG + 1);
+    valid[ct] = tok < L;
+    isq[ct] = valid[ct] && hi < GG;
+    const bool isk = valid[ct] && hi == GG;
+    float nt = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) nt = fmaf((float)x[e], (float)x[e], nt);
-    } else {
+    for (int st = 0; st < NKS; ++st) {
+      bf16x8 x;
+      if (isq[ct]) {
+        x = ld8(q + b * qs.b + (h * Gt + g0 + hi) * qs.h + (int64_t)tok * qs.t + 16 * st + 8 * g);
+      } else if (isk) {
+        x = ld8(kn + b * kns.b + h * kns.h + (int64_t)tok * kns.t + 16 * st + 8 * g);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = (bf16)0.f;
+        for (int e = 0; e < 8; ++e) nt = fmaf((float)x[e], (float)x[e], nt);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = (bf16)0.f;
+      }
+      xb[ct][st] = x;
     }
-    xb[st] = x;
+    nt = wave_sum32(nt);  // squared norm of this column's key (both lane halves)
+    c1[ct] = sl2 * rsqrtf(nt / dn + eps);
   }
-  nt = wave_sum32(nt);  // squared norm of this column's key (both lane halves)
-  const float rt = rsqrtf(nt / dn + eps);
-  const float sl2 = scale * LOG2E_F, c1 = sl2 * rt, c0 = LOG2E_F / scale;
 
-  f32x16 oacc[NDT];
+  f32x16 oacc[NCT][NDT];
+  float m[NCT], l[NCT];
 #pragma unroll
-  for (int t = 0; t < NDT; ++t) oacc[t] = zero16();
-  float m = DEC_NEG, l = 0.f;
+  for (int ct = 0; ct < NCT; ++ct) {
+    m[ct] = DEC_NEG;
+    l[ct] = 0.f;
+#pragma unroll
+    for (int t = 0; t < NDT; ++t) oacc[ct][t] = zero16();
+  }
 
   const bf16* kbase = kc + b * kcs.b + h * kcs.h;
   const bf16* vbase = vc + b * vcs.b + h * vcs.h;
@@ -138,11 +153,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     }
     const int jb = j0 + 32 * t;
     // scores and the squared norms of the tile's keys
-    f32x16 sc = zero16();
+    f32x16 scs[NCT];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) scs[ct] = zero16();
     float nn = 0.f;
 #pragma unroll
     for (int st = 0; st < NKS; ++st) {
-      sc = mfma32(kcur[st], xb[st], sc);
+#pragma unroll
+      for (int ct = 0; ct < NCT; ++ct) scs[ct] = mfma32(kcur[st], xb[ct][st], scs[ct]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) nn = fmaf((float)kcur[st][e], (float)kcur[st][e], nn);
     }
@@ -150,31 +168,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     if (g == 0) sm.nn[w][l32] = nn;
     float nr[16];
     lds_rows16(&sm.nn[w][0], g, nr);
-    // online max of the query columns (lazy: rescale only when a row grows by 2^8)
-    float mx = DEC_NEG;
+    // 1/rms of the keys: once for both column tiles, at the use with one (registers)
+    if constexpr (NCT > 1) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-      if (jb + drow(e, g) < j1) mx = fmaxf(mx, sc[e]);
-    mx = isq ? wave_max32(mx) * sl2 : DEC_NEG;
-    if (__builtin_amdgcn_ballot_w64(mx > m + 8.0f)) {
-      const float mnew = fmaxf(m, mx);
-      const float al = __builtin_amdgcn_exp2f(m - mnew);
-      m = mnew;
-      l *= al;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) oacc[dt][e] *= isq ? al : 1.f;
+      for (int e = 0; e < 16; ++e) nr[e] = rsqrtf(nr[e] / dn + eps);
     }
+    bf16x8 p0[NCT], p1[NCT];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const bool ok = jb + drow(e, g) < j1 && valid;
-      const float arg = isq ? fmaf(sc[e], sl2, -m) : fmaf(c1 * rsqrtf(nr[e] / dn + eps), sc[e], -c0);
-      const float p = ok ? __builtin_amdgcn_exp2f(arg) : 0.f;
-      if (isq) l += p;
-      sc[e] = p;
+    for (int ct = 0; ct < NCT; ++ct) {
+      f32x16& sc = scs[ct];
+      // online max of the query columns (lazy: rescale only when a row grows by 2^8)
+      float mx = DEC_NEG;
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (jb + drow(e, g) < j1) mx = fmaxf(mx, sc[e]);
+      mx = isq[ct] ? wave_max32(mx) * sl2 : DEC_NEG;
+      if (__builtin_amdgcn_ballot_w64(mx > m[ct] + 8.0f)) {
+        const float mnew = fmaxf(m[ct], mx);
+        const float al = __builtin_amdgcn_exp2f(m[ct] - mnew);
+        m[ct] = mnew;
+        l[ct] *= al;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) oacc[ct][dt][e] *= isq[ct] ? al : 1.f;
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const bool ok = jb + drow(e, g) < j1 && valid[ct];
+        const float arg = isq[ct] ? fmaf(sc[e], sl2, -m[ct]) : fmaf(c1[ct] * (NCT > 1 ? nr[e] : rsqrtf(nr[e] / dn + eps)), sc[e], -c0);
+        const float p = ok ? __builtin_amdgcn_exp2f(arg) : 0.f;
+        if (isq[ct]) l[ct] += p;
+        sc[e] = p;
+      }
+      p0[ct] = pack_b(sc, 0);
+      p1[ct] = pack_b(sc, 1);
     }
-    const bf16x8 p0 = pack_b(sc, 0), p1 = pack_b(sc, 1);
     // this tile's V' rows have landed once at most the next tile's loads are in flight
     if (more)
       dma_wait_but<NKS + NST>();
@@ -183,51 +212,64 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     const bf16* vt = sm.u.v[w][cur];
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) {
-      oacc[dt] = mfma32(lds_tr_a<CPR>(vt, 0, dt * 32), p0, oacc[dt]);
-      oacc[dt] = mfma32(lds_tr_a<CPR>(vt, 16, dt * 32), p1, oacc[dt]);
+      const bf16x8 v0 = lds_tr_a<CPR>(vt, 0, dt * 32), v1 = lds_tr_a<CPR>(vt, 16, dt * 32);
+#pragma unroll
+      for (int ct = 0; ct < NCT; ++ct) {
+        oacc[ct][dt] = mfma32(v0, p0[ct], oacc[ct][dt]);
+        oacc[ct][dt] = mfma32(v1, p1[ct], oacc[ct][dt]);
+      }
     }
     if (more) {
 #pragma unroll
       for (int st = 0; st < NKS; ++st) kcur[st] = knx[st];
     }
   }
-  l = wave_sum32(l);
-  __syncthreads();  // every wave is done with its staging buffers (aliased below)
-  if (valid) {
+  // the four waves' columns merged, one column tile at a time: wave -> every fourth column,
+  // lane -> its elements d
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
+  for (int ct = 0; ct < NCT; ++ct) {
+    const float lw = wave_sum32(l[ct]);
+    __syncthreads();  // every wave is done with the staging buffers (the first tile's columns)
+    if (valid[ct]) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) sm.u.fin.so[w][col][dt * 32 + drow(e, g)] = oacc[dt][e];
-    if (isq && g == 0) {
-      sm.u.fin.m[w][col] = m;
-      sm.u.fin.l[w][col] = l;
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sm.u.fin.so[w][l32][dt * 32 + drow(e, g)] = oacc[ct][dt][e];
+      if (isq[ct] && g == 0) {
+        sm.u.fin.m[w][l32] = m[ct];
+        sm.u.fin.l[w][l32] = lw;
+      }
     }
-  }
-  __syncthreads();
-  // combine the 4 waves: thread d of the first D threads owns column d of every token
-  if (tid < D) {
-    const int d = tid;
-    for (int t = 0; t < L; ++t) {
-      const int ck = t * (GG + 1) + GG;
-      part.a[(((int64_t)s * BH + bh) * L + t) * D + d] =
-          sm.u.fin.so[0][ck][d] + sm.u.fin.so[1][ck][d] + sm.u.fin.so[2][ck][d] + sm.u.fin.so[3][ck][d];
-      for (int gg = 0; gg < GG; ++gg) {
-        const int cq = t * (GG + 1) + gg;
-        const float mn =
-            fmaxf(fmaxf(sm.u.fin.m[0][cq], sm.u.fin.m[1][cq]), fmaxf(sm.u.fin.m[2][cq], sm.u.fin.m[3][cq]));
-        float lt = 0.f, ot = 0.f;
+    __syncthreads();
+#pragma unroll 1
+    for (int cl = w; cl < 32; cl += 4) {
+      const int t = (32 * ct + cl) / (GG + 1), gg = 32 * ct + cl - t * (GG + 1);
+      if (t >= L) break;
+      if (gg == GG) {
 #pragma unroll
-        for (int ww = 0; ww < 4; ++ww) {
-          const float al = __builtin_amdgcn_exp2f(sm.u.fin.m[ww][cq] - mn);
-          lt = fmaf(sm.u.fin.l[ww][cq], al, lt);
-          ot = fmaf(sm.u.fin.so[ww][cq][d], al, ot);
-        }
-        const int64_t pi = ((int64_t)s * BH + bh) * (L * GG) + t * GG + gg;
+        for (int d = lane; d < D; d += 64)
+          part.a[(((int64_t)s * BH + bh) * L + t) * D + d] =
+              sm.u.fin.so[0][cl][d] + sm.u.fin.so[1][cl][d] + sm.u.fin.so[2][cl][d] + sm.u.fin.so[3][cl][d];
+        continue;
+      }
+      const float mn = fmaxf(fmaxf(sm.u.fin.m[0][cl], sm.u.fin.m[1][cl]), fmaxf(sm.u.fin.m[2][cl], sm.u.fin.m[3][cl]));
+      float al[4], lt = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) {
+        al[ww] = __builtin_amdgcn_exp2f(sm.u.fin.m[ww][cl] - mn);
+        lt = fmaf(sm.u.fin.l[ww][cl], al[ww], lt);
+      }
+      const int64_t pi = ((int64_t)s * BH + bh) * (L * GG) + t * GG + gg;
+#pragma unroll
+      for (int d = lane; d < D; d += 64) {
+        float ot = 0.f;
+#pragma unroll
+        for (int ww = 0; ww < 4; ++ww) ot = fmaf(sm.u.fin.so[ww][cl][d], al[ww], ot);
         part.o[pi * D + d] = ot;
-        if (d == 0) {
-          part.m[pi] = mn;
-          part.l[pi] = lt;
-        }
+      }
+      if (lane == 0) {
+        part.m[pi] = mn;
+        part.l[pi] = lt;
       }
     }
   }
@@ -241,10 +283,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
 // lanes of a group are merged by lane shuffles.  The new tokens' own rows follow in
 // order: v'_t needs v'_u of the earlier new tokens (u < t), each column only its own
 // column, so the first lane of each group solves its 4 columns of every token without a
-// barrier.  Every workgroup of a kv head computes the v'_t; the g = 0 one writes them and
+// barrier; the outputs then take a token per split lane.  Every workgroup of a kv head computes the v'_t; the g = 0 one writes them and
 // appends (k_t, v'_t) to the caches at rows Tp + t (if write_cache: a group split into
 // chunks of query heads runs this once per chunk, and only the first writes).
-template <int D, int G>
+template <int D, int G, int NCT>
 __global__ __launch_bounds__(256) void lucid_decode_combine_kernel(
     int nsplit, int L, const bf16* __restrict__ q, Strides qs, const bf16* __restrict__ kn, Strides kns,
     const bf16* __restrict__ vn, Strides vns, bf16* __restrict__ kc, Strides kcs, bf16* __restrict__ vc, Strides vcs,
@@ -252,7 +294,7 @@ __global__ __launch_bounds__(256) void lucid_decode_combine_kernel(
     float eps, float dn, DecodePartials part, int Gs, int Gt, int g0, int write_cache) {
   constexpr int CG = D / 4, NSL = 256 / CG;
   static_assert(NSL * CG == 256 && NSL <= 64 && (NSL & (NSL - 1)) == 0, "split lanes of a group within a wave");
-  constexpr int LM = decode_tokens_per_pass<G>();
+  constexpr int LM = decode_tokens_per_pass<G, NCT>();
   __shared__ float kk[LM][LM], qk[LM][LM];  // k_t . k_u (u <= t) and q_tg . k_u (u <= t)
   // merged O, sum_j P_tj v'_j and the new v' rows of every token
   __shared__ __attribute__((aligned(16))) float ovs[LM][D];
@@ -264,26 +306,32 @@ __global__ __launch_bounds__(256) void lucid_decode_combine_kernel(
   const int tid = threadIdx.x, cg = tid / NSL, sl = tid - cg * NSL, d0 = 4 * cg;
   const int GG = G > 0 ? G : Gs;
   const int hq = h * Gt + g0 + g;
-  // dot products among the new tokens: k_t . k_u and q_tg . k_u for u <= t
-  for (int idx = tid; idx < L * L; idx += 256) {
-    const int t = idx / L, u = idx - t * L;
+  // dot products among the new tokens: k_t . k_u and q_tg . k_u for u <= t, D / 8 lanes a pair
+  constexpr int DL = D / 8;
+  for (int idx = tid / DL; idx < L * L; idx += 256 / DL) {
+    const int t = idx / L, u = idx - t * L, i = 8 * (tid % DL);
     if (u > t) continue;
-    const bf16* kt = kn + b * kns.b + h * kns.h + (int64_t)t * kns.t;
-    const bf16* ku = kn + b * kns.b + h * kns.h + (int64_t)u * kns.t;
-    const bf16* qt = q + b * qs.b + hq * qs.h + (int64_t)t * qs.t;
+    const bf16x8 a8 = ld8(kn + b * kns.b + h * kns.h + (int64_t)t * kns.t + i);
+    const bf16x8 b8 = ld8(kn + b * kns.b + h * kns.h + (int64_t)u * kns.t + i);
+    const bf16x8 q8 = ld8(q + b * qs.b + hq * qs.h + (int64_t)t * qs.t + i);
     float dkk = 0.f, dqk = 0.f;
 #pragma unroll
-    for (int i = 0; i < D; i += 8) {
-      const bf16x8 a8 = ld8(kt + i), b8 = ld8(ku + i), q8 = ld8(qt + i);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        dkk = fmaf((float)a8[e], (float)b8[e], dkk);
-        dqk = fmaf((float)q8[e], (float)b8[e], dqk);
-      }
+    for (int e = 0; e < 8; ++e) {
+      dkk = fmaf((float)a8[e], (float)b8[e], dkk);
+      dqk = fmaf((float)q8[e], (float)b8[e], dqk);
     }
-    kk[t][u] = dkk;
-    qk[t][u] = dqk;
+#pragma unroll
+    for (int off = 1; off < DL; off <<= 1) {
+      dkk += __shfl_xor(dkk, off, 64);
+      dqk += __shfl_xor(dqk, off, 64);
+    }
+    if (tid % DL == 0) {
+      kk[t][u] = dkk;
+      qk[t][u] = dqk;
+    }
   }
+  // the first token's value row, wanted after the merge
+  const bf16x4 v40 = *reinterpret_cast<const bf16x4*>(vn + b * vns.b + h * vns.h + d0);
   // the splits' partials of every token: its key column (sum P_tj v'_j) and its query
   // column (t, g), merged with a running max per token
   float M[LM], lv[LM];
@@ -294,7 +342,38 @@ __global__ __launch_bounds__(256) void lucid_decode_combine_kernel(
     lv[t] = 0.f;
     ov[t] = av[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int s = sl; s < nsplit; s += NSL) {
+  int s0 = sl;
+  if (L == 1) {  // one token: four splits' loads in flight at a time (the loop below waits for each in turn)
+    for (; s0 + 3 * NSL < nsplit; s0 += 4 * NSL) {
+      float mi[4], li[4];
+      f32x4 oi[4], ai[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int64_t i = ((int64_t)(s0 + k * NSL) * BH + bh) * GG + g;
+        mi[k] = part.m[i];
+        li[k] = part.l[i];
+        oi[k] = *reinterpret_cast<const f32x4*>(part.o + i * D + d0);
+        ai[k] = *reinterpret_cast<const f32x4*>(part.a + ((int64_t)(s0 + k * NSL) * BH + bh) * D + d0);
+      }
+      const float mn = fmaxf(fmaxf(fmaxf(mi[0], mi[1]), fmaxf(mi[2], mi[3])), M[0]);
+      const float c = __builtin_amdgcn_exp2f(M[0] - mn);
+      lv[0] *= c;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) ov[0][x] *= c;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float e = __builtin_amdgcn_exp2f(mi[k] - mn);
+        lv[0] = fmaf(li[k], e, lv[0]);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          ov[0][x] = fmaf(oi[k][x], e, ov[0][x]);
+          av[0][x] += ai[k][x];
+        }
+      }
+      M[0] = mn;
+    }
+  }
+  for (int s = s0; s < nsplit; s += NSL) {
     const int64_t base = ((int64_t)s * BH + bh) * (L * GG) + g;
 #pragma unroll
     for (int t = 0; t < LM; ++t) {
@@ -349,12 +428,11 @@ __global__ __launch_bounds__(256) void lucid_decode_combine_kernel(
     }
   }
   __syncthreads();  // kk, qk and the merged states
-  if (sl != 0) return;
   // the new rows in order: v'_t = (v_t - a_t - sum_{u<t} P_tu v'_u) / P_tt (columns d0 .. d0+3)
   const float sl2 = scale * LOG2E_F, c0 = LOG2E_F / scale;
-  for (int t = 0; t < L; ++t) {
+  for (int t = 0; sl == 0 && t < L; ++t) {
     const float rt = rsqrtf(kk[t][t] / dn + eps);
-    const bf16x4 v4 = *reinterpret_cast<const bf16x4*>(vn + b * vns.b + h * vns.h + (int64_t)t * vns.t + d0);
+    const bf16x4 v4 = t == 0 ? v40 : *reinterpret_cast<const bf16x4*>(vn + b * vns.b + h * vns.h + (int64_t)t * vns.t + d0);
     const f32x4 a4 = *reinterpret_cast<const f32x4*>(&avs[t][d0]);
     f32x4 x;
 #pragma unroll
@@ -371,10 +449,12 @@ __global__ __launch_bounds__(256) void lucid_decode_combine_kernel(
     const float inv = 1.f / __builtin_amdgcn_exp2f(LOG2E_F * (scale * dn * ms / (ms + eps) - 1.f / scale));
 #pragma unroll
     for (int j = 0; j < 4; ++j) x[j] *= inv;
-    *reinterpret_cast<f32x4*>(&vps[t][d0]) = x;  // read back only by this thread
+    *reinterpret_cast<f32x4*>(&vps[t][d0]) = x;
   }
-  // outputs: the cached part merged with the new keys u <= t (values bf16(v'_u), as cached)
-  for (int t = 0; t < L; ++t) {
+  __syncthreads();
+  // outputs, a token per split lane: the cached part merged with the new keys u <= t (values
+  // bf16(v'_u), as cached)
+  for (int t = sl; t < L; t += NSL) {
     float M2 = ms_[t];
     for (int u = 0; u <= t; ++u) M2 = fmaxf(M2, qk[t][u] * sl2);
     const float c = __builtin_amdgcn_exp2f(ms_[t] - M2);
