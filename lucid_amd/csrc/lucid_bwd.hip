@@ -1379,7 +1379,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void l
       }
       const int cl = chh * 32 + l32;  // row of dV inside the sub-block
       const int r = r0 + cl;
-      bf16* ob = dvb + ((int64_t)bh * T + r) * D;
       bf16* ou = dv_out + b * dvs.b + h * dvs.h + (int64_t)r * dvs.t;
 #pragma unroll
       for (int qq = 0; qq < 4; ++qq) {
@@ -1387,13 +1386,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void l
         bf16x4 bb;
 #pragma unroll
         for (int u = 0; u < 4; ++u) bb[u] = (bf16)o[4 * qq + u];
-        *reinterpret_cast<bf16x4*>(ob + d0) = bb;
         *reinterpret_cast<bf16x4*>(ou + d0) = bb;
         *reinterpret_cast<bf16x4*>(sm.sdv + swz_off<D / 8, SW>(cl, d0 >> 3) + (d0 & 7)) = bb;
       }
     }
+    __syncthreads();
+    // the dV rows, published in whole 16-byte chunks
+    static_assert(64 * (D / 8) == NTHR, "one 16-byte chunk of the solved rows per thread");
+    {
+      const int r = tid >> 3, c8 = tid & 7;
+      st_pub16(pub_base(dvb + (int64_t)bh * T * D), 2u * (unsigned)((r0 + r) * D + 8 * c8),
+               ld8(swz<D / 8, SW>(sm.sdv, r, c8)));
+    }
     dma_wait();
-    publish_counter(cnt, NT - (4 * p + s));  // waits for every wave's stores, then a barrier
+    publish_stored(cnt, NT - (4 * p + s));  // waits for every wave's stores, then a barrier
     // the solved rows against the earlier sub-blocks' columns; the strictly lower in-block
     // column-sum terms for sub-block s's own columns
     if (sbw < s) sweep_rows(sm.sk, sm.sdv, false);

@@ -1764,11 +1764,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void l
     diag_solve(1);
     __syncthreads();
     // V'^T of the block to the T-perm operand copy: 16-byte stores
+    const __amdgpu_buffer_rsrc_t pt = pub_base(vpt + (int64_t)bh * D * T);
     for (int c = tid; c < D * 16; c += NTHR) {
       const int dd = c >> 4, s8 = (c & 15) * 8;
-      *reinterpret_cast<bf16x8*>(vpt + ((int64_t)bh * D + dd) * T + r0 + s8) = ld8(&sm.u.fin.vT[dd][s8]);
+      st_pub16(pt, 2u * ((unsigned)dd * (unsigned)T + (unsigned)(r0 + s8)), ld8(&sm.u.fin.vT[dd][s8]));
     }
-    publish_counter(cnt, 2 * q + 2);
+    publish_stored(cnt, 2 * q + 2);
   };
   // R^T = -C acc for the waves of block half `half` (waves 4 half .. 4 half + 3)
   auto store_r = [&](int half) {
@@ -2075,11 +2076,12 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_fused_fwd_
   __syncthreads();
   diag_solve(1);
   __syncthreads();
+  const __amdgpu_buffer_rsrc_t pt = pub_base(vpt + (int64_t)bh * D * T);
   for (int cc = tid; cc < D * 16; cc += 256) {
     const int dd = cc >> 4, s8 = (cc & 15) * 8;
-    *reinterpret_cast<bf16x8*>(vpt + ((int64_t)bh * D + dd) * T + i0 + s8) = ld8(&sm.u.fin.vT[dd][s8]);
+    st_pub16(pt, 2u * ((unsigned)dd * (unsigned)T + (unsigned)(i0 + s8)), ld8(&sm.u.fin.vT[dd][s8]));
   }
-  publish_counter(cnt, 2 * i2 + 2);
+  publish_stored(cnt, 2 * i2 + 2);
 
   // ---- the attention's diagonal pair: keys i0 .. i0 + 127 ----
   // the block's K rows go to the first staging buffer (its bytes lie inside R^T and X,

@@ -390,15 +390,17 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(KD == 64 && !F32) void path
    }
   };
   // dV^T of chunk cc to the chain operand with 16-byte stores, then publish it
+  const __amdgpu_buffer_rsrc_t ph = pub_base(bw.dvT + (int64_t)bhq * KD * T);
+  const __amdgpu_buffer_rsrc_t pl = pub_base(bw.dvT + (F32 ? bw.lo_dvT + (int64_t)bhq * KD * T : 0));
   auto publish_chunk = [&](int cc) {
     __syncthreads();
     for (int c = tid; c < KD * 8; c += 256) {
       const int dd = c >> 3, s8 = (c & 7) * 8;
-      bf16* dst = bw.dvT + ((int64_t)bhq * KD + dd) * T + j0 + cc * 64 + s8;
-      *reinterpret_cast<bf16x8*>(dst) = ld8(&sm.u.fin.dt[0][dd][cc * 64 + s8]);
-      if constexpr (F32) *reinterpret_cast<bf16x8*>(dst + bw.lo_dvT) = ld8(&sm.u.fin.dt[NP - 1][dd][cc * 64 + s8]);
+      const unsigned off = 2u * ((unsigned)dd * (unsigned)T + (unsigned)(j0 + cc * 64 + s8));
+      st_pub16(ph, off, ld8(&sm.u.fin.dt[0][dd][cc * 64 + s8]));
+      if constexpr (F32) st_pub16(pl, off, ld8(&sm.u.fin.dt[NP - 1][dd][cc * 64 + s8]));
     }
-    publish_counter(cnt, NT - (A + cc));
+    publish_stored(cnt, NT - (A + cc));
   };
   f32x16 dvoB[NVT / 2], dvoA[NVT / 2];
   if (hasB) {

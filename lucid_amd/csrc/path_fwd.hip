@@ -727,13 +727,15 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(KD == 64 && !F32) void path
   }
   // O^T of the workgroup's chunks to the chain operand with 16-byte stores
   const int nch = hasB ? 2 : 1;
+  const __amdgpu_buffer_rsrc_t ph = pub_base(ws.oT + (int64_t)bhq * KD * T);
+  const __amdgpu_buffer_rsrc_t pl = pub_base(ws.oT + (F32 ? ws.lo_oT + (int64_t)bhq * KD * T : 0));
   for (int c = tid; c < KD * 8 * nch; c += 256) {
     const int dd = c / (8 * nch), s8 = (c - dd * 8 * nch) * 8;
-    bf16* dst = ws.oT + ((int64_t)bhq * KD + dd) * T + i0 + s8;
-    *reinterpret_cast<bf16x8*>(dst) = ld8(&sm.u.fin.ot[0][dd][s8]);
-    if constexpr (F32) *reinterpret_cast<bf16x8*>(dst + ws.lo_oT) = ld8(&sm.u.fin.ot[NP - 1][dd][s8]);
+    const unsigned off = 2u * ((unsigned)dd * (unsigned)T + (unsigned)(i0 + s8));
+    st_pub16(ph, off, ld8(&sm.u.fin.ot[0][dd][s8]));
+    if constexpr (F32) st_pub16(pl, off, ld8(&sm.u.fin.ot[NP - 1][dd][s8]));
   }
-  publish_counter(cnt, A + nch);
+  publish_stored(cnt, A + nch);
 }
 
 // ---------------------------------------------------------------------------
