@@ -1228,46 +1228,77 @@ __global__ __launch_bounds__(256) void path_softmax_diag_bwd_kernel(const pin_t<
 // ---------------------------------------------------------------------------
 // Products backward inside one large chunk (cumprod_householder_bwd.py:13-95):
 //   F = dHL_s; for c from the bottom up: dHc_c += SUF_c^T F; F <- F Hc_c^T + dSUF_c
+// A serial chain of at most PR steps in few workgroups: a step is as long as its latencies.
+// Waves 4..7 form dHc_c while waves 0..3 form the next F in the other buffer (one barrier a
+// step), on operands split into bf16 planes when they are stored (Hc_c has its planes from
+// the forward); everything a step adds to or stages for the next is fetched one step ahead.
+// B1 H16 T8192: 51 us a launch (four waves on fp32 operands, loads waited for in each step: 145).
 // grid (NS, B*HQ)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void path_products_bwd_kernel(int HQ, int H, int T, PathFwdWs ws, PathBwdWs bw) {
-  __shared__ __attribute__((aligned(16))) float F[64][68];
-  __shared__ __attribute__((aligned(16))) float S[64][68];
-  __shared__ __attribute__((aligned(16))) float Hs[64][68];
+__global__ __launch_bounds__(512) void path_products_bwd_kernel(int HQ, int H, int T, PathFwdWs ws, PathBwdWs bw) {
+  __shared__ __attribute__((aligned(16))) PlaneMat<2> F[2], S[2], Hm[2];
   const int NT = T / PC, NS = (NT + PR - 1) / PR;
   const int s = blockIdx.x, bhq = blockIdx.y;
   const int G_ = HQ / H;
   const int b = bhq / HQ, hq = bhq - b * HQ, bh = b * H + hq / G_;
   const int cb = s * PR, ce = min(cb + PR, NT) - 1;
-  const int cl = dl_col();
-  // products on the matrix cores (mgemm64, D layout); SUF_c and Hc_c of the next chunk
-  // are fetched into registers while the current one is processed
-  f32x4 ps[4], ph[4];
-  mat_fetch(ps, ws.suf + ((int64_t)bh * NT + cb) * 4096);
-  mat_fetch(ph, ws.hc + ((int64_t)bh * NT + cb) * 4096);
-  load_mat64<false>(F, bw.dhl + ((int64_t)bhq * NS + s) * 4096);
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), w4 = w & 3;
+  const int ht = tid & 255, hr = ht >> 2, hc = 2 * (ht & 3);  // 16 columns of one row per thread of a half
+  f32x4 ps[4];       // waves 4..7: SUF of the next step
+  bf16x8 ph[2][2];   // waves 0..3: planes of Hc of the next step
+  auto fetch = [&](int c) {
+    if (w >= 4) {
+      const float* src = ws.suf + ((int64_t)bh * NT + c) * 4096 + 16 * ht;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) ps[u] = *reinterpret_cast<const f32x4*>(src + 4 * u);
+    } else {
+      const bf16* src = ws.hcs + ((int64_t)bh * NT + c) * 8192 + 16 * ht;
+#pragma unroll
+      for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) ph[pl][u] = ld8(src + 4096 * pl + 8 * u);
+    }
+  };
+  auto put = [&](int buf) {
+    if (w >= 4) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) pl_put8(S[buf], hr, hc + u, ps[2 * u], ps[2 * u + 1]);
+    } else {
+#pragma unroll
+      for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          *reinterpret_cast<bf16x8*>(Hm[buf].p[pl] + swz_off<8>(hr, hc + u)) = ph[pl][u];
+    }
+  };
+  // the matrix a step adds its product to: dHc_c (waves 4..7), dSUF_c (waves 0..3)
+  auto addend = [&](int c) {
+    return pl_load((w >= 4 ? bw.dhc : bw.dsuf) + ((int64_t)bhq * NT + c) * 4096, w4);
+  };
+  fetch(cb);
+  {
+    const float* src = bw.dhl + ((int64_t)bhq * NS + s) * 4096 + 8 * tid;
+    pl_put8(F[0], tid >> 3, tid & 7, *reinterpret_cast<const f32x4*>(src), *reinterpret_cast<const f32x4*>(src + 4));
+  }
+  f32x16 add = addend(cb);
+  put(0);
+  __syncthreads();
   for (int c = cb; c <= ce; ++c) {
-    mat_put(S, ps);
-    mat_put(Hs, ph);
+    const int buf = (c - cb) & 1;
+    const bool more = c < ce;
+    f32x16 next = zero16();
+    if (more) {
+      fetch(c + 1);
+      next = addend(c + 1);
+    }
+    if (w >= 4) {
+      pl_save(bw.dhc + ((int64_t)bhq * NT + c) * 4096, pgemm64<true, false>(S[buf], F[buf], w4, add), w4);
+    } else if (more) {
+      pl_store(F[buf ^ 1], pgemm64<false, true>(F[buf], Hm[buf], w4, add), w4, 0);
+    }
+    if (more) put(buf ^ 1);
+    add = next;
     __syncthreads();
-    if (c < ce) {
-      mat_fetch(ps, ws.suf + ((int64_t)bh * NT + c + 1) * 4096);
-      mat_fetch(ph, ws.hc + ((int64_t)bh * NT + c + 1) * 4096);
-    }
-    {
-      const f32x16 a = mgemm64<true, false>(S, F, zero16());  // dHc_c += SUF_c^T F
-      float* dst = bw.dhc + ((int64_t)bhq * NT + c) * 4096;
-      DL_FOR_E dst[dl_row(e) * 64 + cl] += a[e];
-    }
-    const f32x16 f = mgemm64<false, true>(F, Hs, zero16());  // F <- F Hc_c^T + dSUF_c
-    __syncthreads();
-    {
-      const float* ds = bw.dsuf + ((int64_t)bhq * NT + c) * 4096;
-      DL_FOR_E {
-        const int r = dl_row(e);
-        F[r][cl] = f[e] + ds[r * 64 + cl];
-      }
-    }
   }
 }
 
@@ -1277,146 +1308,224 @@ __global__ __launch_bounds__(256) void path_products_bwd_kernel(int HQ, int H, i
 //   q~ = q - QW W2 (QW = tril(q W^T)), k~ = k - TW^T W (TW = Tm stril(Wb k^T)),
 //   A_diag = tril(q k^T - QW TW).
 // Inputs d q~, d k~, dA_diag, dHc; outputs dq, dk, dw, dbeta (per query head, fp32).
-// The 64x64 products run on the matrix cores (mgemm64, 3-term bf16 split, ~fp32
-// accuracy); every wave keeps its 32x32 tile of each running result in MFMA D layout
-// (rows dl_row(e), column dl_col()).  Operands live in 9 fp32 LDS buffers.
+// The 26 64x64 products run on the matrix cores (pgemm64, 3-term bf16 split, ~fp32 accuracy;
+// the bf16 operands q, k, W of the bf16 instance have no second term) on operands that are
+// split into bf16 planes once, when they are stored.  Eight waves: the products fall into two
+// sets that need each other only at a few barriers, waves 0..3 take the inverse, dq, dk and
+// dTm, waves 4..7 the gradients of W2, QW, TW, W and Wb.  One workgroup fills the LDS, so the
+// second set is also what hides the first one's latencies.
+// B1 H16 T8192 bf16: 258 us with four waves on fp32 operands split at every use, 166 this way
+// (311 MB in and out: 65 us).
 // grid (NT, B*HQ)
 // ---------------------------------------------------------------------------
 template <bool F32>
-__global__ __launch_bounds__(256) void path_wy_bwd_kernel(const pin_t<F32>* __restrict__ q, Strides qs,
+__global__ __launch_bounds__(512) void path_wy_bwd_kernel(const pin_t<F32>* __restrict__ q, Strides qs,
                                                           const pin_t<F32>* __restrict__ k, Strides ks,
-                                                          const pin_t<F32>* __restrict__ w, Strides wst,
+                                                          const pin_t<F32>* __restrict__ w_, Strides wst,
                                                           const pin_t<F32>* __restrict__ beta, Strides bst, int HQ,
                                                           int H, int T, PathFwdWs ws, PathBwdWs bw) {
-  __shared__ __attribute__((aligned(16))) float W[64][68];
-  __shared__ __attribute__((aligned(16))) float Wb[64][68];
-  __shared__ __attribute__((aligned(16))) float Q[64][68];
-  __shared__ __attribute__((aligned(16))) float K[64][68];
-  __shared__ __attribute__((aligned(16))) float Tm[64][68];
-  __shared__ __attribute__((aligned(16))) float S1[64][68];
-  __shared__ __attribute__((aligned(16))) float S2[64][68];
-  __shared__ __attribute__((aligned(16))) float S3[64][68];
-  __shared__ __attribute__((aligned(16))) float S4[64][68];
-  __shared__ float bsh[64];
+  constexpr int NPI = F32 ? 2 : 1;  // planes of the caller's tensors
+  __shared__ __attribute__((aligned(16))) PlaneMat<NPI> W, Q, K;
+  __shared__ __attribute__((aligned(16))) PlaneMat<2> Wb, S1, S2, S3, S4;
+  __shared__ __attribute__((aligned(16))) union {
+    float f[64][68];  // the inverse is formed in fp32
+    PlaneMat<2> p;
+  } Tm;
+  __shared__ float bsh[64], dbs[2][64];
   const int NT = T / PC;
   const int c = blockIdx.x, bhq = blockIdx.y;
   const int G_ = HQ / H;
   const int b = bhq / HQ, hq = bhq - b * HQ, h = hq / G_, bh = b * H + h;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), w4 = w & 3;
+  const bool h0 = w < 4;
+  const int ht = tid & 255, hr = ht >> 2, hc = 2 * (ht & 3);  // 16 columns of one row per thread of a half
+  const int r8 = tid >> 3, c8 = tid & 7;                      // 8 columns of one row per thread
   const int t0 = c * PC;
   const f32x16 z = zero16();
 
-  // The fp32 inputs go to registers first (16 values per thread each) so their
-  // latency overlaps the WY recomputation; each is stored to LDS when its buffer frees.
-  f32x4 pw2[4], pdh[4], pdq[4], pdk[4], pda[4];
-  mat_fetch(pw2, ws.w2 + ((int64_t)bh * T + t0) * 64);
-  mat_fetch(pdh, bw.dhc + ((int64_t)bhq * NT + c) * 4096);
-  mat_fetch(pdq, bw.dqt + ((int64_t)bhq * T + t0) * 64);
-  mat_fetch(pdk, bw.dkt + ((int64_t)bhq * T + t0) * 64);
-  mat_fetch(pda, bw.dad + ((int64_t)bhq * NT + c) * 4096);
-  load_rows64_f32(W, w + b * wst.b + h * wst.h + (int64_t)t0 * wst.t, wst.t);
-  load_rows64_f32(Q, q + b * qs.b + hq * qs.h + (int64_t)t0 * qs.t, qs.t);
-  load_rows64_f32(K, k + b * ks.b + h * ks.h + (int64_t)t0 * ks.t, ks.t);
-  __syncthreads();
-  {
-    const int r = tid >> 2, cc = (tid & 3) * 16;
-    const float bt = (float)beta[b * bst.b + h * bst.h + (int64_t)(t0 + r) * bst.t];
-    if ((tid & 3) == 0) bsh[r] = bt;
+  // fp32 inputs to registers first: their latency passes during the WY recomputation
+  const float* dqt = bw.dqt + ((int64_t)bhq * T + t0) * 64;
+  const float* dkt = bw.dkt + ((int64_t)bhq * T + t0) * 64;
+  auto pair8 = [&](const float* src, f32x4 x[2]) {
+    x[0] = *reinterpret_cast<const f32x4*>(src + 8 * tid);
+    x[1] = *reinterpret_cast<const f32x4*>(src + 8 * tid + 4);
+  };
+  f32x4 pw2[2], pdh[2], pda[2], pdq[4], pdk[4];
+  pair8(ws.w2 + ((int64_t)bh * T + t0) * 64, pw2);
+  pair8(bw.dhc + ((int64_t)bhq * NT + c) * 4096, pdh);
+  pair8(bw.dad + ((int64_t)bhq * NT + c) * 4096, pda);
+  if (!h0) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) Wb[r][cc + e] = bt * W[r][cc + e];
-  }
-  mat_put(S1, pw2);  // W2
-  mat_put(S2, pdh);  // dHc
-  __syncthreads();
-  dl_store(Tm, mgemm64<false, true>(Wb, W, z), 2);
-  __syncthreads();
-  invert_unit_lower64(Tm);
-  f32x16 aW = dl_neg(mgemm64<false, true>(S1, S2, z));   // -W2 dHc^T
-  f32x16 aW2 = dl_neg(mgemm64<false, false>(W, S2, z));  // -W dHc
-  dl_store(S3, mgemm64<false, true>(Q, W, z), 1);        // QW
-  __syncthreads();
-  mat_put(S2, pdq);  // d q~
-  __syncthreads();
-  f32x16 aq = dl_load(S2);
-  f32x16 dQW = dl_neg(mgemm64<false, true>(S2, S1, z));  // -dq~ W2^T
-  {
-    const f32x16 t = mgemm64<true, false>(S3, S2, z);    // QW^T dq~
-    DL_FOR_E aW2[e] -= t[e];
-  }
-  dl_store(S4, mgemm64<false, true>(Wb, K, z), 2);       // WBK
-  __syncthreads();
-  dl_store(S1, mgemm64<false, false>(Tm, S4, z), 0);     // TW
-  mat_put(S2, pdk);                                       // d k~
-  __syncthreads();
-  f32x16 ak = dl_load(S2);
-  f32x16 dTW = dl_neg(mgemm64<false, true>(W, S2, z));   // -W dk~^T
-  {
-    const f32x16 t = mgemm64<false, false>(S1, S2, z);   // TW dk~
-    DL_FOR_E aW[e] -= t[e];
-  }
-  __syncthreads();
-  mat_put(S2, pda);  // dA_diag
-  __syncthreads();
-  aq = mgemm64<false, false>(S2, K, aq);  // dq += dA K
-  ak = mgemm64<true, false>(S2, Q, ak);   // dk += dA^T Q
-  {
-    const f32x16 t = mgemm64<false, true>(S2, S1, z);   // dA TW^T
-    const f32x16 t5 = mgemm64<true, false>(S3, S2, z);  // QW^T dA
-    DL_FOR_E {
-      dQW[e] -= t[e];
-      dTW[e] -= t5[e];
+    for (int u = 0; u < 4; ++u) {
+      pdq[u] = *reinterpret_cast<const f32x4*>(dqt + 16 * ht + 4 * u);
+      pdk[u] = *reinterpret_cast<const f32x4*>(dkt + 16 * ht + 4 * u);
     }
   }
-  __syncthreads();
-  dl_store(S2, dQW, 1);
-  dl_store(S1, dTW, 0);
-  __syncthreads();
-  aq = mgemm64<false, false>(S2, W, aq);         // dq += tril(dQW) W
-  aW = mgemm64<true, false>(S2, Q, aW);          // dW += tril(dQW)^T q
-  f32x16 dTm = mgemm64<false, true>(S1, S4, z);  // dTm = dTW WBK^T
-  dl_store(S3, mgemm64<true, false>(Tm, S1, z), 2);  // dWBK = stril(Tm^T dTW)
-  __syncthreads();
-  f32x16 aWb = mgemm64<false, false>(S3, K, z);  // dWb = dWBK k
-  ak = mgemm64<true, false>(S3, Wb, ak);         // dk += dWBK^T Wb
-  dl_store(S2, aW2, 0);                          // dW2
-  __syncthreads();
-  dTm = mgemm64<false, true>(S2, Wb, dTm);  // dTm += dW2 Wb^T
-  aWb = mgemm64<true, false>(Tm, S2, aWb);  // dWb += Tm^T dW2
-  dl_store(S1, dTm, 0);
-  __syncthreads();
-  dl_store(S3, mgemm64<true, false>(Tm, S1, z), 0);  // Tm^T dTm
-  __syncthreads();
-  dl_store(S4, dl_neg(mgemm64<false, true>(S3, Tm, z)), 2);  // da = -stril((Tm^T dTm) Tm^T)
-  __syncthreads();
-  aWb = mgemm64<false, false>(S4, W, aWb);  // dWb += da W
-  aW = mgemm64<true, false>(S4, Wb, aW);    // dW += da^T Wb
-  // dW += beta dWb; dbeta_r = sum_c dWb[r][c] W[r][c] (row sums through S2)
-  const int cl = dl_col();
-  DL_FOR_E {
-    const int r = dl_row(e);
-    aW[e] += bsh[r] * aWb[e];
-    S2[r][cl] = aWb[e] * W[r][cl];
-  }
-  const int64_t rowbase = ((int64_t)bhq * T + t0) * 64;
-  DL_FOR_E {
-    const int64_t off = rowbase + dl_row(e) * 64 + cl;
-    bw.dq[off] = aq[e];
-    bw.dk[off] = ak[e];
-    bw.dw[off] = aW[e];
-  }
-  __syncthreads();
+  // eight values of the caller's row r8 into the planes; returns them in fp32
+  auto rows_in = [&](PlaneMat<NPI>& M, const pin_t<F32>* src, f32x4 x[2]) {
+    if constexpr (F32) {
+      x[0] = *reinterpret_cast<const f32x4*>(src);
+      x[1] = *reinterpret_cast<const f32x4*>(src + 4);
+      pl_put8(M, r8, c8, x[0], x[1]);
+    } else {
+      const bf16x8 v = ld8(src);
+      *reinterpret_cast<bf16x8*>(M.p[0] + swz_off<8>(r8, c8)) = v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e >> 2][e & 3] = (float)v[e];
+    }
+  };
   {
-    const int r = tid >> 2, cc = (tid & 3) * 16;
+    f32x4 x[2];
+    rows_in(Q, q + b * qs.b + hq * qs.h + (int64_t)(t0 + r8) * qs.t + 8 * c8, x);
+    rows_in(K, k + b * ks.b + h * ks.h + (int64_t)(t0 + r8) * ks.t + 8 * c8, x);
+    rows_in(W, w_ + b * wst.b + h * wst.h + (int64_t)(t0 + r8) * wst.t + 8 * c8, x);
+    const float bt = (float)beta[b * bst.b + h * bst.h + (int64_t)(t0 + r8) * bst.t];
+    if (c8 == 0) bsh[r8] = bt;
+    pl_put8(Wb, r8, c8, bt * x[0], bt * x[1]);
+  }
+  pl_put8(S1, r8, c8, pw2[0], pw2[1]);  // W2
+  pl_put8(S2, r8, c8, pdh[0], pdh[1]);  // dHc
+  __syncthreads();
+  if (h0) {
+    const f32x16 a = pgemm64<false, true>(Wb, W, w4, z);
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd)
+      *reinterpret_cast<f32x4*>(&Tm.f[pl_row(w4)][pl_col(w4, qd)]) = pl_quad(a, w4, qd, 2);
+  } else {
+    pl_store(S3, pgemm64<false, true>(Q, W, w4, z), w4, 1);  // QW
+  }
+  __syncthreads();
+  // the inverse (waves 0..3, invert_unit_lower64's steps) beside what does not need it
+  f32x16 aq = z, ak = z, dTm = z;                            // waves 0..3
+  f32x16 aW = z, aW2 = z, dQW = z, dTW = z, aWb = z;         // waves 4..7
+  auto sub = [](f32x16 x, const f32x16& y) {
+    DL_FOR_E x[e] -= y[e];
+    return x;
+  };
+  auto put16 = [&](PlaneMat<2>& M, const f32x4 x[4]) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) pl_put8(M, hr, hc + u, x[2 * u], x[2 * u + 1]);
+  };
+  const MergeQuad<16> m16(ht);
+  const MergeQuad<32> m32(ht);
+  f32x4 mq;
+  if (h0) {
+    invert_lower16(Tm.f, w, tid & 63);
+  } else {
+    aW = dl_neg(pgemm64<false, true>(S1, S2, w4, z));   // -W2 dHc^T
+    aW2 = dl_neg(pgemm64<false, false>(W, S2, w4, z));  // -W dHc
+  }
+  __syncthreads();
+  if (h0) mq = m16.product<false>(Tm.f);
+  else put16(S2, pdq);  // d q~
+  __syncthreads();
+  if (h0) {
+    m16.put(Tm.f, mq);
+  } else {
+    pl_store(S4, pgemm64<false, true>(Wb, K, w4, z), w4, 2);  // WBK
+    dQW = dl_neg(pgemm64<false, true>(S2, S1, w4, z));        // -dq~ W2^T
+  }
+  __syncthreads();
+  if (h0) mq = m16.product<true>(Tm.f);
+  else aW2 = sub(aW2, pgemm64<true, false>(S3, S2, w4, z));  // QW^T dq~
+  __syncthreads();
+  if (h0) m16.put(Tm.f, -mq);
+  else put16(S2, pdk);  // d k~
+  __syncthreads();
+  if (h0) mq = m32.product<false>(Tm.f);
+  else dTW = dl_neg(pgemm64<false, true>(W, S2, w4, z));  // -W dk~^T
+  __syncthreads();
+  if (h0) m32.put(Tm.f, mq);
+  __syncthreads();
+  if (h0) mq = m32.product<true>(Tm.f);
+  __syncthreads();
+  if (h0) m32.put(Tm.f, -mq);
+  __syncthreads();
+  {  // to planes, in place
+    f32x4 x[2];
+    x[0] = *reinterpret_cast<const f32x4*>(&Tm.f[r8][8 * c8]);
+    x[1] = *reinterpret_cast<const f32x4*>(&Tm.f[r8][8 * c8 + 4]);
+    __syncthreads();
+    pl_put8(Tm.p, r8, c8, x[0], x[1]);
+  }
+  __syncthreads();
+  if (h0) pl_store(S1, pgemm64<false, false>(Tm.p, S4, w4, z), w4, 0);  // TW
+  __syncthreads();
+  if (h0) {
+    aq = pl_load(dqt, w4);
+    ak = pl_load(dkt, w4);
+  } else {
+    aW = sub(aW, pgemm64<false, false>(S1, S2, w4, z));  // TW dk~
+  }
+  __syncthreads();
+  pl_put8(S2, r8, c8, pda[0], pda[1]);  // dA_diag
+  __syncthreads();
+  if (h0) {
+    aq = pgemm64<false, false>(S2, K, w4, aq);  // dq += dA K
+    ak = pgemm64<true, false>(S2, Q, w4, ak);   // dk += dA^T Q
+  } else {
+    dQW = sub(dQW, pgemm64<false, true>(S2, S1, w4, z));  // dA TW^T
+    dTW = sub(dTW, pgemm64<true, false>(S3, S2, w4, z));  // QW^T dA
+  }
+  __syncthreads();
+  if (!h0) {
+    pl_store(S2, dQW, w4, 1);
+    pl_store(S1, dTW, w4, 0);
+  }
+  __syncthreads();
+  if (h0) {
+    aq = pgemm64<false, false>(S2, W, w4, aq);   // dq += tril(dQW) W
+    dTm = pgemm64<false, true>(S1, S4, w4, z);   // dTm = dTW WBK^T
+  } else {
+    aW = pgemm64<true, false>(S2, Q, w4, aW);                    // dW += tril(dQW)^T q
+    pl_store(S3, pgemm64<true, false>(Tm.p, S1, w4, z), w4, 2);  // dWBK = stril(Tm^T dTW)
+  }
+  __syncthreads();
+  if (h0) {
+    ak = pgemm64<true, false>(S3, Wb, w4, ak);  // dk += dWBK^T Wb
+  } else {
+    pl_store(S2, aW2, w4, 0);                     // dW2
+    aWb = pgemm64<false, false>(S3, K, w4, z);  // dWb = dWBK k
+  }
+  __syncthreads();
+  if (h0) {
+    pl_store(S1, pgemm64<false, true>(S2, Wb, w4, dTm), w4, 0);  // dTm += dW2 Wb^T
+  } else {
+    aWb = pgemm64<true, false>(Tm.p, S2, w4, aWb);  // dWb += Tm^T dW2
+  }
+  __syncthreads();
+  if (h0) pl_store(S3, pgemm64<true, false>(Tm.p, S1, w4, z), w4, 0);  // Tm^T dTm
+  __syncthreads();
+  if (h0) pl_store(S4, dl_neg(pgemm64<false, true>(S3, Tm.p, w4, z)), w4, 2);  // da = -stril((Tm^T dTm) Tm^T)
+  __syncthreads();
+  const int64_t rowbase = ((int64_t)bhq * T + t0) * 64;
+  if (h0) {
+    pl_save(bw.dq + rowbase, aq, w4);
+    pl_save(bw.dk + rowbase, ak, w4);
+  } else {
+    aWb = pgemm64<false, false>(S4, W, w4, aWb);  // dWb += da W
+    aW = pgemm64<true, false>(S4, Wb, w4, aW);    // dW += da^T Wb
+    // dW += beta dWb; dbeta_r = sum_c dWb[r][c] W[r][c]
+    const int r = pl_row(w4);
+    const float bt = bsh[r];
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; i += 4) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(&S2[r][cc + i]);
-      s += (v[0] + v[1]) + (v[2] + v[3]);
+    for (int qd = 0; qd < 4; ++qd) {
+      const int c0 = pl_col(w4, qd), off = swz_off<8>(r, c0 >> 3) + (c0 & 7);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float x = (float)W.p[0][off + u];
+        if constexpr (F32) x += (float)W.p[NPI - 1][off + u];
+        s = fmaf(aWb[4 * qd + u], x, s);
+        aW[4 * qd + u] += bt * aWb[4 * qd + u];
+      }
     }
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
-    if ((tid & 3) == 0) bw.db[(int64_t)bhq * T + t0 + r] = s;
+    s = wave_sum32(s);
+    if ((tid & 63) < 32) dbs[w4 & 1][r] = s;
+    pl_save(bw.dw + rowbase, aW, w4);
   }
+  __syncthreads();
+  if (tid < 64) bw.db[(int64_t)bhq * T + t0 + tid] = dbs[0][tid] + dbs[1][tid];
 }
 
 // ---------------------------------------------------------------------------

@@ -226,10 +226,10 @@ int launch_back(const void* q, const int64_t* q_strides, const void* k, const in
                        PS(q_strides), (const bf16*)k, PS(k_strides), (const bf16*)w, PS(w_strides), (const bf16*)beta,
                        PS(beta_strides), HQ, H, T, ws, bw);
   } else {
-    LUCID_TIMED_LAUNCH(phip, "path_products_bwd_kernel", lucid::path_products_bwd_kernel, dim3(NS, BHq), st, HQ, H, T,
-                       ws, bw);
-    LUCID_TIMED_LAUNCH(phip, "path_wy_bwd_kernel", lucid::path_wy_bwd_kernel<F32>, dim3(NT, BHq), st, (const TI*)q,
-                       PS(q_strides), (const TI*)k, PS(k_strides), (const TI*)w, PS(w_strides), (const TI*)beta,
+    LUCID_TIMED_LAUNCH_B(phip, "path_products_bwd_kernel", lucid::path_products_bwd_kernel, dim3(NS, BHq), dim3(512),
+                         st, HQ, H, T, ws, bw);
+    LUCID_TIMED_LAUNCH_B(phip, "path_wy_bwd_kernel", lucid::path_wy_bwd_kernel<F32>, dim3(NT, BHq), dim3(512), st,
+                       (const TI*)q, PS(q_strides), (const TI*)k, PS(k_strides), (const TI*)w, PS(w_strides), (const TI*)beta,
                        PS(beta_strides), HQ, H, T, ws, bw);
   }
   LUCID_TIMED_LAUNCH(phip, "path_reduce_kernel", lucid::path_reduce_kernel<F32>, dim3((T + 3) / 4, BH), st, HQ, H, T,

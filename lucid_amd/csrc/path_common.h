@@ -86,55 +86,59 @@ __device__ __forceinline__ void zero44(float acc[4][4]) {
     for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
 }
 
-// One merge of two inverted s x s diagonal blocks A = [a, a+s), B = [a+s, a+2s) of a
-// unit lower matrix (I + N): X_BA = -X_B (N_BA X_A), computed in place in the N_BA block
-// in two products; each thread owns 4 consecutive columns of one row of a pair.
+// One merge of two inverted S x S diagonal blocks A = [a, a+S), B = [a+S, a+2S) of a unit
+// lower matrix (I + N): X_BA = -X_B (N_BA X_A), computed in place in the N_BA block in two
+// products (Y = N_BA X_A, then -X_B Y) with a barrier after each read and each write; thread
+// qd owns 4 consecutive columns of one row of a pair.
+template <int S>
+struct MergeQuad {
+  bool act;
+  int i, j0, ao, bo;
+  __device__ __forceinline__ explicit MergeQuad(int qd) {
+    constexpr int QPP = S * S / 4;  // column quads per pair
+    act = qd < (64 / (2 * S)) * QPP;
+    const int p = qd / QPP, rem = qd - p * QPP;
+    i = rem / (S / 4);
+    j0 = 4 * (rem - i * (S / 4));
+    ao = 2 * p * S;
+    bo = ao + S;
+  }
+  // Y = N_BA X_A (X = false) or X_B Y (X = true)
+  template <bool X>
+  __device__ __forceinline__ f32x4 product(const float (*M)[68]) const {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    if (act) {
+#pragma unroll
+      for (int kk = 0; kk < S; ++kk) {
+        const float a = M[bo + i][(X ? bo : ao) + kk];
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&M[(X ? bo : ao) + kk][ao + j0]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = fmaf(a, x[e], acc[e]);
+      }
+    }
+    return acc;
+  }
+  __device__ __forceinline__ void put(float (*M)[68], const f32x4& x) const {
+    if (act) *reinterpret_cast<f32x4*>(&M[bo + i][ao + j0]) = x;
+  }
+};
+
 template <int S>
 __device__ __forceinline__ void merge_lower_blocks(float (*M)[68]) {
-  constexpr int QPP = S * S / 4;         // column quads per pair
-  constexpr int NQ = (64 / (2 * S)) * QPP;  // quads of all pairs
-  const int qd = threadIdx.x;
-  const bool act = qd < NQ;
-  const int p = qd / QPP, rem = qd - p * QPP;
-  const int i = rem / (S / 4), j0 = 4 * (rem - i * (S / 4));
-  const int ao = 2 * p * S, bo = ao + S;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  if (act) {  // Y = N_BA X_A
-#pragma unroll
-    for (int kk = 0; kk < S; ++kk) {
-      const float a = M[bo + i][ao + kk];
-      const f32x4 x = *reinterpret_cast<const f32x4*>(&M[ao + kk][ao + j0]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = fmaf(a, x[e], acc[e]);
-    }
-  }
+  const MergeQuad<S> m(threadIdx.x);
+  const f32x4 y = m.template product<false>(M);
   __syncthreads();
-  if (act) *reinterpret_cast<f32x4*>(&M[bo + i][ao + j0]) = acc;
+  m.put(M, y);
   __syncthreads();
-  if (act) {  // X_BA = -X_B Y
-    acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kk = 0; kk < S; ++kk) {
-      const float a = M[bo + i][bo + kk];
-      const f32x4 y = *reinterpret_cast<const f32x4*>(&M[bo + kk][ao + j0]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = fmaf(a, y[e], acc[e]);
-    }
-  }
+  const f32x4 x = m.template product<true>(M);
   __syncthreads();
-  if (act) *reinterpret_cast<f32x4*>(&M[bo + i][ao + j0]) = -acc;
+  m.put(M, -x);
   __syncthreads();
 }
 
-// (I + M)^-1 in place for a strictly lower 64x64 fp32 LDS matrix M (its diagonal and
-// strictly upper part must hold zeros; the result has a unit diagonal and zeros above).
-// Called by all 256 threads of the block; the caller syncs before, the function syncs
-// before returning.  Wave w inverts the 16x16 diagonal block w by forward substitution
-// (lane c < 16 solves column c: x_r = delta_rc - sum_{k<r} M_rk x_k); the blocks are
-// then merged 16 -> 32 -> 64 through X_BA = -X_B N_BA X_A.  A 64-deep solve in one
-// wave has four times the dependent work and leaves three waves idle.
-__device__ __forceinline__ void invert_unit_lower64(float (*M)[68]) {
-  const int w = threadIdx.x >> 6, c = threadIdx.x & 63;
+// The four 16x16 diagonal blocks of (I + M)^-1 in place (wave w < 4: block w) by forward
+// substitution: lane c < 16 solves column c, x_r = delta_rc - sum_{k<r} M_rk x_k.
+__device__ __forceinline__ void invert_lower16(float (*M)[68], int w, int c) {
   if (c < 16) {
     const int o = 16 * w;
     float x[16];
@@ -157,6 +161,16 @@ __device__ __forceinline__ void invert_unit_lower64(float (*M)[68]) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) M[o + r][o + c] = x[r];
   }
+}
+
+// (I + M)^-1 in place for a strictly lower 64x64 fp32 LDS matrix M (its diagonal and
+// strictly upper part must hold zeros; the result has a unit diagonal and zeros above).
+// Called by all 256 threads of the block; the caller syncs before, the function syncs
+// before returning.  Wave w inverts the 16x16 diagonal block w; the blocks are then merged
+// 16 -> 32 -> 64 through X_BA = -X_B N_BA X_A.  A 64-deep solve in one wave has four times
+// the dependent work and leaves three waves idle.
+__device__ __forceinline__ void invert_unit_lower64(float (*M)[68]) {
+  invert_lower16(M, threadIdx.x >> 6, threadIdx.x & 63);
   __syncthreads();
   merge_lower_blocks<16>(M);
   merge_lower_blocks<32>(M);
@@ -344,5 +358,108 @@ __device__ __forceinline__ f32x16 dl_neg(f32x16 x) {
   return x;
 }
 
+// ---------------------------------------------------------------------------
+// 64x64 matrices held in LDS as bf16 planes, split once when they are written: plane 0 the
+// rounded value, plane 1 (NP = 2) the rest, so a product reads operands that mgemm64 would
+// gather and split anew at every use (same 3-term products, same rounding).  Rows of 128
+// bytes, 16-byte chunks swizzled (chunk c of row r at c ^ (r & 7)); columns come through
+// transposing reads.  NP = 1: a matrix of bf16 values, whose second term is zero and left out.
+// Tiles are transposed to mgemm64's: of wave w4's 32x32 tile (rows 32 (w4 >> 1), columns
+// 32 (w4 & 1)), lane l holds row l % 32, columns drow(e, l / 32).
+// ---------------------------------------------------------------------------
+template <int NP>
+struct PlaneMat {
+  bf16 p[NP][64 * 64];
+};
+
+// opA(A) opB(B) + acc for wave w4 of four
+template <bool TA, bool TB, int NA, int NB>
+__device__ __forceinline__ f32x16 pgemm64(const PlaneMat<NA>& A, const PlaneMat<NB>& B, int w4, f32x16 acc) {
+  const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
+  const int m0 = 32 * (w4 >> 1), n0 = 32 * (w4 & 1);
+  // rows r0 + l32 of X, depth 16 st + slot; PERM: depth 16 st + jmap(slot), the transposing reads' order
+  auto rows = [&](const bf16* X, int r0, int st, auto perm) {
+    if constexpr (!decltype(perm)::value) return ld8(swz<8>(X, r0 + l32, 2 * st + g));
+    const bf16x4 a = *reinterpret_cast<const bf16x4*>(swz<8>(X, r0 + l32, 2 * st) + 4 * g);
+    const bf16x4 b = *reinterpret_cast<const bf16x4*>(swz<8>(X, r0 + l32, 2 * st + 1) + 4 * g);
+    return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  };
+#pragma unroll
+  for (int st = 0; st < 4; ++st) {
+    bf16x8 a[NA], b[NB];
+#pragma unroll
+    for (int pl = 0; pl < NA; ++pl) {
+      if constexpr (TA) a[pl] = lds_tr_a<8>(A.p[pl], 16 * st, m0);
+      else a[pl] = rows(A.p[pl], m0, st, std::bool_constant<!TB>{});
+    }
+#pragma unroll
+    for (int pl = 0; pl < NB; ++pl) {
+      if constexpr (!TB) b[pl] = lds_tr_a<8>(B.p[pl], 16 * st, n0);
+      else b[pl] = rows(B.p[pl], n0, st, std::bool_constant<TA>{});
+    }
+    acc = mfma32(b[0], a[0], acc);
+    if constexpr (NA == 2) acc = mfma32(b[0], a[1], acc);
+    if constexpr (NB == 2) acc = mfma32(b[1], a[0], acc);
+  }
+  return acc;
+}
+
+// row and first column of quad q (four columns, elements 4 q .. 4 q + 3) of this lane's tile
+__device__ __forceinline__ int pl_row(int w4) { return 32 * (w4 >> 1) + ((int)threadIdx.x & 31); }
+__device__ __forceinline__ int pl_col(int w4, int q) {
+  return 32 * (w4 & 1) + 8 * q + 4 * (((int)threadIdx.x >> 5) & 1);
+}
+// M[tile] <- x; mode 0: all, 1: col <= row (tril), 2: col < row (strictly lower)
+__device__ __forceinline__ f32x4 pl_quad(const f32x16& x, int w4, int q, int mode) {
+  const int r = pl_row(w4), c0 = pl_col(w4, q);
+  f32x4 f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const bool keep = mode == 0 || (mode == 1 ? c0 + u <= r : c0 + u < r);
+    f[u] = keep ? x[4 * q + u] : 0.f;
+  }
+  return f;
+}
+__device__ __forceinline__ void pl_store(PlaneMat<2>& M, const f32x16& x, int w4, int mode) {
+  const int r = pl_row(w4);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c0 = pl_col(w4, q);
+    const f32x4 f = pl_quad(x, w4, q, mode);
+    bf16x4 h, l;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      h[u] = (bf16)f[u];
+      l[u] = (bf16)(f[u] - (float)h[u]);
+    }
+    const int off = swz_off<8>(r, c0 >> 3) + (c0 & 7);
+    *reinterpret_cast<bf16x4*>(M.p[0] + off) = h;
+    *reinterpret_cast<bf16x4*>(M.p[1] + off) = l;
+  }
+}
+// 16-byte chunk c of row r from eight fp32 values
+template <int NP>
+__device__ __forceinline__ void pl_put8(PlaneMat<NP>& M, int r, int c, const f32x4& x, const f32x4& y) {
+  const float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  bf16x8 h, l;
+  split_vals(v, h, l);
+  *reinterpret_cast<bf16x8*>(M.p[0] + swz_off<8>(r, c)) = h;
+  if constexpr (NP == 2) *reinterpret_cast<bf16x8*>(M.p[1] + swz_off<8>(r, c)) = l;
+}
+// this lane's tile of a row-major fp32 64x64 matrix (row stride 64), and back
+__device__ __forceinline__ f32x16 pl_load(const float* __restrict__ src, int w4) {
+  f32x16 x;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 f = *reinterpret_cast<const f32x4*>(src + pl_row(w4) * 64 + pl_col(w4, q));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[4 * q + u] = f[u];
+  }
+  return x;
+}
+__device__ __forceinline__ void pl_save(float* __restrict__ dst, const f32x16& x, int w4) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) *reinterpret_cast<f32x4*>(dst + pl_row(w4) * 64 + pl_col(w4, q)) = pl_quad(x, w4, q, 0);
+}
 
 }  // namespace lucid
