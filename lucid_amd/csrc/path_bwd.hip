@@ -1361,24 +1361,12 @@ __global__ __launch_bounds__(512) void path_wy_bwd_kernel(const pin_t<F32>* __re
       pdk[u] = *reinterpret_cast<const f32x4*>(dkt + 16 * ht + 4 * u);
     }
   }
-  // eight values of the caller's row r8 into the planes; returns them in fp32
-  auto rows_in = [&](PlaneMat<NPI>& M, const pin_t<F32>* src, f32x4 x[2]) {
-    if constexpr (F32) {
-      x[0] = *reinterpret_cast<const f32x4*>(src);
-      x[1] = *reinterpret_cast<const f32x4*>(src + 4);
-      pl_put8(M, r8, c8, x[0], x[1]);
-    } else {
-      const bf16x8 v = ld8(src);
-      *reinterpret_cast<bf16x8*>(M.p[0] + swz_off<8>(r8, c8)) = v;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e >> 2][e & 3] = (float)v[e];
-    }
-  };
+  const pin_t<F32>* wp = w_ + b * wst.b + h * wst.h + (int64_t)t0 * wst.t;
   {
     f32x4 x[2];
-    rows_in(Q, q + b * qs.b + hq * qs.h + (int64_t)(t0 + r8) * qs.t + 8 * c8, x);
-    rows_in(K, k + b * ks.b + h * ks.h + (int64_t)(t0 + r8) * ks.t + 8 * c8, x);
-    rows_in(W, w_ + b * wst.b + h * wst.h + (int64_t)(t0 + r8) * wst.t + 8 * c8, x);
+    pl_rows_in<F32>(Q, q + b * qs.b + hq * qs.h + (int64_t)(t0 + r8) * qs.t + 8 * c8, r8, c8, x);
+    pl_rows_in<F32>(K, k + b * ks.b + h * ks.h + (int64_t)(t0 + r8) * ks.t + 8 * c8, r8, c8, x);
+    pl_rows_in<F32>(W, wp + (int64_t)r8 * wst.t + 8 * c8, r8, c8, x);
     const float bt = (float)beta[b * bst.b + h * bst.h + (int64_t)(t0 + r8) * bst.t];
     if (c8 == 0) bsh[r8] = bt;
     pl_put8(Wb, r8, c8, bt * x[0], bt * x[1]);
@@ -1406,40 +1394,38 @@ __global__ __launch_bounds__(512) void path_wy_bwd_kernel(const pin_t<F32>* __re
 #pragma unroll
     for (int u = 0; u < 2; ++u) pl_put8(M, hr, hc + u, x[2 * u], x[2 * u + 1]);
   };
-  const MergeQuad<16> m16(ht);
-  const MergeQuad<32> m32(ht);
-  f32x4 mq;
+  InvertSteps inv(ht);
   if (h0) {
-    invert_lower16(Tm.f, w, tid & 63);
+    inv.step<0>(Tm.f, w4);
   } else {
     aW = dl_neg(pgemm64<false, true>(S1, S2, w4, z));   // -W2 dHc^T
     aW2 = dl_neg(pgemm64<false, false>(W, S2, w4, z));  // -W dHc
   }
   __syncthreads();
-  if (h0) mq = m16.product<false>(Tm.f);
+  if (h0) inv.step<1>(Tm.f, w4);
   else put16(S2, pdq);  // d q~
   __syncthreads();
   if (h0) {
-    m16.put(Tm.f, mq);
+    inv.step<2>(Tm.f, w4);
   } else {
     pl_store(S4, pgemm64<false, true>(Wb, K, w4, z), w4, 2);  // WBK
     dQW = dl_neg(pgemm64<false, true>(S2, S1, w4, z));        // -dq~ W2^T
   }
   __syncthreads();
-  if (h0) mq = m16.product<true>(Tm.f);
+  if (h0) inv.step<3>(Tm.f, w4);
   else aW2 = sub(aW2, pgemm64<true, false>(S3, S2, w4, z));  // QW^T dq~
   __syncthreads();
-  if (h0) m16.put(Tm.f, -mq);
+  if (h0) inv.step<4>(Tm.f, w4);
   else put16(S2, pdk);  // d k~
   __syncthreads();
-  if (h0) mq = m32.product<false>(Tm.f);
+  if (h0) inv.step<5>(Tm.f, w4);
   else dTW = dl_neg(pgemm64<false, true>(W, S2, w4, z));  // -W dk~^T
   __syncthreads();
-  if (h0) m32.put(Tm.f, mq);
+  if (h0) inv.step<6>(Tm.f, w4);
   __syncthreads();
-  if (h0) mq = m32.product<true>(Tm.f);
+  if (h0) inv.step<7>(Tm.f, w4);
   __syncthreads();
-  if (h0) m32.put(Tm.f, -mq);
+  if (h0) inv.step<8>(Tm.f, w4);
   __syncthreads();
   {  // to planes, in place
     f32x4 x[2];
@@ -1508,17 +1494,11 @@ __global__ __launch_bounds__(512) void path_wy_bwd_kernel(const pin_t<F32>* __re
     // dW += beta dWb; dbeta_r = sum_c dWb[r][c] W[r][c]
     const int r = pl_row(w4);
     const float bt = bsh[r];
+    const f32x16 wr = pl_rows<F32>(W, wp, wst.t, w4);
     float s = 0.f;
-#pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-      const int c0 = pl_col(w4, qd), off = swz_off<8>(r, c0 >> 3) + (c0 & 7);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        float x = (float)W.p[0][off + u];
-        if constexpr (F32) x += (float)W.p[NPI - 1][off + u];
-        s = fmaf(aWb[4 * qd + u], x, s);
-        aW[4 * qd + u] += bt * aWb[4 * qd + u];
-      }
+    DL_FOR_E {
+      s = fmaf(aWb[e], wr[e], s);
+      aW[e] += bt * aWb[e];
     }
     s = wave_sum32(s);
     if ((tid & 63) < 32) dbs[w4 & 1][r] = s;

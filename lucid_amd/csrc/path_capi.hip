@@ -172,8 +172,8 @@ int launch_front(const void* q, const int64_t* q_strides, const void* k, const i
                        HQ, H, T, ws);
     return 0;
   }
-  LUCID_TIMED_LAUNCH(phip, "path_chunk_kernel", lucid::path_chunk_kernel<F32>, dim3(NT, BHq), st, (const TI*)q,
-                     PS(q_strides), (const TI*)k, PS(k_strides), (const TI*)w, PS(w_strides), (const TI*)beta,
+  LUCID_TIMED_LAUNCH_B(phip, "path_chunk_kernel", lucid::path_chunk_kernel<F32>, dim3(NT, BHq), dim3(512), st,
+                       (const TI*)q, PS(q_strides), (const TI*)k, PS(k_strides), (const TI*)w, PS(w_strides), (const TI*)beta,
                      PS(beta_strides), HQ, H, T, scale, softmax, ws);
   LUCID_TIMED_LAUNCH(phip, "path_large_kernel", lucid::path_large_kernel<F32>, dim3(NS, BH), st, T, ws);
   LUCID_TIMED_LAUNCH(phip, "path_transport_kernel", lucid::path_transport_kernel<F32>, dim3(BHq, (NT + 1) / 2), st, HQ,

@@ -163,6 +163,27 @@ __device__ __forceinline__ void invert_lower16(float (*M)[68], int w, int c) {
   }
 }
 
+// Step st = 0 .. 8 of invert_unit_lower64 for the four waves w4 (thread ht of their 256), a
+// barrier of the whole block after each: lets other waves of the block work between them.
+struct InvertSteps {
+  MergeQuad<16> m16;
+  MergeQuad<32> m32;
+  f32x4 x;
+  __device__ __forceinline__ explicit InvertSteps(int ht) : m16(ht), m32(ht) {}
+  template <int ST>
+  __device__ __forceinline__ void step(float (*M)[68], int w4) {
+    if constexpr (ST == 0) invert_lower16(M, w4, threadIdx.x & 63);
+    if constexpr (ST == 1) x = m16.product<false>(M);
+    if constexpr (ST == 2) m16.put(M, x);
+    if constexpr (ST == 3) x = m16.product<true>(M);
+    if constexpr (ST == 4) m16.put(M, -x);
+    if constexpr (ST == 5) x = m32.product<false>(M);
+    if constexpr (ST == 6) m32.put(M, x);
+    if constexpr (ST == 7) x = m32.product<true>(M);
+    if constexpr (ST == 8) m32.put(M, -x);
+  }
+};
+
 // (I + M)^-1 in place for a strictly lower 64x64 fp32 LDS matrix M (its diagonal and
 // strictly upper part must hold zeros; the result has a unit diagonal and zeros above).
 // Called by all 256 threads of the block; the caller syncs before, the function syncs
@@ -446,12 +467,12 @@ __device__ __forceinline__ void pl_put8(PlaneMat<NP>& M, int r, int c, const f32
   *reinterpret_cast<bf16x8*>(M.p[0] + swz_off<8>(r, c)) = h;
   if constexpr (NP == 2) *reinterpret_cast<bf16x8*>(M.p[1] + swz_off<8>(r, c)) = l;
 }
-// this lane's tile of a row-major fp32 64x64 matrix (row stride 64), and back
-__device__ __forceinline__ f32x16 pl_load(const float* __restrict__ src, int w4) {
+// this lane's tile of row-major fp32 64x64 rows (row stride st; 64 for a matrix), and back
+__device__ __forceinline__ f32x16 pl_load(const float* __restrict__ src, int w4, int64_t st = 64) {
   f32x16 x;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const f32x4 f = *reinterpret_cast<const f32x4*>(src + pl_row(w4) * 64 + pl_col(w4, q));
+    const f32x4 f = *reinterpret_cast<const f32x4*>(src + pl_row(w4) * st + pl_col(w4, q));
 #pragma unroll
     for (int u = 0; u < 4; ++u) x[4 * q + u] = f[u];
   }
@@ -460,6 +481,54 @@ __device__ __forceinline__ f32x16 pl_load(const float* __restrict__ src, int w4)
 __device__ __forceinline__ void pl_save(float* __restrict__ dst, const f32x16& x, int w4) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) *reinterpret_cast<f32x4*>(dst + pl_row(w4) * 64 + pl_col(w4, q)) = pl_quad(x, w4, q, 0);
+}
+
+// this lane's tile of rows of the caller's tensor in fp32 (row stride st), whose bf16 planes
+// are in M: from the plane where that is the whole value, else from memory
+template <bool F32>
+__device__ __forceinline__ f32x16 pl_rows(const PlaneMat<F32 ? 2 : 1>& M, const pin_t<F32>* __restrict__ src,
+                                          int64_t st, int w4) {
+  if constexpr (F32) return pl_load(src, w4, st);
+  f32x16 x;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c0 = pl_col(w4, q);
+    const bf16x4 v = *reinterpret_cast<const bf16x4*>(M.p[0] + swz_off<8>(pl_row(w4), c0 >> 3) + (c0 & 7));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[4 * q + u] = (float)v[u];
+  }
+  return x;
+}
+// eight values of the caller's row (chunk c of row r) into the planes; x: the values in fp32
+template <bool F32>
+__device__ __forceinline__ void pl_rows_in(PlaneMat<F32 ? 2 : 1>& M, const pin_t<F32>* __restrict__ src, int r, int c,
+                                           f32x4 x[2]) {
+  if constexpr (F32) {
+    x[0] = *reinterpret_cast<const f32x4*>(src);
+    x[1] = *reinterpret_cast<const f32x4*>(src + 4);
+    pl_put8(M, r, c, x[0], x[1]);
+  } else {
+    const bf16x8 v = ld8(src);
+    *reinterpret_cast<bf16x8*>(M.p[0] + swz_off<8>(r, c)) = v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e >> 2][e & 3] = (float)v[e];
+  }
+}
+// this lane's tile to row-major bf16 rows (row stride 64) and, NP = 2, the rest at dst + lo
+template <int NP>
+__device__ __forceinline__ void pl_save_split(bf16* __restrict__ dst, int64_t lo, const f32x16& x, int w4) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    bf16x4 h, l;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      h[u] = (bf16)x[4 * q + u];
+      l[u] = (bf16)(x[4 * q + u] - (float)h[u]);
+    }
+    bf16* d = dst + pl_row(w4) * 64 + pl_col(w4, q);
+    *reinterpret_cast<bf16x4*>(d) = h;
+    if constexpr (NP == 2) *reinterpret_cast<bf16x4*>(d + lo) = l;
+  }
 }
 
 }  // namespace lucid

@@ -49,128 +49,166 @@ struct PathFwdWs {
 // ---------------------------------------------------------------------------
 // WY form and in-chunk transforms (triangular_solve_fwd.py:118-148, parallel.py:39-51)
 // grid (NT, B*HQ).  kv-head outputs are written by the first query head of each group.
+// The products run on bf16 planes (pgemm64) in two sets of four waves: waves 0..3 form T_inv
+// while waves 4..7 form what does not need it, then waves 4..7 form L_diag and its inverse
+// while waves 0..3 write Hc, k~ and q~.  B1 H16 T8192 bf16: 145 us with four
+// waves on fp32 operands split at every use, 111 this way (262 MB in and out: 55 us).
 // ---------------------------------------------------------------------------
 // F32: fp32 inputs; k~ is written as hi / lo planes
 template <bool F32>
-__global__ __launch_bounds__(256) void path_chunk_kernel(const pin_t<F32>* __restrict__ q, Strides qs,
+__global__ __launch_bounds__(512) void path_chunk_kernel(const pin_t<F32>* __restrict__ q, Strides qs,
                                                          const pin_t<F32>* __restrict__ k, Strides ks,
-                                                         const pin_t<F32>* __restrict__ w, Strides wst,
+                                                         const pin_t<F32>* __restrict__ w_, Strides wst,
                                                          const pin_t<F32>* __restrict__ beta, Strides bst, int HQ, int H,
                                                          int T, float scale, int softmax, PathFwdWs ws) {
-  __shared__ __attribute__((aligned(16))) float Wm[64][68];
-  __shared__ __attribute__((aligned(16))) float Wb[64][68];
-  __shared__ __attribute__((aligned(16))) float Tm[64][68];
-  __shared__ __attribute__((aligned(16))) float W2s[64][68];
-  __shared__ __attribute__((aligned(16))) float Qs[64][68];
-  __shared__ __attribute__((aligned(16))) float Ks[64][68];
-  __shared__ __attribute__((aligned(16))) float X[64][68];
+  __shared__ __attribute__((aligned(16))) PlaneMat<F32 ? 2 : 1> W, Q, K;
+  __shared__ __attribute__((aligned(16))) PlaneMat<2> Wb, QW, W2, TW;
+  __shared__ __attribute__((aligned(16))) union {
+    float f[64][68];  // the inverses are formed in fp32
+    PlaneMat<2> p;
+  } Tm, X;            // X: WBK, then L_diag
   const int c = blockIdx.x, bhq = blockIdx.y;
   const int NT = T / PC;
   const int G = HQ / H;
   const int b = bhq / HQ, hq = bhq - b * HQ, h = hq / G;
   const int bh = b * H + h;
   const bool kvw = (hq % G) == 0;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), w4 = w & 3;
+  const bool h0 = w < 4;
+  const int ht = tid & 255, r8 = tid >> 3, c8 = tid & 7;
   const int t0 = c * PC;
   const f32x16 z = zero16();
-  const int cl = dl_col();
   if (c == 0 && tid == 0) ws.counters[bhq] = 0;
 
-  load_rows64_f32(Wm, w + b * wst.b + h * wst.h + (int64_t)t0 * wst.t, wst.t);
-  load_rows64_f32(Qs, q + b * qs.b + hq * qs.h + (int64_t)t0 * qs.t, qs.t);
-  load_rows64_f32(Ks, k + b * ks.b + h * ks.h + (int64_t)t0 * ks.t, ks.t);
-  __syncthreads();
+  const pin_t<F32>* qp = q + b * qs.b + hq * qs.h + (int64_t)t0 * qs.t;
+  const pin_t<F32>* kp = k + b * ks.b + h * ks.h + (int64_t)t0 * ks.t;
   {
-    const int r = tid >> 2, cc = (tid & 3) * 16;
-    const float bt = (float)beta[b * bst.b + h * bst.h + (int64_t)(t0 + r) * bst.t];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) Wb[r][cc + e] = bt * Wm[r][cc + e];
+    f32x4 x[2];
+    pl_rows_in<F32>(Q, qp + (int64_t)r8 * qs.t + 8 * c8, r8, c8, x);
+    pl_rows_in<F32>(K, kp + (int64_t)r8 * ks.t + 8 * c8, r8, c8, x);
+    pl_rows_in<F32>(W, w_ + b * wst.b + h * wst.h + (int64_t)(t0 + r8) * wst.t + 8 * c8, r8, c8, x);
+    const float bt = (float)beta[b * bst.b + h * bst.h + (int64_t)(t0 + r8) * bst.t];
+    pl_put8(Wb, r8, c8, bt * x[0], bt * x[1]);
   }
   __syncthreads();
-  // Products on the matrix cores (mgemm64); each wave keeps its 32x32 tile in D layout.
   // a = stril(beta W W^T) -> Tm, then T_inv = (I + a)^-1 in place
-  dl_store(Tm, mgemm64<false, true>(Wb, Wm, z), 2);
-  __syncthreads();
-  invert_unit_lower64(Tm);
-  // W2 = T_inv (beta W)
-  {
-    const f32x16 acc = mgemm64<false, false>(Tm, Wb, z);
-    dl_store(W2s, acc, 0);
-    if (kvw) {
-      float* dst = ws.w2 + ((int64_t)bh * T + t0) * 64;
-      DL_FOR_E dst[dl_row(e) * 64 + cl] = acc[e];
-    }
+  f32x16 qk = z;  // waves 4..7
+  InvertSteps inv(ht);
+  if (h0) {
+    const f32x16 a = pgemm64<false, true>(Wb, W, w4, z);
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd)
+      *reinterpret_cast<f32x4*>(&Tm.f[pl_row(w4)][pl_col(w4, qd)]) = pl_quad(a, w4, qd, 2);
   }
   __syncthreads();
-  // Hc = I - W^T W2
-  if (kvw) {
-    const f32x16 acc = mgemm64<true, false>(Wm, W2s, z);
-    float* dst = ws.hc + ((int64_t)bh * NT + c) * 4096;
-    bf16* dsts = ws.hcs + ((int64_t)bh * NT + c) * 8192;
-    DL_FOR_E {
-      const int r = dl_row(e);
-      const float x = (r == cl ? 1.f : 0.f) - acc[e];
-      dst[r * 64 + cl] = x;
-      put_split<2>(dsts, 4096, r * 64 + cl, x);
-    }
-  }
-  // WBK = stril(beta W K^T) -> X
-  dl_store(X, mgemm64<false, true>(Wb, Ks, z), 2);
+  if (h0) inv.step<0>(Tm.f, w4);
+  else pl_store(X.p, pgemm64<false, true>(Wb, K, w4, z), w4, 2);  // WBK = stril(beta W K^T)
   __syncthreads();
-  // TW = T_inv WBK -> Wb (every read of beta W came before the last barrier)
-  dl_store(Wb, mgemm64<false, false>(Tm, X, z), 0);
+  if (h0) inv.step<1>(Tm.f, w4);
+  else pl_store(QW, pgemm64<false, true>(Q, W, w4, z), w4, 1);  // QW = tril(Q W^T)
   __syncthreads();
-  // k~ = K - TW^T W
-  if (kvw) {
-    const f32x16 acc = mgemm64<true, false>(Wb, Wm, z);
-    bf16* dst = ws.kt + ((int64_t)bh * T + t0) * 64;
-    DL_FOR_E {
-      const int r = dl_row(e);
-      put_split<F32 ? 2 : 1>(dst, ws.lo_kt, r * 64 + cl, Ks[r][cl] - acc[e]);
-    }
-  }
-  // QW = tril(Q W^T) -> X (every read of WBK came before the last barrier)
-  dl_store(X, mgemm64<false, true>(Qs, Wm, z), 1);
+  if (h0) inv.step<2>(Tm.f, w4);
   __syncthreads();
-  // q~ = Q - QW W2
-  {
-    const f32x16 acc = mgemm64<false, false>(X, W2s, z);
-    float* dst = ws.qt + ((int64_t)bhq * T + t0) * 64;
-    DL_FOR_E {
-      const int r = dl_row(e);
-      dst[r * 64 + cl] = Qs[r][cl] - acc[e];
-    }
+  if (h0) inv.step<3>(Tm.f, w4);
+  else qk = pgemm64<false, true>(Q, K, w4, z);
+  __syncthreads();
+  if (h0) inv.step<4>(Tm.f, w4);
+  __syncthreads();
+  if (h0) inv.step<5>(Tm.f, w4);
+  __syncthreads();
+  if (h0) inv.step<6>(Tm.f, w4);
+  __syncthreads();
+  if (h0) inv.step<7>(Tm.f, w4);
+  __syncthreads();
+  if (h0) inv.step<8>(Tm.f, w4);
+  __syncthreads();
+  {  // to planes, in place
+    f32x4 x[2];
+    x[0] = *reinterpret_cast<const f32x4*>(&Tm.f[r8][8 * c8]);
+    x[1] = *reinterpret_cast<const f32x4*>(&Tm.f[r8][8 * c8 + 4]);
+    __syncthreads();
+    pl_put8(Tm.p, r8, c8, x[0], x[1]);
   }
-  // A_diag = tril(Q K^T - QW TW); L_diag = stril(exp(s A - 1/s)) -> W2s, global
+  __syncthreads();
+  if (h0) {  // W2 = T_inv (beta W)
+    const f32x16 acc = pgemm64<false, false>(Tm.p, Wb, w4, z);
+    pl_store(W2, acc, w4, 0);
+    if (kvw) pl_save(ws.w2 + ((int64_t)bh * T + t0) * 64, acc, w4);
+  } else {  // TW = T_inv WBK
+    pl_store(TW, pgemm64<false, false>(Tm.p, X.p, w4, z), w4, 0);
+  }
+  __syncthreads();
+  // A_diag = tril(Q K^T - QW TW); L_diag = stril(exp(s A - 1/s)) -> X, global
   // (PaTH softmax: the logits themselves, diagonal included; no inverse)
-  const f32x16 qk = mgemm64<false, true>(Qs, Ks, z);
-  const f32x16 qt = mgemm64<false, false>(X, Wb, z);
-  float* dst = ws.ld + ((int64_t)bhq * NT + c) * 4096;
-  if (softmax) {
-    DL_FOR_E {
-      const int r = dl_row(e);
-      dst[r * 64 + cl] = cl <= r ? qk[e] - qt[e] : 0.f;
+  if (!h0) {
+    const f32x16 qt = pgemm64<false, false>(QW, TW, w4, z);
+    float* dst = ws.ld + ((int64_t)bhq * NT + c) * 4096;
+    f32x16 a;
+    if (softmax) {
+      DL_FOR_E a[e] = qk[e] - qt[e];
+    } else {
+      const float sl2 = scale * LOG2E_F, cc0 = LOG2E_F / scale;
+      DL_FOR_E a[e] = __builtin_amdgcn_exp2f(fmaf(qk[e] - qt[e], sl2, -cc0));
     }
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) {
+      const int r = pl_row(w4), c0 = pl_col(w4, qd);
+      const f32x4 f = pl_quad(a, w4, qd, softmax ? 1 : 2);
+      *reinterpret_cast<f32x4*>(dst + r * 64 + c0) = f;
+      if (!softmax) *reinterpret_cast<f32x4*>(&X.f[r][c0]) = f;
+    }
+  } else if (kvw) {  // Hc = I - W^T W2
+    f32x16 acc = dl_neg(pgemm64<true, false>(W, W2, w4, z));
+    DL_FOR_E {
+      if (pl_col(w4, e >> 2) + (e & 3) == pl_row(w4)) acc[e] = 1.f + acc[e];
+    }
+    pl_save(ws.hc + ((int64_t)bh * NT + c) * 4096, acc, w4);
+    pl_save_split<2>(ws.hcs + ((int64_t)bh * NT + c) * 8192, 4096, acc, w4);
+  }
+  __syncthreads();
+  // Y = (I + L_diag)^-1 (waves 4..7) beside k~ = K - TW^T W and q~ = Q - QW W2
+  auto ktilde = [&]() {
+    if (!kvw) return;
+    const f32x16 t = pgemm64<true, false>(TW, W, w4, z);
+    f32x16 x = pl_rows<F32>(K, kp, ks.t, w4);
+    DL_FOR_E x[e] -= t[e];
+    pl_save_split<F32 ? 2 : 1>(ws.kt + ((int64_t)bh * T + t0) * 64, ws.lo_kt, x, w4);
+  };
+  auto qtilde = [&]() {
+    const f32x16 t = pgemm64<false, false>(QW, W2, w4, z);
+    f32x16 x = pl_rows<F32>(Q, qp, qs.t, w4);
+    DL_FOR_E x[e] -= t[e];
+    pl_save(ws.qt + ((int64_t)bhq * T + t0) * 64, x, w4);
+  };
+  if (softmax) {
+    if (h0) ktilde();
+    else qtilde();
     return;
   }
-  __syncthreads();  // the q~ product above still reads W2s
-  {
-    const float sl2 = scale * LOG2E_F, cc0 = LOG2E_F / scale;
-    DL_FOR_E {
-      const int r = dl_row(e);
-      const float v = cl < r ? __builtin_amdgcn_exp2f(fmaf(qk[e] - qt[e], sl2, -cc0)) : 0.f;
-      W2s[r][cl] = v;
-      dst[r * 64 + cl] = v;
-    }
-  }
+  if (h0) ktilde();
+  else inv.step<0>(X.f, w4);
   __syncthreads();
-  invert_unit_lower64(W2s);
+  if (h0) qtilde();
+  else inv.step<1>(X.f, w4);
+  __syncthreads();
+  if (!h0) inv.step<2>(X.f, w4);
+  __syncthreads();
+  if (!h0) inv.step<3>(X.f, w4);
+  __syncthreads();
+  if (!h0) inv.step<4>(X.f, w4);
+  __syncthreads();
+  if (!h0) inv.step<5>(X.f, w4);
+  __syncthreads();
+  if (!h0) inv.step<6>(X.f, w4);
+  __syncthreads();
+  if (!h0) inv.step<7>(X.f, w4);
+  __syncthreads();
+  if (!h0) inv.step<8>(X.f, w4);
+  __syncthreads();
   {
-    float* dy = ws.y + ((int64_t)bhq * NT + c) * 4096;
-    for (int i = 0; i < 4; ++i) {
-      const int f = 4 * (tid + 256 * i);
-      *reinterpret_cast<f32x4*>(dy + f) = *reinterpret_cast<const f32x4*>(&W2s[f >> 6][f & 63]);
-    }
+    float* dy = ws.y + ((int64_t)bhq * NT + c) * 4096 + 8 * tid;
+    *reinterpret_cast<f32x4*>(dy) = *reinterpret_cast<const f32x4*>(&X.f[r8][8 * c8]);
+    *reinterpret_cast<f32x4*>(dy + 4) = *reinterpret_cast<const f32x4*>(&X.f[r8][8 * c8 + 4]);
   }
 }
 
