@@ -380,12 +380,14 @@ __global__ __launch_bounds__(64 * (WGR / RW)) LUCID_TWO_WAVES_IF(EXACT ? D == 64
   constexpr int NB = stage_bufs(D, F32);
   const int nblk = (T + WGR - 1) / WGR;
   const int id = blockIdx.x;
-  const int bhq = id % BHq;
-  const int ib = nblk - 1 - id / BHq;
-  const int b = bhq / Hq, hq = bhq - b * Hq;
-  const int h = hq / (Hq / Hkv);
-  const int bh = b * Hkv + h;
-  if ((mass[bh] > kExactMass) != EXACT) return;  // the other instance handles this head
+  const int G = Hq / Hkv;
+  const InstanceHeads<EXACT> heads(mass, BHq / G);
+  const int nq = heads.n * G;  // query heads of this instance
+  if (id >= nblk * nq) return;
+  const int slot = id % nq, ib = nblk - 1 - id / nq;
+  const int bh = heads.head(slot / G);
+  const int b = bh / Hkv, h = bh - b * Hkv;
+  const int hq = h * G + slot % G, bhq = b * Hq + hq;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;
   const int r0 = ib * WGR;
@@ -661,8 +663,9 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !EXACT) void luc
 
   const int NT = T / 64, NP = T / 128;
   const int id = blockIdx.x;
-  const int p = NP - 1 - id / BH, bh = id - (id / BH) * BH;
-  if ((mass[bh] > kExactMass) != EXACT) return;  // the other instance solves this head
+  const InstanceHeads<EXACT> heads(mass, BH);
+  if (id >= NP * heads.n) return;
+  const int p = NP - 1 - id / heads.n, bh = heads.head(id % heads.n);
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;
@@ -1199,8 +1202,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void l
 
   const int NT = T / 64, NP = T / 256;
   const int id = blockIdx.x;
-  const int p = NP - 1 - id / BH, bh = id - (id / BH) * BH;
-  if (mass[bh] > kExactMass) return;  // the exact instance of the 128-column chain solves this head
+  const InstanceHeads<false> heads(mass, BH);  // the exact instance of the 128-column chain solves the others
+  if (id >= NP * heads.n) return;
+  const int p = NP - 1 - id / heads.n, bh = heads.head(id % heads.n);
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;
@@ -1474,8 +1478,9 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && (!EXACT || (NT =
   constexpr int WGR = 128 * NT;  // rows per workgroup
   const int nblk = (T + WGR - 1) / WGR;
   const int id = blockIdx.x;
-  const int ib = nblk - 1 - id / BH, bh = id - (id / BH) * BH;  // heavy (late) blocks first
-  if ((mass[bh] > kExactMass) != EXACT) return;  // the other instance handles this head
+  const InstanceHeads<EXACT> heads(mass, BH);
+  if (id >= nblk * heads.n) return;
+  const int ib = nblk - 1 - id / heads.n, bh = heads.head(id % heads.n);  // heavy (late) blocks first
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;

@@ -21,6 +21,43 @@ struct Strides {
 // (N(0,1)-like) give m ~ 1e-2; keys along a shared direction give m ~ T.
 constexpr float kExactMass = 4.0f;
 
+// The heads of one chain instance (EXACT: mass above kExactMass), known only on the device:
+// both instances are launched over a grid for all BH heads, and the ids of each go to its own
+// heads first, densely, as if they were all there are (the rest return).  Leaving every
+// second id idle instead left half of the chip idle: ids go round robin over XCDs and shader
+// engines, so the working ones fell on the same half of them (B1 Hq32 Hkv4 d64 T16000, two
+// heads of each kind: dQ 1394 + 2149 -> 865 + 1295 us, row sums 396 + 552 -> 391 + 475, dV
+// chains 483 + 1069 -> 461 + 751).
+template <bool EXACT>
+struct InstanceHeads {
+  const float* mass;
+  int BH;
+  unsigned long long m0;  // the instance's heads among the first 64
+  int n;                  // and among all
+
+  __device__ __forceinline__ unsigned long long chunk(int c0) const {
+    const int i = c0 + (int)(threadIdx.x & 63);
+    return __ballot(i < BH && (mass[min(i, BH - 1)] > kExactMass) == EXACT);
+  }
+  __device__ __forceinline__ InstanceHeads(const float* mass_, int BH_) : mass(mass_), BH(BH_) {
+    m0 = chunk(0);
+    n = __popcll(m0);
+    for (int c0 = 64; c0 < BH; c0 += 64) n += __popcll(chunk(c0));
+  }
+  // the instance's head number k (0 <= k < n)
+  __device__ __forceinline__ int head(int k) const {
+    unsigned long long m = m0;
+    int c0 = 0;
+    for (int c = __popcll(m); k >= c; c = __popcll(m)) {
+      k -= c;
+      c0 += 64;
+      m = chunk(c0);
+    }
+    const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+    return c0 + __ffsll(__ballot(((m >> (threadIdx.x & 63)) & 1) && below == k)) - 1;
+  }
+};
+
 // Staged tiles in flight in the backward sweeps: three buffers (the tile in use, the next
 // one landed, the one after in flight), two for the fp32-input instances at head dim 128,
 // whose hi and lo tiles would not fit three deep in the 160 KB of LDS (the next tile is

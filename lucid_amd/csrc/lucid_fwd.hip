@@ -830,8 +830,9 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
   __shared__ __attribute__((aligned(16))) PfwdSmem<D, EXACT, F32> sm;
 
   const int id = blockIdx.x;
-  const int i2 = id / BH, bh = id - (id / BH) * BH;
-  if ((mass[bh] > kExactMass) != EXACT) return;  // the other instance solves this head
+  const InstanceHeads<EXACT> heads(mass, BH);
+  if (id >= (T / 128) * heads.n) return;
+  const int i2 = id / heads.n, bh = heads.head(id % heads.n);
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;
@@ -1245,14 +1246,20 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
   constexpr int WGR = 128 * NT;  // rows per workgroup
   const int nblk = (T + WGR - 1) / WGR;
   const int id = blockIdx.x;
-  const int bhq = id % BHq;
-  const int ib = nblk - 1 - id / BHq;
+  int bhq = id % BHq, ib = nblk - 1 - id / BHq;
+  // skip_fast: the fused forward has already written O and lse for the heads of the bf16
+  // chains; this launch covers the heads of the exact chains only
+  if (skip_fast) {
+    const int G = Hq / Hkv;
+    const InstanceHeads<true> heads(mass, BHq / G);
+    const int nq = heads.n * G;
+    if (id >= nblk * nq) return;
+    ib = nblk - 1 - id / nq;
+    bhq = heads.head(id % nq / G) * G + id % nq % G;
+  }
   const int b = bhq / Hq, hq = bhq - b * Hq;
   const int h = hq / (Hq / Hkv);
   const int bh = b * Hkv + h;
-  // skip_fast: the fused forward has already written O and lse for the heads of the bf16
-  // chains; this launch covers the heads of the exact chains only
-  if (skip_fast && !(mass[bh] > kExactMass)) return;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;
   const int r0 = ib * WGR;
@@ -1579,8 +1586,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void l
   static_assert(sizeof(bf16) * 128 * D <= sizeof(sm.u.fin.Rt), "block K^ rows must fit in R^T's bytes");
 
   const int id = blockIdx.x;
-  const int p = id / BH, bh = id - (id / BH) * BH;  // ids grow with p: every wait is on a lower id
-  if (mass[bh] > kExactMass) return;  // the exact instance of lucid_precond_fwd_kernel solves this head
+  const InstanceHeads<false> heads(mass, BH);  // the exact instance of lucid_precond_fwd_kernel solves the others
+  if (id >= (int)((T + 255) / 256) * heads.n) return;
+  const int p = id / heads.n, bh = heads.head(id % heads.n);  // ids grow with p: every wait is on a lower id
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;
@@ -1844,8 +1852,9 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_fused_fwd_
   __shared__ __attribute__((aligned(16))) FusedSmem<D> sm;
 
   const int id = blockIdx.x;
-  const int i2 = id / BH, bh = id - (id / BH) * BH;
-  if (mass[bh] > kExactMass) return;  // the exact chain and attention kernels cover this head
+  const InstanceHeads<false> heads(mass, BH);  // the exact chain and attention kernels cover the others
+  if (id >= (T / 128) * heads.n) return;
+  const int i2 = id / heads.n, bh = heads.head(id % heads.n);
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;
