@@ -155,6 +155,19 @@ int lucid_attn_bwd_f32(const float* dout, const int64_t* do_strides, const float
                        const int64_t* dk_strides, float* dv, const int64_t* dv_strides, void* bwd_ws, int B, int Hq,
                        int Hkv, int T, int D, float scale, void* stream);
 
+/* The same on operands of exactly D columns a row (D a multiple of 4): nothing of q, k, v or dout
+ * beyond column D - 1 is read, so rows need no padding to 64 or 128 columns, and their strides
+ * need only be multiples of 4 elements (pointers 16-byte aligned).  o, dq, dk and dv are padded
+ * rows as above, and the two forms' workspaces are interchangeable. */
+int lucid_attn_fwd_f32_rows(const float* q, const int64_t* q_strides, const float* k, const int64_t* k_strides,
+                       const float* v, const int64_t* v_strides, float* o, const int64_t* o_strides, float* vprime,
+                       float* lse, void* fwd_ws, int B, int Hq, int Hkv, int T, int D, float scale, float eps,
+                       void* stream);
+int lucid_attn_bwd_f32_rows(const float* dout, const int64_t* do_strides, const float* o, const int64_t* o_strides,
+                       const float* lse, const void* fwd_ws, float* dq, const int64_t* dq_strides, float* dk,
+                       const int64_t* dk_strides, float* dv, const int64_t* dv_strides, void* bwd_ws, int B, int Hq,
+                       int Hkv, int T, int D, float scale, void* stream);
+
 /* The two seams below (get_v_prime and eager_lucid_attention_forward) on fp32 tensors, head
  * dims up to 128: the same contracts as lucid_get_v_prime / lucid_precond_bwd and lucid_attn_vp_fwd /
  * lucid_attn_vp_bwd, with fp32 inputs (v_prime included) and fp32 outputs.  Workspaces:

@@ -49,6 +49,10 @@ _SIGS = {
                                 _int, _int, _int, _int, _int, _flt, _flt, _vp], _int),
         "lucid_attn_bwd_f32": ([_vp, _i64p, _vp, _i64p, _vp, _vp, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp,
                                 _int, _int, _int, _int, _int, _flt, _vp], _int),
+        "lucid_attn_fwd_f32_rows": ([_vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _vp, _vp,
+                                _int, _int, _int, _int, _int, _flt, _flt, _vp], _int),
+        "lucid_attn_bwd_f32_rows": ([_vp, _i64p, _vp, _i64p, _vp, _vp, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp,
+                                _int, _int, _int, _int, _int, _flt, _vp], _int),
         "lucid_v_prime_f32_workspace_bytes": ([_int] * 4, _sz),
         "lucid_get_v_prime_f32": ([_vp, _i64p, _vp, _i64p, _vp, _vp, _int, _int, _int, _int, _flt, _flt, _vp], _int),
         "lucid_precond_bwd_f32": ([_vp, _i64p, _vp, _vp, _i64p, _vp, _i64p, _vp, _int, _int, _int, _int, _flt, _vp],

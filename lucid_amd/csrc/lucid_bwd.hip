@@ -43,15 +43,18 @@ __global__ __launch_bounds__(256) void lucid_bwd_prep_kernel(const bf16* __restr
   const bf16* opp = o + b * os.b + hq * os.h + (int64_t)t * os.t;
   const bf16* olp = olo + ((int64_t)bhq * T + t) * D;
   float acc = 0.f;
-  if constexpr (F32) {  // fp32 dO and O themselves
-    const float* df = lo.dof + b * dos.b + hq * dos.h + (int64_t)t * dos.t + seg * SEG;
-    const float* of = lo.o + b * os.b + hq * os.h + (int64_t)t * os.t + seg * SEG;
+  if constexpr (F32) {  // fp32 dO and O themselves; a row's four threads read neighbouring 16 bytes
+    const float* df = lo.dof + b * dos.b + hq * dos.h + (int64_t)t * dos.t;
+    const float* of = lo.o + b * os.b + hq * os.h + (int64_t)t * os.t;
 #pragma unroll
-    for (int c = 0; c < SEG; c += 4) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(df + c);
-      const f32x4 x = *reinterpret_cast<const f32x4*>(of + c);
+    for (int i = 0; i < D; i += 16) {
+      const int c = i + 4 * seg;
+      if (c < lo.dc) {  // columns from lo.dc on: zero, not read
+        const f32x4 a = *reinterpret_cast<const f32x4*>(df + c);
+        const f32x4 x = *reinterpret_cast<const f32x4*>(of + c);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = fmaf(a[e], x[e], acc);
+        for (int e = 0; e < 4; ++e) acc = fmaf(a[e], x[e], acc);
+      }
     }
   } else {
 #pragma unroll

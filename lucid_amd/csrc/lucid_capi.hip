@@ -208,12 +208,13 @@ int check_ws(const char* name, const void* p) {
   return LUCID_OK;
 }
 
-int check_tensor(const char* name, const void* p, const int64_t* s) {
+int check_tensor(const char* name, const void* p, const int64_t* s, int mult = 8) {
   if (!p) return fail(std::string(name) + " is null");
   if (!s) return fail(std::string(name) + " strides are null");
   if (reinterpret_cast<uintptr_t>(p) % 16) return fail(std::string(name) + " must be 16-byte aligned");
   for (int i = 0; i < 3; ++i)
-    if (s[i] % 8) return fail(std::string(name) + " strides must be multiples of 8 elements");
+    if (s[i] % mult)
+      return fail(std::string(name) + " strides must be multiples of " + std::to_string(mult) + " elements");
   return LUCID_OK;
 }
 
@@ -605,20 +606,28 @@ lucid::Strides rows_strides(int H, int T, int D) {
   return lucid::Strides{(int64_t)H * T * D, (int64_t)T * D, (int64_t)D};
 }
 
+// Columns of an fp32 operand's rows that are read: the head dim up to the next 16 bytes (a row
+// is padded with zeros that far at least), all D where the call has no head dim (dn = 0).
 template <int D>
-int launch_split(const void* x, const int64_t* xs, int B, int H, int T, bf16* hi, bf16* lo, hipStream_t st,
+int read_cols(float dn) {
+  return dn > 0.f ? ((int)dn + 3) & ~3 : D;
+}
+
+template <int D>
+int launch_split(const void* x, const int64_t* xs, int B, int H, int T, float dn, bf16* hi, bf16* lo, hipStream_t st,
                  const float* center = nullptr) {
   LUCID_LAUNCH("lucid_split_kernel", lucid::lucid_split_kernel<D>, dim3(T / 64, B * H), st, (const float*)x,
-               S(xs), H, T, hi, lo, center);
+               S(xs), H, T, read_cols<D>(dn), hi, lo, center);
   return LUCID_OK;
 }
 
 // The attention's keys: K - (mean key of the head) as a bf16 pair in w.kch / w.kcl.
 template <int D>
-int launch_centered_keys(const void* k, const int64_t* ks, const FwdWs& w, int B, int Hkv, int T, hipStream_t st) {
+int launch_centered_keys(const void* k, const int64_t* ks, const FwdWs& w, int B, int Hkv, int T, float dn,
+                         hipStream_t st) {
   LUCID_LAUNCH("lucid_key_mean_kernel", lucid::lucid_key_mean_kernel<D>, dim3(B * Hkv), st, (const float*)k,
-               S(ks), Hkv, T, w.kmean);
-  return launch_split<D>(k, ks, B, Hkv, T, w.kch, w.kcl, st, w.kmean);
+               S(ks), Hkv, T, read_cols<D>(dn), w.kmean);
+  return launch_split<D>(k, ks, B, Hkv, T, dn, w.kch, w.kcl, st, w.kmean);
 }
 
 // V' = P^-1 V from fp32 K and V (K split into w.kh / w.kl).
@@ -628,11 +637,12 @@ int launch_precond_fwd_f32(const void* k, const int64_t* ks, const void* v, cons
                            hipStream_t st) {
   const int BH = B * Hkv;
   const lucid::Strides ck = rows_strides(Hkv, T, D);
-  if (int rc = launch_split<D>(k, ks, B, Hkv, T, w.kh, w.kl, st)) return rc;
+  if (int rc = launch_split<D>(k, ks, B, Hkv, T, dn, w.kh, w.kl, st)) return rc;
   lucid::Lo lo{};
   lo.k = w.kl;
   lo.kt = w.ktl;
   lo.v = static_cast<const float*>(v);
+  lo.dc = read_cols<D>(dn);
   LUCID_LAUNCH("lucid_prep_f32_kernel", (lucid::lucid_prep_kernel<D, true>), dim3(T / 64, BH), st, w.kh, ck, Hkv,
                T, eps, dn, scale, w.rinv, w.kt, w.pinv, w.counters, w.mass, kForceExact, lo, w.ktl, nullptr);
   LUCID_LAUNCH("lucid_zx_f32_kernel", (lucid::lucid_zx_kernel<D, true>), dim3(T / 128, BH), st, w.kh, ck, Hkv, T,
@@ -653,7 +663,7 @@ template <int D>
 int launch_attn_fwd_f32(const void* q, const int64_t* qs, void* o, const int64_t* os, float* lse, const FwdWs& w,
                         int B, int Hq, int Hkv, int T, float scale, float dn, hipStream_t st) {
   const int BHq = B * Hq;
-  if (int rc = launch_split<D>(q, qs, B, Hq, T, w.qh, w.ql, st)) return rc;
+  if (int rc = launch_split<D>(q, qs, B, Hq, T, dn, w.qh, w.ql, st)) return rc;
   lucid::Lo lo{};
   lo.q = w.ql;
   lo.k = w.kcl;
@@ -688,7 +698,7 @@ int launch_fwd_f32(const void* q, const int64_t* qs, const void* k, const int64_
                    const int64_t* vs, void* o, const int64_t* os, float* vprime, float* lse, const FwdWs& w, int B,
                    int Hq, int Hkv, int T, float scale, float eps, float dn, hipStream_t st) {
   if (int rc = launch_precond_fwd_f32<D>(k, ks, v, vs, vprime, w, B, Hkv, T, scale, eps, dn, st)) return rc;
-  if (int rc = launch_centered_keys<D>(k, ks, w, B, Hkv, T, st)) return rc;
+  if (int rc = launch_centered_keys<D>(k, ks, w, B, Hkv, T, dn, st)) return rc;
   return launch_attn_fwd_f32<D>(q, qs, o, os, lse, w, B, Hq, Hkv, T, scale, dn, st);
 }
 
@@ -701,13 +711,14 @@ int launch_attn_bwd_f32(const void* dout, const int64_t* dos, const void* o, con
                         float scale, float dn, hipStream_t st) {
   const int BH = B * Hkv, BHq = B * Hq;
   const lucid::Strides cq = rows_strides(Hq, T, D), ck = rows_strides(Hkv, T, D);
-  if (int rc = launch_split<D>(dout, dos, B, Hq, T, w.doh, w.dol, st)) return rc;
+  if (int rc = launch_split<D>(dout, dos, B, Hq, T, dn, w.doh, w.dol, st)) return rc;
   lucid::Lo lo{};
   lo.q = f.ql;
   lo.k = f.kcl;
   lo.dout = w.dol;
   lo.o = static_cast<const float*>(o);
   lo.dof = static_cast<const float*>(dout);
+  lo.dc = read_cols<D>(dn);
   // delta reads fp32 dO and O with their own strides (the bf16 operands are unused)
   LUCID_LAUNCH("lucid_bwd_prep_f32_kernel", (lucid::lucid_bwd_prep_kernel<D, true>), dim3(T / 64, BHq), st,
                (const bf16*)dout, S(dos), (const bf16*)o, S(os), f.olo, f.mass, Hq, Hkv, T, w.delta, w.counters, BH,
@@ -802,7 +813,7 @@ int launch_attn_vp_fwd_f32(const void* q, const int64_t* qs, const void* k, cons
                            const int64_t* vs, void* o, const int64_t* os, float* lse, const FwdWs& w, int B, int Hq,
                            int Hkv, int T, float eps, float scale, float dn, hipStream_t st) {
   const int BH = B * Hkv;
-  if (int rc = launch_centered_keys<D>(k, ks, w, B, Hkv, T, st)) return rc;
+  if (int rc = launch_centered_keys<D>(k, ks, w, B, Hkv, T, dn, st)) return rc;
   LUCID_LAUNCH("lucid_vp_layout_f32_kernel", (lucid::lucid_vp_layout_kernel<D, float, true>), dim3(T / 64, BH), st,
                w.kch, rows_strides(Hkv, T, D), (const float*)vp, S(vs), Hkv, T, eps, dn, w.rinv, w.vpb, w.vpt, w.mass,
                kForceExact, w.vpbl, w.vptl);
@@ -1094,6 +1105,47 @@ int precond_bwd_f32_impl(const float* dvprime, const int64_t* dvprime_strides, c
                                      scale, dn, static_cast<hipStream_t>(stream));
 }
 
+// mult: what the input strides must be multiples of (8 elements; 4 where only whole rows of the
+// head dim are read)
+int attn_fwd_f32_impl(int mult, const float* q, const int64_t* q_strides, const float* k, const int64_t* k_strides,
+                       const float* v, const int64_t* v_strides, float* o, const int64_t* o_strides, float* vprime,
+                       float* lse, void* fwd_ws, int B, int Hq, int Hkv, int T, int D, float scale, float eps,
+                       void* stream) {
+  g_last_error.clear();
+  if (int rc = check_dims(B, Hq, Hkv, T, D)) return rc;
+  if (int rc = check_tensor("q", q, q_strides, mult)) return rc;
+  if (int rc = check_tensor("k", k, k_strides, mult)) return rc;
+  if (int rc = check_tensor("v", v, v_strides, mult)) return rc;
+  if (int rc = check_tensor("o", o, o_strides)) return rc;
+  if (!vprime || !lse || !fwd_ws) return fail("vprime, lse and fwd_ws must be non-null");
+  if (int rc = check_ws("fwd_ws", fwd_ws)) return rc;
+  if (int rc = chain_check()) return rc;
+  const FwdWs w = carve_fwd(fwd_ws, B, Hq, Hkv, T, D, true);
+  return (padded_dim(D) == 64 ? launch_fwd_f32<64> : launch_fwd_f32<128>)(q, q_strides, k, k_strides, v, v_strides, o, o_strides, vprime, lse, w, B, Hq, Hkv, T,
+                        scale, eps, (float)D, static_cast<hipStream_t>(stream));
+}
+
+int attn_bwd_f32_impl(int mult, const float* dout, const int64_t* do_strides, const float* o, const int64_t* o_strides,
+                       const float* lse, const void* fwd_ws, float* dq, const int64_t* dq_strides, float* dk,
+                       const int64_t* dk_strides, float* dv, const int64_t* dv_strides, void* bwd_ws, int B, int Hq,
+                       int Hkv, int T, int D, float scale, void* stream) {
+  g_last_error.clear();
+  if (int rc = check_dims(B, Hq, Hkv, T, D)) return rc;
+  if (int rc = check_tensor("dout", dout, do_strides, mult)) return rc;
+  if (int rc = check_tensor("o", o, o_strides)) return rc;
+  if (int rc = check_tensor("dq", dq, dq_strides)) return rc;
+  if (int rc = check_tensor("dk", dk, dk_strides)) return rc;
+  if (int rc = check_tensor("dv", dv, dv_strides)) return rc;
+  if (!lse || !fwd_ws || !bwd_ws) return fail("lse, fwd_ws and bwd_ws must be non-null");
+  if (int rc = check_ws("fwd_ws", fwd_ws)) return rc;
+  if (int rc = check_ws("bwd_ws", bwd_ws)) return rc;
+  if (int rc = chain_check()) return rc;
+  const FwdWs f = carve_fwd(const_cast<void*>(fwd_ws), B, Hq, Hkv, T, D, true);
+  const BwdWs w = carve_bwd(bwd_ws, B, Hq, Hkv, T, D, true);
+  return (padded_dim(D) == 64 ? launch_bwd_f32<64> : launch_bwd_f32<128>)(dout, do_strides, o, o_strides, lse, f, dq, dq_strides, dk, dk_strides, dv, dv_strides, w,
+                        B, Hq, Hkv, T, scale, (float)D, static_cast<hipStream_t>(stream));
+}
+
 }  // namespace
 
 extern "C" {
@@ -1294,39 +1346,34 @@ int lucid_attn_fwd_f32(const float* q, const int64_t* q_strides, const float* k,
                        const float* v, const int64_t* v_strides, float* o, const int64_t* o_strides, float* vprime,
                        float* lse, void* fwd_ws, int B, int Hq, int Hkv, int T, int D, float scale, float eps,
                        void* stream) {
-  g_last_error.clear();
-  if (int rc = check_dims(B, Hq, Hkv, T, D)) return rc;
-  if (int rc = check_tensor("q", q, q_strides)) return rc;
-  if (int rc = check_tensor("k", k, k_strides)) return rc;
-  if (int rc = check_tensor("v", v, v_strides)) return rc;
-  if (int rc = check_tensor("o", o, o_strides)) return rc;
-  if (!vprime || !lse || !fwd_ws) return fail("vprime, lse and fwd_ws must be non-null");
-  if (int rc = check_ws("fwd_ws", fwd_ws)) return rc;
-  if (int rc = chain_check()) return rc;
-  const FwdWs w = carve_fwd(fwd_ws, B, Hq, Hkv, T, D, true);
-  return (padded_dim(D) == 64 ? launch_fwd_f32<64> : launch_fwd_f32<128>)(q, q_strides, k, k_strides, v, v_strides, o, o_strides, vprime, lse, w, B, Hq, Hkv, T,
-                        scale, eps, (float)D, static_cast<hipStream_t>(stream));
+  return attn_fwd_f32_impl(8, q, q_strides, k, k_strides, v, v_strides, o, o_strides, vprime, lse, fwd_ws, B, Hq, Hkv, T,
+                           D, scale, eps, stream);
 }
 
 int lucid_attn_bwd_f32(const float* dout, const int64_t* do_strides, const float* o, const int64_t* o_strides,
                        const float* lse, const void* fwd_ws, float* dq, const int64_t* dq_strides, float* dk,
                        const int64_t* dk_strides, float* dv, const int64_t* dv_strides, void* bwd_ws, int B, int Hq,
                        int Hkv, int T, int D, float scale, void* stream) {
-  g_last_error.clear();
-  if (int rc = check_dims(B, Hq, Hkv, T, D)) return rc;
-  if (int rc = check_tensor("dout", dout, do_strides)) return rc;
-  if (int rc = check_tensor("o", o, o_strides)) return rc;
-  if (int rc = check_tensor("dq", dq, dq_strides)) return rc;
-  if (int rc = check_tensor("dk", dk, dk_strides)) return rc;
-  if (int rc = check_tensor("dv", dv, dv_strides)) return rc;
-  if (!lse || !fwd_ws || !bwd_ws) return fail("lse, fwd_ws and bwd_ws must be non-null");
-  if (int rc = check_ws("fwd_ws", fwd_ws)) return rc;
-  if (int rc = check_ws("bwd_ws", bwd_ws)) return rc;
-  if (int rc = chain_check()) return rc;
-  const FwdWs f = carve_fwd(const_cast<void*>(fwd_ws), B, Hq, Hkv, T, D, true);
-  const BwdWs w = carve_bwd(bwd_ws, B, Hq, Hkv, T, D, true);
-  return (padded_dim(D) == 64 ? launch_bwd_f32<64> : launch_bwd_f32<128>)(dout, do_strides, o, o_strides, lse, f, dq, dq_strides, dk, dk_strides, dv, dv_strides, w,
-                        B, Hq, Hkv, T, scale, (float)D, static_cast<hipStream_t>(stream));
+  return attn_bwd_f32_impl(8, dout, do_strides, o, o_strides, lse, fwd_ws, dq, dq_strides, dk, dk_strides, dv,
+                           dv_strides, bwd_ws, B, Hq, Hkv, T, D, scale, stream);
+}
+
+int lucid_attn_fwd_f32_rows(const float* q, const int64_t* q_strides, const float* k, const int64_t* k_strides,
+                       const float* v, const int64_t* v_strides, float* o, const int64_t* o_strides, float* vprime,
+                       float* lse, void* fwd_ws, int B, int Hq, int Hkv, int T, int D, float scale, float eps,
+                       void* stream) {
+  if (D % 4) return fail("lucid_attn_fwd_f32_rows: head dim must be a multiple of 4");
+  return attn_fwd_f32_impl(4, q, q_strides, k, k_strides, v, v_strides, o, o_strides, vprime, lse, fwd_ws, B, Hq, Hkv, T,
+                           D, scale, eps, stream);
+}
+
+int lucid_attn_bwd_f32_rows(const float* dout, const int64_t* do_strides, const float* o, const int64_t* o_strides,
+                       const float* lse, const void* fwd_ws, float* dq, const int64_t* dq_strides, float* dk,
+                       const int64_t* dk_strides, float* dv, const int64_t* dv_strides, void* bwd_ws, int B, int Hq,
+                       int Hkv, int T, int D, float scale, void* stream) {
+  if (D % 4) return fail("lucid_attn_bwd_f32_rows: head dim must be a multiple of 4");
+  return attn_bwd_f32_impl(4, dout, do_strides, o, o_strides, lse, fwd_ws, dq, dq_strides, dk, dk_strides, dv,
+                           dv_strides, bwd_ws, B, Hq, Hkv, T, D, scale, stream);
 }
 
 size_t lucid_v_prime_f32_workspace_bytes(int B, int Hkv, int T, int D) {

@@ -83,6 +83,7 @@ struct Lo {
   const float* v;    // fp32 V [B, H, T, D], strides vs (the chain's right-hand side)
   const float* o;    // fp32 O, strides as the kernel's o (delta of the backward)
   const float* dof;  // fp32 dO, strides as the kernel's dout (delta of the backward)
+  int dc;            // columns read of v's, o's and dof's rows (a multiple of 4; zero from there on)
 };
 
 // bf16 of the residual x - hi for D-layout values e = 8h .. 8h+7 (hi = pack_b(x, h)):

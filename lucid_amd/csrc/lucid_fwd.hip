@@ -258,44 +258,45 @@ __global__ __launch_bounds__(256) void lucid_rows_out_kernel(const float* __rest
   }
 }
 
-// fp32 inputs: a strided fp32 [B][H][T][D] tensor to the bf16 pair the MFMA operands are
-// built from, hi = bf16(x) and lo = bf16(x - hi) (x = hi + lo to ~2^-16 relative), both
-// written as contiguous [BH][T][D] rows.  center (fp32 [BH][D], or null): x - center[bh]
-// is split instead.  grid (T/64, B*H)
+// fp32 inputs: the first dc columns (a multiple of 4) of a strided fp32 [B][H][T] tensor's rows
+// to the bf16 pair the MFMA operands are built from, hi = bf16(x) and lo = bf16(x - hi)
+// (x = hi + lo to ~2^-16 relative), both written as contiguous [BH][T][D] rows with zeros from
+// column dc on.  center (fp32 [BH][D], or null): x - center[bh] is split instead.  Memory
+// bound: D / 8 neighbouring threads take a row, 16 bytes of each plane per thread (B8 Hq32
+// Hkv4 T2048 d68: the four splits of a training pass 160 us; with 32 columns per thread, of
+// rows padded to 128, 398).  grid (T/64, B*H)
 template <int D>
 __global__ __launch_bounds__(256) void lucid_split_kernel(const float* __restrict__ src, Strides ss, int H, int T,
-                                                          bf16* __restrict__ hi, bf16* __restrict__ lo,
+                                                          int dc, bf16* __restrict__ hi, bf16* __restrict__ lo,
                                                           const float* __restrict__ center) {
-  constexpr int SEG = D / 4;
+  constexpr int CPR = D / 8, RP = 256 / CPR;  // 8-column chunks per row, rows per pass
   const int bh = blockIdx.y, b = bh / H, h = bh - b * H;
-  const int row = threadIdx.x >> 2, seg = threadIdx.x & 3;
-  const int t = blockIdx.x * 64 + row;
-  const float* s = src + b * ss.b + h * ss.h + (int64_t)t * ss.t + seg * SEG;
-  const float* cen = center ? center + (int64_t)bh * D + seg * SEG : nullptr;
-  const int64_t off = ((int64_t)bh * T + t) * D + seg * SEG;
+  const int row = threadIdx.x / CPR, c = 8 * (threadIdx.x % CPR);
+  const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+  f32x4 c0 = z, c1 = z;
+  if (center) {
+    c0 = *reinterpret_cast<const f32x4*>(center + (int64_t)bh * D + c);
+    c1 = *reinterpret_cast<const f32x4*>(center + (int64_t)bh * D + c + 4);
+  }
+  const float* s = src + b * ss.b + h * ss.h + c;
 #pragma unroll
-  for (int c = 0; c < SEG; c += 8) {
-    f32x4 x0 = *reinterpret_cast<const f32x4*>(s + c);
-    f32x4 x1 = *reinterpret_cast<const f32x4*>(s + c + 4);
-    if (cen) {
-      const f32x4 c0 = *reinterpret_cast<const f32x4*>(cen + c);
-      const f32x4 c1 = *reinterpret_cast<const f32x4*>(cen + c + 4);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        x0[u] -= c0[u];
-        x1[u] -= c1[u];
-      }
-    }
-    bf16x8 a, r;
+  for (int r = 0; r < 64; r += RP) {
+    const int t = blockIdx.x * 64 + r + row;
+    f32x4 x0 = z, x1 = z;
+    if (c < dc) x0 = *reinterpret_cast<const f32x4*>(s + (int64_t)t * ss.t);
+    if (c + 4 < dc) x1 = *reinterpret_cast<const f32x4*>(s + (int64_t)t * ss.t + 4);
+    bf16x8 a, q;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      a[u] = (bf16)x0[u];
-      a[u + 4] = (bf16)x1[u];
-      r[u] = (bf16)(x0[u] - (float)a[u]);
-      r[u + 4] = (bf16)(x1[u] - (float)a[u + 4]);
+      const float y0 = x0[u] - c0[u], y1 = x1[u] - c1[u];
+      a[u] = (bf16)y0;
+      a[u + 4] = (bf16)y1;
+      q[u] = (bf16)(y0 - (float)a[u]);
+      q[u + 4] = (bf16)(y1 - (float)a[u + 4]);
     }
-    *reinterpret_cast<bf16x8*>(hi + off + c) = a;
-    *reinterpret_cast<bf16x8*>(lo + off + c) = r;
+    const int64_t off = ((int64_t)bh * T + t) * D + c;
+    *reinterpret_cast<bf16x8*>(hi + off) = a;
+    *reinterpret_cast<bf16x8*>(lo + off) = q;
   }
 }
 
@@ -308,13 +309,13 @@ __global__ __launch_bounds__(256) void lucid_split_kernel(const float* __restric
 // 256 / (D/4) row phases x D/4 four-column groups, fixed summation order.  grid (B*H)
 template <int D>
 __global__ __launch_bounds__(256) void lucid_key_mean_kernel(const float* __restrict__ k, Strides ks, int H, int T,
-                                                             float* __restrict__ mean) {
+                                                             int dc, float* __restrict__ mean) {
   constexpr int CG = D / 4, PH = 256 / CG;
   static_assert(CG * PH == 256, "four-column groups x row phases = 256 threads");
   __shared__ f32x4 part[PH][CG];
   const int bh = blockIdx.x, b = bh / H, h = bh - b * H;
   const int ph = threadIdx.x / CG, c4 = threadIdx.x % CG;
-  const float* kp = k + b * ks.b + h * ks.h + 4 * c4;
+  const float* kp = k + b * ks.b + h * ks.h + min(4 * c4, dc - 4);  // columns from dc on are not read (zero below)
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
   for (int t = ph; t < T; t += PH) {
@@ -330,7 +331,7 @@ __global__ __launch_bounds__(256) void lucid_key_mean_kernel(const float* __rest
 #pragma unroll
       for (int u = 0; u < 4; ++u) tot[u] += part[r][c4][u];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) tot[u] /= (float)T;
+    for (int u = 0; u < 4; ++u) tot[u] = 4 * c4 < dc ? tot[u] / (float)T : 0.f;
     *reinterpret_cast<f32x4*>(mean + (int64_t)bh * D + 4 * c4) = tot;
   }
 }
@@ -883,7 +884,9 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
       for (int qd = 0; qd < 4; ++qd) {
         float vv[4];
         if constexpr (F32) {  // the fp32 right-hand side itself
-          const f32x4 x = *reinterpret_cast<const f32x4*>(lo.v + b * vs.b + h * vs.h + roff + t * 32 + 8 * qd + 4 * g);
+          const int d0 = t * 32 + 8 * qd + 4 * g;  // columns from lo.dc on: zero, not read
+          f32x4 x = {0.f, 0.f, 0.f, 0.f};
+          if (d0 < lo.dc) x = *reinterpret_cast<const f32x4*>(lo.v + b * vs.b + h * vs.h + roff + d0);
 #pragma unroll
           for (int u = 0; u < 4; ++u) vv[u] = x[u];
         } else {

@@ -116,16 +116,26 @@ def _fwd(q, k, v, scale, eps, dn):
     return o, vprime, lse, ws
 
 
+def _whole_rows(t: torch.Tensor) -> bool:
+    """Whether the kernels can read fp32 ``t`` [.., d] without padding its rows to 64 or 128 columns:
+    d a multiple of 4 short of those, unit stride, 4-element strides, 16-byte aligned."""
+    d = t.shape[-1]
+    return (t.dtype == torch.float32 and d % 4 == 0 and d != _padded_dim(d) and t.stride(-1) == 1
+            and not any(s % 4 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0)
+
+
 def _fwd_f32(q, k, v, scale, eps, dn):
+    """Operands padded to 64 or 128 columns, or whole rows of dn columns (_whole_rows)."""
     lib = _lib.load()
-    B, Hq, T, D = q.shape
+    B, Hq, T, _ = q.shape
+    D = _padded_dim(dn)
     Hkv = k.shape[1]
     dev = q.device
     o = torch.empty(B, T, Hq, D, dtype=torch.float32, device=dev)
     vprime = torch.empty(B, Hkv, T, D, dtype=torch.float32, device=dev)
     lse = torch.empty(B, Hq, T, dtype=torch.float32, device=dev)
     ws = torch.empty(lib.lucid_fwd_f32_workspace_bytes(B, Hq, Hkv, T, dn), dtype=torch.uint8, device=dev)
-    rc = lib.lucid_attn_fwd_f32(
+    rc = (lib.lucid_attn_fwd_f32 if q.shape[3] == D else lib.lucid_attn_fwd_f32_rows)(
         _lib.ptr(q), _lib.strides3(q, (0, 1, 2)), _lib.ptr(k), _lib.strides3(k, (0, 1, 2)),
         _lib.ptr(v), _lib.strides3(v, (0, 1, 2)), _lib.ptr(o), _lib.strides3(o, (0, 2, 1)),
         _lib.ptr(vprime), _lib.ptr(lse), _lib.ptr(ws), B, Hq, Hkv, T, dn, float(scale), float(eps),
@@ -147,16 +157,15 @@ def _time_major(x: torch.Tensor) -> bool:
     return x.dim() == 4 and x.shape[1] > 1 and x.stride(1) < x.stride(2)
 
 
-def _bwd_f32(do, q, k, o, lse, ws, scale, dn, layouts=(False, False, False)):
+def _bwd_f32(do, Hkv, o, lse, ws, scale, dn, layouts=(False, False, False)):
     lib = _lib.load()
-    B, Hq, T, D = q.shape
-    Hkv = k.shape[1]
-    dev = q.device
+    B, T, Hq, D = o.shape
+    dev = o.device
     dq = _grad_buf(B, Hq, T, D, torch.float32, dev, layouts[0])
     dk = _grad_buf(B, Hkv, T, D, torch.float32, dev, layouts[1])
     dv = _grad_buf(B, Hkv, T, D, torch.float32, dev, layouts[2])
     bws = torch.empty(lib.lucid_bwd_f32_workspace_bytes(B, Hq, Hkv, T, dn), dtype=torch.uint8, device=dev)
-    rc = lib.lucid_attn_bwd_f32(
+    rc = (lib.lucid_attn_bwd_f32 if do.shape[3] == D else lib.lucid_attn_bwd_f32_rows)(
         _lib.ptr(do), _lib.strides3(do, (0, 2, 1)), _lib.ptr(o), _lib.strides3(o, (0, 2, 1)),
         _lib.ptr(lse), _lib.ptr(ws), _lib.ptr(dq), _lib.strides3(dq, (0, 1, 2)),
         _lib.ptr(dk), _lib.strides3(dk, (0, 1, 2)), _lib.ptr(dv), _lib.strides3(dv, (0, 1, 2)),
@@ -213,13 +222,19 @@ class LucidAttentionFunction(torch.autograd.Function):
             return (q.new_empty(B, t, Hq, D),
                     torch.empty(B, k.shape[1], t, D, dtype=torch.float32, device=q.device))
         tp, dp = _padded_len(t), _padded_dim(dn)
-        if t != tp or dn != dp:
+        ctx.f32 = q.dtype == torch.float32
+        # fp32 operands are split into padded bf16 pairs anyway, so whole 128-row blocks of rows of
+        # whole 16-byte chunks are read as they are (a training pass of B8 Hq32 Hkv4 T2048 d68
+        # pads for 199 us otherwise and reads the padding for about 150)
+        if t == tp and _whole_rows(q) and _whole_rows(k) and _whole_rows(v):
+            qp, kp, vp_ = q, k, v
+        elif t != tp or dn != dp:
             qp, kp, vp_ = _pad_rows((q, k, v), tp, dp)
         else:
             qp, kp, vp_ = _prep(q, tp), _prep(k, tp), _prep(v, tp)
-        ctx.f32 = q.dtype == torch.float32
         o, vprime, lse, ws = (_fwd_f32 if ctx.f32 else _fwd)(qp, kp, vp_, scale, eps, dn)
-        ctx.save_for_backward(qp, kp, o, lse, ws)
+        # fp32: the workspace holds the split operands
+        ctx.save_for_backward(*(() if ctx.f32 else (qp, kp)), o, lse, ws)
         ctx.scale, ctx.eps, ctx.t, ctx.dn = scale, eps, t, dn
         # the gradients are written in the memory order of the operands they belong to
         ctx.layouts = (_time_major(q), _time_major(k), _time_major(v))
@@ -236,13 +251,16 @@ class LucidAttentionFunction(torch.autograd.Function):
         if ctx.empty:
             return (do.new_zeros(ctx.shapes[0]), do.new_zeros(ctx.shapes[1]), do.new_zeros(ctx.shapes[1]),
                     None, None, None)
-        qp, kp, o, lse, ws = ctx.saved_tensors
-        t, tp, dn, dp = ctx.t, qp.shape[2], ctx.dn, qp.shape[3]
-        do = _prep_do(do, torch.float32 if ctx.f32 else torch.bfloat16, tp, dp)
+        *operands, o, lse, ws = ctx.saved_tensors
+        t, dn = ctx.t, ctx.dn
+        _, tp, _, dp = o.shape
         if ctx.f32:
-            dq, dk, dv = _bwd_f32(do, qp, kp, o, lse, ws, ctx.scale, ctx.dn, ctx.layouts)
+            if t != tp or not _whole_rows(do):
+                do = _prep_do(do, torch.float32, tp, dp)
+            dq, dk, dv = _bwd_f32(do, ctx.shapes[1][1], o, lse, ws, ctx.scale, dn, ctx.layouts)
         else:
-            dq, dk, dv = _bwd(do, qp, kp, o, lse, ws, ctx.scale, ctx.eps, ctx.dn, ctx.layouts)
+            do = _prep_do(do, torch.bfloat16, tp, dp)
+            dq, dk, dv = _bwd(do, *operands, o, lse, ws, ctx.scale, ctx.eps, dn, ctx.layouts)
         return dq[:, :, :t, :dn], dk[:, :, :t, :dn], dv[:, :, :t, :dn], None, None, None
 
 
