@@ -82,8 +82,8 @@ __global__ __launch_bounds__(256) void lucid_bwd_prep_kernel(const bf16* __restr
 }
 
 // ---------------------------------------------------------------------------
-// Column sweep for the attention part.  Workgroup = 128 keys of one kv head,
-// wave w owns keys 32w..32w+31 (one n-tile, lane <-> key j); sweeps the G query
+// Column sweep for the attention part.  Workgroup = 128 keys of one kv head (256, NW = 8
+// waves, in the bf16 instance at head dim 128), wave w owns keys 32w..32w+31 (one n-tile, lane <-> key j); sweeps the G query
 // heads of the group and every 64-row query tile at or below the diagonal.
 // Each query tile (Q and dO rows, lse2, delta) is staged once per workgroup in
 // LDS by direct global->LDS loads (three buffers, two tiles ahead, swizzled);
@@ -91,7 +91,12 @@ __global__ __launch_bounds__(256) void lucid_bwd_prep_kernel(const bf16* __restr
 //   S[i][j] = Q_i . K_j, P = exp2(c S - lse2_i)
 //   dV'^T[d][j] += dO^T[d][i] P[i][j];  dP[i][j] = dO_i . V'_j
 //   dS = P (dP - delta_i);  dK^T[d][j] += Q^T[d][i] dS[i][j]
-// At d = 64 two workgroups share a CU (<= 256 registers per lane).
+// At d = 64 two workgroups share a CU (<= 256 registers per lane).  At d = 128 the staged tiles
+// leave room for one workgroup, so eight waves share them, two per SIMD: every operand is read
+// from LDS twice per wave (rows and transposed), 64 KB per 32-row step and 64 keys against
+// 1024 cycles of products, and the second wave fills the other's waits.  The 256 registers
+// hold the accumulators and K, V' operands (192); at most four row operands are in flight.
+// B1 Hq32 Hkv8 T8192 d128: 1544 us with four waves of up to 512 registers, 1400 this way.
 // ---------------------------------------------------------------------------
 template <int D, bool F32 = false>
 struct DkdvSmem {
@@ -108,8 +113,8 @@ struct DkdvSmem {
 // three MFMAs (S = Q.K four, lo*lo included); P and dS are split into hi and lo.
 // DA: the head-dim columns that can be nonzero (zero-padded rows of a smaller head dim; the
 // products skip the k-steps and tiles that would only meet zero columns, whose outputs stay 0)
-template <int D, bool F32 = false, int DA = D>
-__global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid_attn_bwd_dkdv_kernel(
+template <int D, bool F32 = false, int DA = D, int NW = 4>
+__global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF(NW == 8 || (D == 64 && !F32)) void lucid_attn_bwd_dkdv_kernel(
     const bf16* __restrict__ q, Strides qs, const bf16* __restrict__ k, Strides ks, const bf16* __restrict__ vpb,
     const bf16* __restrict__ dout, Strides dos, const bf16* __restrict__ seeds, float* __restrict__ dvp, float* __restrict__ dka, int Hq, int Hkv, int T, int BH, float scale, Lo lo,
     const bf16* __restrict__ vpbl, int nsplit, float* __restrict__ part) {
@@ -119,7 +124,8 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
   constexpr int NDT_A = (DA + 31) / 32, NKS_A = DA / 16;
   static_assert(DA % 16 == 0 && DA <= D, "active head dim");
   // newest vector-memory ops of a step, per wave
-  constexpr int STAGE_OPS = (F32 ? 4 : 2) * (64 * (D / 8) / 256);
+  constexpr int NTHR = 64 * NW, COLS = 32 * NW;  // keys per workgroup
+  constexpr int STAGE_OPS = (F32 ? 4 : 2) * (64 * (D / 8) / NTHR);
   __shared__ __attribute__((aligned(16))) DkdvSmem<D, F32> sm;
   constexpr int NB = stage_bufs(D, F32);
   const int id = blockIdx.x;
@@ -129,8 +135,8 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
   const int G = Hq / Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 5, l32 = lane & 31;
-  const int jw = jb * 128 + w * 32;  // first key of this wave
-  const int jrow = jw + l32;
+  const int jw = jb * COLS + w * 32;  // first key of this wave
+  const int jrow = NW == 4 ? jw + l32 : min(jw + l32, T - 1);  // waves behind the last key only stage
   const bf16* kh = k + b * ks.b + h * ks.h;
   const float c = scale * LOG2E_F;
 
@@ -151,7 +157,7 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
     adk[t] = zero16();
   }
   const int nt64 = T / 64;
-  const int it_first = jb * 2;            // first query tile any wave needs
+  const int it_first = jb * (COLS / 64);            // first query tile any wave needs
   const int ntile = nt64 - it_first;      // query tiles per query head
   // step s of a column block: query head s / ntile, tile it_first + s % ntile; this
   // workgroup's share is the steps s0 .. s0 + nsteps - 1
@@ -159,21 +165,21 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
   const int nsteps = (int)((int64_t)G * ntile * (sp + 1) / nsplit) - s0;
   const int it_w = jw / 64;               // this wave's diagonal tile
   const int kloc = jw - it_w * 64 + l32;  // this lane's key inside its diagonal tile
-  int plan_q[64 * (D / 8) / 256], plan_o[64 * (D / 8) / 256];
+  int plan_q[64 * (D / 8) / NTHR], plan_o[64 * (D / 8) / NTHR];
   // head dim 64: the conflict-free swizzle (every staged tile is read twice per wave, in rows
   // and transposed, so the LDS bandwidth matters here)
   constexpr int SW = D == 64 ? 1 : 0;
-  dma_plan<64, D / 8, 256, SW>(qs.t, plan_q);
-  dma_plan<64, D / 8, 256, SW>(dos.t, plan_o);
+  dma_plan<64, D / 8, NTHR, SW>(qs.t, plan_q);
+  dma_plan<64, D / 8, NTHR, SW>(dos.t, plan_o);
   auto stage = [&](int s) {
     const int gi = (s0 + s) / ntile, it = it_first + s0 + s - gi * ntile, buf = s % NB;
     const int hq = h * G + gi, bhq = b * Hq + hq, i0 = it * 64;
     if (w < 2) dma_1k(seeds + ((int64_t)bhq * T + i0 + 32 * w) * 16, &sm.seed[buf][32 * w][0]);  // 2 KB of seed rows
-    dma_stage<64, D / 8>(plan_q, q + b * qs.b + hq * qs.h + (int64_t)i0 * qs.t, sm.q[buf]);
-    dma_stage<64, D / 8>(plan_o, dout + b * dos.b + hq * dos.h + (int64_t)i0 * dos.t, sm.dO[buf]);
+    dma_stage<64, D / 8, NTHR>(plan_q, q + b * qs.b + hq * qs.h + (int64_t)i0 * qs.t, sm.q[buf]);
+    dma_stage<64, D / 8, NTHR>(plan_o, dout + b * dos.b + hq * dos.h + (int64_t)i0 * dos.t, sm.dO[buf]);
     if constexpr (F32) {
-      dma_stage<64, D / 8>(plan_q, lo.q + b * qs.b + hq * qs.h + (int64_t)i0 * qs.t, sm.ql[buf]);
-      dma_stage<64, D / 8>(plan_o, lo.dout + b * dos.b + hq * dos.h + (int64_t)i0 * dos.t, sm.dOl[buf]);
+      dma_stage<64, D / 8, NTHR>(plan_q, lo.q + b * qs.b + hq * qs.h + (int64_t)i0 * qs.t, sm.ql[buf]);
+      dma_stage<64, D / 8, NTHR>(plan_o, lo.dout + b * dos.b + hq * dos.h + (int64_t)i0 * dos.t, sm.dOl[buf]);
     }
   };
   if (nsteps > 0) stage(0);
@@ -184,18 +190,24 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
     dma_wait();
   }
   __syncthreads();
-  int tro[NDT], tro2[NDT], rdo[NKS];  // lane offsets of the transposing (two loads) and the row reads
+  // lane offsets of the transposing (two loads) and the row reads; eight waves: the first of
+  // each only, the others differ from it in chunk bits (registers are what limits them)
+  constexpr bool XO = NW == 8;
+  int tro_[XO ? 1 : NDT], tro2_[XO ? 1 : NDT], rdo_[XO ? 1 : NKS];
 #pragma unroll
-  for (int t = 0; t < NDT; ++t) lds_tr_lane_offs<D / 8, SW>(t * 32, tro[t], tro2[t]);
+  for (int t = 0; t < (XO ? 1 : NDT); ++t) lds_tr_lane_offs<D / 8, SW>(t * 32, tro_[t], tro2_[t]);
 #pragma unroll
-  for (int st = 0; st < NKS; ++st) rdo[st] = swz_off<D / 8, SW>(l32, 2 * st + g);
+  for (int st = 0; st < (XO ? 1 : NKS); ++st) rdo_[st] = swz_off<D / 8, SW>(l32, 2 * st + g);
+  auto tro = [&](int t) { return XO ? tro_[0] ^ (t * 32) : tro_[t]; };
+  auto tro2 = [&](int t) { return XO ? (tro_[0] ^ (t * 32)) + 8 * D : tro2_[t]; };
+  auto rdo = [&](int st) { return XO ? rdo_[0] ^ (st * 16) : rdo_[st]; };
   const bf16x8 ones = seed_ones(g);
   // one 64-row query tile in buffer buf (a compile-time index, so that every LDS operand
   // address is a lane offset plus an immediate); DIAG: the tile holding this wave's keys
   // (causal mask)
   auto tile = [&](auto bufc, const bool DIAG) __attribute__((always_inline)) {
     const int buf = bufc;
-#pragma unroll
+#pragma unroll(NW == 8 ? 1 : 2)
     for (int mt = 0; mt < 2; ++mt) {
       if (DIAG && mt * 32 + 31 < kloc - l32) continue;  // rows all above this wave's keys
       // the per-row terms enter through the matrix cores: a rank-3 product with `ones`
@@ -207,15 +219,18 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
       {
         bf16x8 qa[NKS];
 #pragma unroll
-        for (int st = 0; st < NKS_A; ++st) qa[st] = ld8(sm.q[buf] + rdo[st] + mt * 32 * D);
+        for (int st = 0; st < (XO ? 0 : NKS_A); ++st) qa[st] = ld8(sm.q[buf] + rdo(st) + mt * 32 * D);
         // (lanes 32..63 read the same row: they meet the zero rows of `ones`)
         f32x16 sc = mfma32(ld8(&sm.seed[buf][mt * 32 + l32][0]), ones, zero16());
 #pragma unroll
-        for (int st = 0; st < NKS_A; ++st) sc = mfma32(qa[st], kb[st], sc);
+        for (int st = 0; st < NKS_A; ++st) {
+          sc = mfma32(XO ? ld8(sm.q[buf] + rdo(st) + mt * 32 * D) : qa[st], kb[st], sc);
+          if (XO && (st & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // at most four operands in flight
+        }
         if constexpr (F32) {
 #pragma unroll
           for (int st = 0; st < NKS_A; ++st) {
-            const bf16x8 qal = ld8(sm.ql[buf] + rdo[st] + mt * 32 * D);
+            const bf16x8 qal = ld8(sm.ql[buf] + rdo(st) + mt * 32 * D);
             sc = mfma32(qa[st], kbl[st], sc);
             sc = mfma32(qal, kb[st], sc);
             sc = mfma32(qal, kbl[st], sc);
@@ -232,31 +247,34 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
       }
 #pragma unroll
       for (int t = 0; t < NDT_A; ++t) {
-        const bf16x8 o0 = lds_tr_a_at2<D / 8>(sm.dO[buf], tro[t], tro2[t], mt * 32);
-        const bf16x8 o1 = lds_tr_a_at2<D / 8>(sm.dO[buf], tro[t], tro2[t], mt * 32 + 16);
+        const bf16x8 o0 = lds_tr_a_at2<D / 8>(sm.dO[buf], tro(t), tro2(t), mt * 32);
+        const bf16x8 o1 = lds_tr_a_at2<D / 8>(sm.dO[buf], tro(t), tro2(t), mt * 32 + 16);
         adv[t] = mfma32(o0, pb0, adv[t]);
         adv[t] = mfma32(o1, pb1, adv[t]);
         if constexpr (F32) {
           adv[t] = mfma32(o0, pack_lo(pv, 0, pb0), adv[t]);
           adv[t] = mfma32(o1, pack_lo(pv, 1, pb1), adv[t]);
-          adv[t] = mfma32(lds_tr_a_at2<D / 8>(sm.dOl[buf], tro[t], tro2[t], mt * 32), pb0, adv[t]);
-          adv[t] = mfma32(lds_tr_a_at2<D / 8>(sm.dOl[buf], tro[t], tro2[t], mt * 32 + 16), pb1, adv[t]);
+          adv[t] = mfma32(lds_tr_a_at2<D / 8>(sm.dOl[buf], tro(t), tro2(t), mt * 32), pb0, adv[t]);
+          adv[t] = mfma32(lds_tr_a_at2<D / 8>(sm.dOl[buf], tro(t), tro2(t), mt * 32 + 16), pb1, adv[t]);
         }
       }
       f32x16 ds;
       {
         bf16x8 da[NKS];
 #pragma unroll
-        for (int st = 0; st < NKS_A; ++st) da[st] = ld8(sm.dO[buf] + rdo[st] + mt * 32 * D);
+        for (int st = 0; st < (XO ? 0 : NKS_A); ++st) da[st] = ld8(sm.dO[buf] + rdo(st) + mt * 32 * D);
         // dP - delta: the accumulator starts at -delta (stored negated)
         f32x16 dp = mfma32(ld8(&sm.seed[buf][mt * 32 + l32][8]), ones, zero16());
 #pragma unroll
-        for (int st = 0; st < NKS_A; ++st) dp = mfma32(da[st], vb[st], dp);
+        for (int st = 0; st < NKS_A; ++st) {
+          dp = mfma32(XO ? ld8(sm.dO[buf] + rdo(st) + mt * 32 * D) : da[st], vb[st], dp);
+          if (XO && (st & 1)) __builtin_amdgcn_sched_barrier(0);  // two: P is live beside dP
+        }
         if constexpr (F32) {
 #pragma unroll
           for (int st = 0; st < NKS_A; ++st) {
             dp = mfma32(da[st], vbl[st], dp);
-            dp = mfma32(ld8(sm.dOl[buf] + rdo[st] + mt * 32 * D), vb[st], dp);
+            dp = mfma32(ld8(sm.dOl[buf] + rdo(st) + mt * 32 * D), vb[st], dp);
           }
         }
 #pragma unroll
@@ -266,15 +284,15 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
       }
 #pragma unroll
       for (int t = 0; t < NDT_A; ++t) {
-        const bf16x8 q0 = lds_tr_a_at2<D / 8>(sm.q[buf], tro[t], tro2[t], mt * 32);
-        const bf16x8 q1 = lds_tr_a_at2<D / 8>(sm.q[buf], tro[t], tro2[t], mt * 32 + 16);
+        const bf16x8 q0 = lds_tr_a_at2<D / 8>(sm.q[buf], tro(t), tro2(t), mt * 32);
+        const bf16x8 q1 = lds_tr_a_at2<D / 8>(sm.q[buf], tro(t), tro2(t), mt * 32 + 16);
         adk[t] = mfma32(q0, pb0, adk[t]);
         adk[t] = mfma32(q1, pb1, adk[t]);
         if constexpr (F32) {
           adk[t] = mfma32(q0, pack_lo(ds, 0, pb0), adk[t]);
           adk[t] = mfma32(q1, pack_lo(ds, 1, pb1), adk[t]);
-          adk[t] = mfma32(lds_tr_a_at2<D / 8>(sm.ql[buf], tro[t], tro2[t], mt * 32), pb0, adk[t]);
-          adk[t] = mfma32(lds_tr_a_at2<D / 8>(sm.ql[buf], tro[t], tro2[t], mt * 32 + 16), pb1, adk[t]);
+          adk[t] = mfma32(lds_tr_a_at2<D / 8>(sm.ql[buf], tro(t), tro2(t), mt * 32), pb0, adk[t]);
+          adk[t] = mfma32(lds_tr_a_at2<D / 8>(sm.ql[buf], tro(t), tro2(t), mt * 32 + 16), pb1, adk[t]);
         }
       }
     }
@@ -296,6 +314,7 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(D == 64 && !F32) void lucid
       if (s + 2 < nsteps) step(std::integral_constant<int, 2>{}, s + 2);
     }
   }
+  if (NW > 4 && jw >= T) return;
   // the first share of a block writes dV' and dK themselves, the others their partial sums
   const int64_t nel = (int64_t)BH * T * D;
   float* ov = (sp == 0 ? dvp : part + (int64_t)(2 * sp - 2) * nel) + ((int64_t)bh * T + jrow) * D;

@@ -154,10 +154,11 @@ struct BwdWs {
 // slots finish together.  A share keeps at least eight 64-row steps in the longest block, so
 // that its start and its partial sums stay small beside its sweep.  B1 Hq32 Hkv4 T16000 d64
 // (500 blocks on 512 slots): 3.92 ms in one share, 2.58 in two, 2.52 in three (with the
-// sum of the partials, 0.02), 2.48 in eight; B1 Hq32 Hkv8 T8192 d128 (512 blocks on 256 slots)
-// 1.57 ms in one, 1.58 in two, 1.72 in eight.
+// sum of the partials, 0.02), 2.48 in eight; B1 Hq32 Hkv8 T8192
+// d128 (256 blocks of 256 keys on 256 slots): 1.40 ms in two.
 int dkdv_splits(int BH, int G, int T, int D, bool f32) {
-  const int64_t jobs = (int64_t)BH * (T / 128), slots = padded_dim(D) == 64 && !f32 ? 512 : 256;
+  const bool wide = padded_dim(D) == 128 && !f32;  // 256 keys a workgroup, else 128
+  const int64_t jobs = (int64_t)BH * (wide ? (T + 255) / 256 : T / 128), slots = padded_dim(D) == 64 && !f32 ? 512 : 256;
   const int64_t want = (2 * slots + jobs - 1) / jobs, most = (int64_t)G * (T / 64) / 8;
   const int64_t ns = want < most ? want : most;
   return ns < 1 ? 1 : ns < 8 ? (int)ns : 8;
@@ -378,8 +379,9 @@ int launch_attn_bwd(const void* dout, const int64_t* dos, const void* q, const i
   const int nsp = dkdv_splits(BH, Hq / Hkv, T, D, false);
   auto sweeps = [&](auto dac) -> int {
     constexpr int DA = decltype(dac)::value;
-    LUCID_LAUNCH("lucid_attn_bwd_dkdv_kernel", (lucid::lucid_attn_bwd_dkdv_kernel<D, false, DA>),
-                 dim3((T / 128) * BH * nsp), st, (const bf16*)q, S(qs), (const bf16*)k, S(ks), f.vpb,
+    constexpr int NW = D == 128 ? 8 : 4;
+    LUCID_LAUNCH_B("lucid_attn_bwd_dkdv_kernel", (lucid::lucid_attn_bwd_dkdv_kernel<D, false, DA, NW>),
+                   dim3((T + 32 * NW - 1) / (32 * NW) * BH * nsp), dim3(64 * NW), st, (const bf16*)q, S(qs), (const bf16*)k, S(ks), f.vpb,
                  (const bf16*)dout, S(dos), w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH, scale, lucid::Lo{}, nullptr, nsp,
                  w.dkdv);
     if (nsp > 1)
