@@ -147,24 +147,35 @@ struct BwdWs {
   size_t bytes;
 };
 
-// Shares that the dK/dV' sweep of a 128-key column block is cut into.  The blocks of a
+// The dK/dV' sweep of bf16 operands at head dim 128 takes 256 keys a workgroup (eight waves)
+// instead of 128 (four) where that is faster: at up to 96 columns, whose instances stay within
+// 256 registers, from T = 1024 (B4 H8 d96 T1024 42.4 -> 39.4 us, B1 Hq32 Hkv4 d96 T8192 3657 ->
+// 3279 us a training pass; a block of 128 rows leaves half of the waves idle: 14.2 -> 17.8 us);
+// at 128 columns, where they spill, in long sweeps (training passes of B1 Hq32 Hkv8: T2048 kernel
+// 116 -> 129 us, T8192 4318 -> 4202 us, T32768 56.7 -> 55.0 ms).
+bool dkdv_wide(int D, int T, bool f32) { return !f32 && D > 64 && T >= (D <= 96 ? 1024 : 8192); }
+
+// Shares that the dK/dV' sweep of a column block is cut into.  The blocks of a
 // causal sweep are as long as G (T - key) / 64 steps, so a launch of at most one block per
 // resident workgroup takes as long as the longest block, twice the mean; with twice as many
 // workgroups as slots (two per CU for bf16 at 64 columns, else one), longest first, the
 // slots finish together.  A share keeps at least eight 64-row steps in the longest block, so
 // that its start and its partial sums stay small beside its sweep.  B1 Hq32 Hkv4 T16000 d64
 // (500 blocks on 512 slots): 3.92 ms in one share, 2.58 in two, 2.52 in three (with the
-// sum of the partials, 0.02), 2.48 in eight; B1 Hq32 Hkv8 T8192
-// d128 (256 blocks of 256 keys on 256 slots): 1.40 ms in two.
-int dkdv_splits(int BH, int G, int T, int D, bool f32) {
-  const bool wide = padded_dim(D) == 128 && !f32;  // 256 keys a workgroup, else 128
-  const int64_t jobs = (int64_t)BH * (wide ? (T + 255) / 256 : T / 128), slots = padded_dim(D) == 64 && !f32 ? 512 : 256;
+// sum of the partials, 0.02), 2.48 in eight; B1 Hq32 Hkv8 T8192 d128 (512 blocks of 128 keys on
+// 256 slots) 1.57 ms in one, 1.58 in two, 1.72 in eight.
+int dkdv_splits(int BH, int Hq, int Hkv, int T, int D, bool f32) {
+  if (BH < 1 || Hkv < 1 || T < 128) return 1;  // (workspace queries take any sizes)
+  const int G = Hq / Hkv;
+  const int64_t jobs = (int64_t)BH * (dkdv_wide(D, T, f32) ? (T + 255) / 256 : T / 128);
+  const int64_t slots = padded_dim(D) == 64 && !f32 ? 512 : 256;
   const int64_t want = (2 * slots + jobs - 1) / jobs, most = (int64_t)G * (T / 64) / 8;
   const int64_t ns = want < most ? want : most;
   return ns < 1 ? 1 : ns < 8 ? (int)ns : 8;
 }
 
 BwdWs carve_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = false) {
+  const int nsp = dkdv_splits(B * Hkv, Hq, Hkv, T, D, f32);
   D = padded_dim(D);
   const size_t BH = (size_t)B * Hkv, BHq = (size_t)B * Hq;
   BwdWs w{};
@@ -189,7 +200,7 @@ BwdWs carve_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = fal
     w.doh = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
     w.dol = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
   }
-  w.dkdv = reinterpret_cast<float*>(take((dkdv_splits(B * Hkv, Hq / Hkv, T, D, f32) - 1) * 2 * BH * T * D * 4));
+  w.dkdv = reinterpret_cast<float*>(take((size_t)(nsp - 1) * 2 * BH * T * D * 4));
   w.bytes = off;
   return w;
 }
@@ -376,14 +387,23 @@ int launch_attn_bwd(const void* dout, const int64_t* dos, const void* q, const i
   // operands need the registers).  DA: the active head-dim columns (zero-padded rows of a smaller head dim)
   constexpr int RW = D == 128 ? 32 : 64;
   constexpr int XWGR = D == 128 ? 128 : 256;
-  const int nsp = dkdv_splits(BH, Hq / Hkv, T, D, false);
+  const int nsp = dkdv_splits(BH, Hq, Hkv, T, (int)dn, false);
   auto sweeps = [&](auto dac) -> int {
     constexpr int DA = decltype(dac)::value;
-    constexpr int NW = D == 128 ? 8 : 4;
-    LUCID_LAUNCH_B("lucid_attn_bwd_dkdv_kernel", (lucid::lucid_attn_bwd_dkdv_kernel<D, false, DA, NW>),
-                   dim3((T + 32 * NW - 1) / (32 * NW) * BH * nsp), dim3(64 * NW), st, (const bf16*)q, S(qs), (const bf16*)k, S(ks), f.vpb,
-                 (const bf16*)dout, S(dos), w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH, scale, lucid::Lo{}, nullptr, nsp,
-                 w.dkdv);
+    auto dkdv = [&](auto nwc) -> int {
+      constexpr int NW = decltype(nwc)::value;
+      LUCID_LAUNCH_B("lucid_attn_bwd_dkdv_kernel", (lucid::lucid_attn_bwd_dkdv_kernel<D, false, DA, NW>),
+                     dim3((T + 32 * NW - 1) / (32 * NW) * BH * nsp), dim3(64 * NW), st, (const bf16*)q, S(qs),
+                     (const bf16*)k, S(ks), f.vpb, (const bf16*)dout, S(dos), w.seeds, w.dvp, w.dka, Hq, Hkv, T, BH,
+                     scale, lucid::Lo{}, nullptr, nsp, w.dkdv);
+      return LUCID_OK;
+    };
+    int rc;
+    if constexpr (D == 128)
+      rc = dkdv_wide((int)dn, T, false) ? dkdv(std::integral_constant<int, 8>{}) : dkdv(std::integral_constant<int, 4>{});
+    else
+      rc = dkdv(std::integral_constant<int, 4>{});
+    if (rc) return rc;
     if (nsp > 1)
       LUCID_LAUNCH("lucid_dkdv_sum_kernel", lucid::lucid_dkdv_sum_kernel, dim3(((int64_t)BH * T * D / 4 + 255) / 256, 2),
                    st, w.dvp, w.dka, w.dkdv, nsp, (int64_t)BH * T * D / 4);
@@ -508,6 +528,7 @@ FwdWs carve_attn_vp(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 =
 // preconditioner part dV' (as fp32), dV and its lo part, the column sums and counters.
 // (f32 with attn: the bf16 pair of dO as well.)
 BwdWs carve_seam_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool attn, bool f32 = false) {
+  const int nsp = dkdv_splits(B * Hkv, Hq, Hkv, T, D, f32);
   D = padded_dim(D);
   const size_t BH = (size_t)B * Hkv, BHq = (size_t)B * Hq;
   BwdWs w{};
@@ -527,7 +548,7 @@ BwdWs carve_seam_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool attn
       w.doh = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
       w.dol = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
     }
-    w.dkdv = reinterpret_cast<float*>(take((dkdv_splits(B * Hkv, Hq / Hkv, T, D, f32) - 1) * 2 * BH * T * D * 4));
+    w.dkdv = reinterpret_cast<float*>(take((size_t)(nsp - 1) * 2 * BH * T * D * 4));
   } else {
     w.dvb = reinterpret_cast<bf16*>(take(BH * T * D * 2));
     w.dvbl = reinterpret_cast<bf16*>(take(BH * T * D * 2));
@@ -728,7 +749,7 @@ int launch_attn_bwd_f32(const void* dout, const int64_t* dos, const void* o, con
   // head dim 128: four waves of 32 rows for dQ (128 rows per workgroup, one wave per SIMD),
   // so that the hi/lo operands of a wave stay in registers
   constexpr int RW = D == 128 ? 32 : 64, WGR = D == 128 ? 128 : 256;
-  const int nsp = dkdv_splits(BH, Hq / Hkv, T, D, true);
+  const int nsp = dkdv_splits(BH, Hq, Hkv, T, (int)dn, true);
   const dim3 gsum(((int64_t)BH * T * D / 4 + 255) / 256, 2), gkv((T / 128) * BH * nsp), gq(((T + WGR - 1) / WGR) * BHq), bq(64 * (WGR / RW));
   if constexpr (D == 128) {
     const int da = active_dims<D>(dn);

@@ -68,3 +68,11 @@ def test_split_column_sweep_of_the_attention_seam(vp_dtype):
     (torch.softmax(s, -1) @ vr).transpose(1, 2).backward(do.double())
     for n, x, r in (("dq", q, qr), ("dk", k, kr), ("dvp", vp, vr)):
         check(n, (x.grad.double() - r.grad).abs().max().item(), r.grad.abs().max().item())
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T,d", [(1, 4, 2, 1152, 96), (1, 3, 1, 1024, 80), (2, 2, 2, 1408, 68),
+                                          (1, 2, 1, 8320, 128), (1, 1, 1, 8192, 100)])
+def test_256_key_column_blocks(B, Hq, Hkv, T, d):
+    """Head dims above 64 at the lengths of the eight-wave sweep, with and without half a block at
+    the end (T an odd multiple of 128)."""
+    test_split_column_sweep(B, Hq, Hkv, T, d, torch.bfloat16)
