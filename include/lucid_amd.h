@@ -75,7 +75,8 @@ int lucid_get_precision(void);
 /* Forward kernel schedule for the calls that follow on the calling thread (thread-local;
  * no counterpart in the reference).  On (default): at head dim <= 64 with one query head per kv head, the
  * preconditioner chain and the causal attention of each 128-row block run in one fused
- * kernel (lucid_fused_fwd_kernel) that feeds every staged key tile to both; off: the chain
+ * kernel (lucid_fused_fwd_kernel) that feeds every staged key tile to both, at the sizes where
+ * that is faster (short sequences, and many heads beside their length); off: always the chain
  * kernel, then the attention kernel.  Both give the same O, V' and lse up to the rounding
  * order of the attention's online softmax.  Any nonzero value means on. */
 int lucid_set_fused_forward(int on);

@@ -83,7 +83,8 @@ __global__ __launch_bounds__(256) void lucid_bwd_prep_kernel(const bf16* __restr
 
 // ---------------------------------------------------------------------------
 // Column sweep for the attention part.  Workgroup = 128 keys of one kv head (256, NW = 8
-// waves, in the bf16 instance at head dim 128 for the sizes of dkdv_wide), wave w owns keys 32w..32w+31 (one n-tile, lane <-> key j); sweeps the G query
+// waves, in the bf16 instance at head dim 128 for the sizes of dkdv_wide), wave w owns keys
+// 32w..32w+31 (one n-tile, lane <-> key j); sweeps the G query
 // heads of the group and every 64-row query tile at or below the diagonal.
 // Each query tile (Q and dO rows, lse2, delta) is staged once per workgroup in
 // LDS by direct global->LDS loads (three buffers, two tiles ahead, swizzled);

@@ -249,6 +249,8 @@ lucid::Strides S(const int64_t* s) { return lucid::Strides{s[0], s[1], s[2]}; }
 //     (8, 65536) 41823/40999, (32, 4096) 541/629, (32, 8192) 1545/1541, (32, 16384) 5468/4985
 //   backward at 64, against 256 columns: (16, 1024) 166/188, (32, 4096) 701/843, (16, 16384) 3921/4031,
 //     (16, 32768) 14535/14460, (32, 32768) 30392/29882, (8, 65536) 29477/29962
+// (taken before the others' operands were written through: 3 % off the fused kernel at (64, 4096),
+// nothing off the 256-column chain at (16, 32768))
 bool linked_fwd64(int64_t BH, int64_t T) {
   return T >= 2048 && (BH <= 8 || (BH <= 16 && T <= 8192) || T >= 1536 * BH);
 }

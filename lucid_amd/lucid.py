@@ -296,7 +296,8 @@ def set_fused_forward(on: bool = True) -> None:
 
     On (default): at head dim <= 64 with one query head per kv head the preconditioner chain
     and the causal attention of each 128-row block run in one fused kernel that feeds every
-    staged key tile to both; off: the chain kernel, then the attention kernel.  The results
+    staged key tile to both, at the sizes where that is faster (short sequences, and many heads
+    beside their length); off: always the chain kernel, then the attention kernel.  The results
     agree up to the rounding order of the attention's online softmax.
     """
     lib = _lib.load()
