@@ -28,8 +28,7 @@ constexpr float DEC_NEG = -1e30f;  // finite "minus infinity" for empty softmax 
 // arrays hold the 8 tokens of its smallest group.  NCT = 2 (groups of 4 and 8, calls of more
 // tokens than one tile takes): one read of the cache and one combine for twice the tokens, at
 // one wave per SIMD at head dim 128 (B8 Hq32 Hkv4 d68, 2900 rows, 5 tokens: two passes of
-// 24 + 13 us, 74.8 us a call; one pass 28 + 13, 44.6; Hq32 Hkv8 d128, 128K rows, 12 tokens
-// 311 -> 217 us).
+// 24 + 13 us, 74.8 us a call, 59.1 in one; Hq32 Hkv8 d128, 128K rows, 12 tokens 311 -> 271 us).
 template <int G, int NCT>
 constexpr int decode_tokens_per_pass() {
   return G > 0 ? 32 * NCT / (G + 1) : 8;
