@@ -22,7 +22,8 @@
  * the inputs (dout included) and written zero in the outputs; the dot products are
  * unchanged and the RMS of k_norm divides by D itself (the attention sweeps of D in
  * 65 .. 96 leave out the columns beyond 80 or 96, whose products are zero).  Workspace
- * sizes take D and are those of Dp.
+ * sizes take D and are those of Dp; those of the attention and its seams never fall as B or T
+ * grows, so one buffer made for the largest batch and the longest sequence serves the others.
  */
 #ifndef LUCID_AMD_H
 #define LUCID_AMD_H

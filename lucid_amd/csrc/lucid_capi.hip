@@ -143,7 +143,8 @@ struct BwdWs {
   bf16* link;    // [BH][T/128][2][128][128] -X_p^T P_{p+1,p}^T, likewise
   int* counters; // [BH]
   bf16 *doh, *dol; // fp32 inputs only: the bf16 pair of dO ([BHq][T][D] rows)
-  float* dkdv;   // [2 (dkdv_splits - 1)][BH][T][D] partial dV' and dK of a split column sweep
+  float* dkdv;   // [2 (dkdv_splits - 1)][BH][T][D] partial dV' and dK of a split column sweep, within
+                 // dkdv_part_bytes; in carve_bwd in the bytes of dvb .. link, which are written later
   size_t bytes;
 };
 
@@ -164,20 +165,33 @@ bool dkdv_wide(int D, int T, bool f32) { return !f32 && D > 64 && T >= (D <= 96 
 // (500 blocks on 512 slots): 3.92 ms in one share, 2.58 in two, 2.52 in three (with the
 // sum of the partials, 0.02), 2.48 in eight; B1 Hq32 Hkv8 T8192 d128 (512 blocks of 128 keys on
 // 256 slots) 1.57 ms in one, 1.58 in two, 1.72 in eight.
+int64_t dkdv_slots(int D, bool f32) { return padded_dim(D) == 64 && !f32 ? 512 : 256; }
+int64_t dkdv_most_splits(int Hq, int Hkv, int T) {
+  const int64_t n = (int64_t)(Hq / Hkv) * (T / 64) / 8;
+  return n < 1 ? 1 : n < 8 ? n : 8;
+}
 int dkdv_splits(int BH, int Hq, int Hkv, int T, int D, bool f32) {
-  if (BH < 1 || Hkv < 1 || T < 128) return 1;  // (workspace queries take any sizes)
-  const int G = Hq / Hkv;
   const int64_t jobs = (int64_t)BH * (dkdv_wide(D, T, f32) ? (T + 255) / 256 : T / 128);
-  const int64_t slots = padded_dim(D) == 64 && !f32 ? 512 : 256;
-  const int64_t want = (2 * slots + jobs - 1) / jobs, most = (int64_t)G * (T / 64) / 8;
-  const int64_t ns = want < most ? want : most;
-  return ns < 1 ? 1 : ns < 8 ? (int)ns : 8;
+  const int64_t want = (2 * dkdv_slots(D, f32) + jobs - 1) / jobs, most = dkdv_most_splits(Hq, Hkv, T);
+  return (int)(want < most ? want : most);
+}
+
+// Bytes kept for a split sweep's partial sums.  Sizes are those of the padded head dim, and a
+// workspace sized for the longest sequence and the largest batch serves the shorter and
+// smaller, while the shares fall in steps as the blocks grow in number: so this is a bound for
+// every D of one padded dim that never falls as B or T grows.  ns - 1 < 2 slots / jobs and a
+// block takes at most 128 (256: dkdv_wide) rows, so (ns - 1) BH T < 2 slots rows a block.
+size_t dkdv_part_bytes(int BH, int Hq, int Hkv, int T, int D, bool f32) {
+  if (BH < 1 || Hkv < 1 || T < 128) return 0;  // (workspace queries take any sizes)
+  const int64_t rows = (dkdv_most_splits(Hq, Hkv, T) - 1) * BH * T;
+  const int64_t most = 2 * dkdv_slots(D, f32) * (padded_dim(D) == 128 && !f32 ? 256 : 128);
+  return (size_t)(rows < most ? rows : most) * 2 * padded_dim(D) * 4;
 }
 
 BwdWs carve_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = false) {
-  const int nsp = dkdv_splits(B * Hkv, Hq, Hkv, T, D, f32);
   D = padded_dim(D);
   const size_t BH = (size_t)B * Hkv, BHq = (size_t)B * Hq;
+  const size_t parts = dkdv_part_bytes(B * Hkv, Hq, Hkv, T, D, f32);
   BwdWs w{};
   size_t off = 0;
   char* p = static_cast<char*>(base);
@@ -190,17 +204,19 @@ BwdWs carve_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 = fal
   w.seeds = reinterpret_cast<bf16*>(take(BHq * T * 32));
   w.dvp = reinterpret_cast<float*>(take(BH * T * D * 4));
   w.dka = reinterpret_cast<float*>(take(BH * T * D * 4));
+  const size_t chain = off;
+  w.dkdv = reinterpret_cast<float*>(take(0));
   w.dvb = reinterpret_cast<bf16*>(take(BH * T * D * 2));
   w.dvbl = reinterpret_cast<bf16*>(take(BH * T * D * 2));
   w.colsum = reinterpret_cast<float*>(take(BH * T * D * 4));
   w.xt = reinterpret_cast<bf16*>(take(BH * (T / 128) * 32768 * 2));
   w.link = reinterpret_cast<bf16*>(take(BH * (T / 128) * 32768 * 2));
+  if (off - chain < parts) take(parts - (off - chain));
   w.counters = reinterpret_cast<int*>(take(BH * 4));
   if (f32) {
     w.doh = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
     w.dol = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
   }
-  w.dkdv = reinterpret_cast<float*>(take((size_t)(nsp - 1) * 2 * BH * T * D * 4));
   w.bytes = off;
   return w;
 }
@@ -530,9 +546,9 @@ FwdWs carve_attn_vp(void* base, int B, int Hq, int Hkv, int T, int D, bool f32 =
 // preconditioner part dV' (as fp32), dV and its lo part, the column sums and counters.
 // (f32 with attn: the bf16 pair of dO as well.)
 BwdWs carve_seam_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool attn, bool f32 = false) {
-  const int nsp = dkdv_splits(B * Hkv, Hq, Hkv, T, D, f32);
   D = padded_dim(D);
   const size_t BH = (size_t)B * Hkv, BHq = (size_t)B * Hq;
+  const size_t parts = dkdv_part_bytes(B * Hkv, Hq, Hkv, T, D, f32);
   BwdWs w{};
   size_t off = 0;
   char* p = static_cast<char*>(base);
@@ -550,7 +566,7 @@ BwdWs carve_seam_bwd(void* base, int B, int Hq, int Hkv, int T, int D, bool attn
       w.doh = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
       w.dol = reinterpret_cast<bf16*>(take(BHq * T * D * 2));
     }
-    w.dkdv = reinterpret_cast<float*>(take((size_t)(nsp - 1) * 2 * BH * T * D * 4));
+    w.dkdv = reinterpret_cast<float*>(take(parts));
   } else {
     w.dvb = reinterpret_cast<bf16*>(take(BH * T * D * 2));
     w.dvbl = reinterpret_cast<bf16*>(take(BH * T * D * 2));
