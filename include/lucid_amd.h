@@ -145,7 +145,8 @@ int lucid_attn_bwd(const void* dout, const int64_t* do_strides, const void* q, c
  * bf16 pairs (hi + lo) through split MFMA products and every head runs the exact chain
  * instances, so the results are within ~1e-4 relative of an fp64 evaluation.  The forward
  * workspace (lucid_fwd_f32_workspace_bytes) holds the split copies of Q and K and must stay
- * alive until lucid_attn_bwd_f32; the backward reads o as written by the forward. */
+ * alive until lucid_attn_bwd_f32; the backward reads o as written by the forward.  vprime may be
+ * v itself (contiguous rows of Dp), here and in the fp32 solves below: V' then replaces V. */
 size_t lucid_fwd_f32_workspace_bytes(int B, int Hq, int Hkv, int T, int D);
 size_t lucid_bwd_f32_workspace_bytes(int B, int Hq, int Hkv, int T, int D);
 int lucid_attn_fwd_f32(const float* q, const int64_t* q_strides, const float* k, const int64_t* k_strides,

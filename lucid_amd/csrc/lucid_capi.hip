@@ -288,9 +288,8 @@ int launch_precond_fwd(const void* k, const int64_t* ks, const void* v, const in
   // the 256-row chain keeps its own in-block coupling; only the exact heads read links then
   const bool wide = D == 128 && !linked_fwd128(BH, T);
   LUCID_LAUNCH("lucid_link_kernel", (lucid::lucid_link_kernel<D, false, false>), dim3(T / 128, BH), st,
-               (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, vprime, w.vpbl, w.khat,
-               nullptr, nullptr, w.mass, wide,
-               lucid::Lo{});
+               (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, w.vpt, w.vptl, w.vpbl,
+               w.khat, nullptr, nullptr, w.mass, wide, lucid::Lo{});
   // both instances of the chain: each solves the heads of its precision and returns at
   // once for the others
   if (g_precision != LUCID_PRECISION_EXACT) {
@@ -370,9 +369,8 @@ int launch_fwd(const void* q, const int64_t* qs, const void* k, const int64_t* k
       if (g_precision != LUCID_PRECISION_FAST) {
         // heads of the exact chains: their chain, then their attention (skip_fast)
         LUCID_LAUNCH("lucid_link_kernel", (lucid::lucid_link_kernel<D, false, false>), dim3(T / 128, BH), st,
-                     (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, vprime, w.vpbl, w.khat,
-                     nullptr, nullptr, w.mass, 1,
-                     lucid::Lo{});
+                     (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, w.vpt, w.vptl,
+                     w.vpbl, w.khat, nullptr, nullptr, w.mass, 1, lucid::Lo{});
         LUCID_LAUNCH("lucid_precond_fwd_exact_kernel", (lucid::lucid_precond_fwd_kernel<D, true>),
                      dim3((T / 128) * BH), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH, w.rinv,
                      w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.mass, w.counters,
@@ -456,7 +454,7 @@ int launch_precond_bwd(const void* k, const int64_t* ks, const FwdWs& f, void* d
   const bool wide = D == 64 && !linked_bwd64(BH, T);
   LUCID_LAUNCH("lucid_link_bwd_kernel", (lucid::lucid_link_kernel<D, false, true>), dim3(T / 128, BH), st, (const bf16*)k,
                S(ks), Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, nullptr, nullptr,
-               nullptr, w.xt, w.link, f.mass, wide, lucid::Lo{});
+               nullptr, nullptr, w.xt, w.link, f.mass, wide, lucid::Lo{});
   if (wide) {
     LUCID_LAUNCH_B("lucid_precond_bwd_col_wide_kernel", lucid::lucid_precond_bwd_col_wide_kernel<64>,
                    dim3((T / 256) * BH), dim3(512), st, (const bf16*)k, S(ks), Hkv, T, BH, f.rinv, f.khat, scale,
@@ -689,8 +687,8 @@ int launch_precond_fwd_f32(const void* k, const int64_t* ks, const void* v, cons
   LUCID_LAUNCH("lucid_zx_f32_kernel", (lucid::lucid_zx_kernel<D, true>), dim3(T / 128, BH), st, w.kh, ck, Hkv, T,
                w.rinv, scale, w.pinv, w.zx, lo);
   LUCID_LAUNCH("lucid_link_f32_kernel", (lucid::lucid_link_kernel<D, true, false>), dim3(T / 128, BH), st, w.kh, ck,
-               Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, vprime, w.vpbl, w.khat,
-               nullptr, nullptr, w.mass, 0, lo);
+               Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, w.vpt, w.vptl, w.vpbl, w.khat, nullptr,
+               nullptr, w.mass, 0, lo);
   // the chain reads V as fp32 through lo.v with V's own strides (its bf16 operand is unused)
   LUCID_LAUNCH("lucid_precond_fwd_f32_kernel", (lucid::lucid_precond_fwd_kernel<D, true, true>),
                dim3((T / 128) * BH), st, w.kh, ck, (const bf16*)v, S(vs), Hkv, T, BH, w.rinv, w.khat, scale, vprime,
@@ -811,8 +809,8 @@ int launch_precond_bwd_f32(const FwdWs& f, void* dk, const int64_t* dks, void* d
   lo.k = f.kl;
   lo.kt = f.ktl;
   LUCID_LAUNCH("lucid_link_bwd_f32_kernel", (lucid::lucid_link_kernel<D, true, true>), dim3(T / 128, BH), st, f.kh, ck,
-               Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, nullptr, nullptr, nullptr, w.xt,
-               w.link, f.mass, 0, lo);
+               Hkv, T, f.rinv, scale, f.pinv, f.zx, nullptr, nullptr, nullptr, nullptr, nullptr,
+               w.xt, w.link, f.mass, 0, lo);
   auto col_chain = [&](auto dac) -> int {  // over the active head-dim columns
     LUCID_LAUNCH("lucid_precond_bwd_col_f32_kernel",
                  (lucid::lucid_precond_bwd_col_kernel<D, true, true, decltype(dac)::value>), dim3((T / 128) * BH), st,

@@ -541,9 +541,10 @@ __global__ __launch_bounds__(256) void lucid_zx_kernel(const bf16* __restrict__ 
 // E(k, m) = exp(s r_k r_m K_k.K_m - 1/s) (fp32 inputs: all four hi/lo terms).  link and xt are
 // bf16 hi / lo planes [128 rows][128 columns in T-perm order] (the lo plane of a link only for
 // exact heads).  The forward's links take no workspace of their own: row n of block i's hi
-// plane lies in V' row n of the block (vp32), the halves of its lo row in rows n of vpbl and of
-// khat (which the exact chains do not read), and y in olo; block i's workgroup reads them before
-// it, alone, writes V' and its lo part there, and the attention writes olo later still.  The products of exact heads are fp32
+// plane lies where the block's columns of V'^T will (link_row), the halves of its lo row in rows
+// n of vpbl and of khat (which the exact chains do not read), and y in olo; block i's workgroup
+// reads them before it, alone, writes V' and its lo part there, and the attention writes olo
+// later still.  (Not in the caller's vprime, which an fp32 solve in place reads as V.)  The products of exact heads are fp32
 // MFMAs (bf16 chains: 3-term bf16 splits): along a shared key direction X takes differences of nearly equal rows of E, which
 // 16-bit operands would leave only part of (largest V' error of the fp32 path at T = 1024: 9.9e-4
 // with the splits, 6.2e-4 with fp32 products, 6.5e-4 in a chain without links).  Bound by its
@@ -552,12 +553,19 @@ __global__ __launch_bounds__(256) void lucid_zx_kernel(const bf16* __restrict__ 
 // 16 values are the operands of 16 two-deep steps); Xop is shared through LDS.  exact_only: heads of the bf16 chains return at once
 // (their chain does not read the links).  grid (T/128, B*Hkv)
 // ---------------------------------------------------------------------------
+// row n of the hi plane of a forward link: the block's 128 columns (256 bytes, T-perm) of V'^T row
+// n, at head dim 64 of its lo part's row n - 64 from n = 64 on
+template <int D, typename P>
+__device__ __forceinline__ P* link_row(P* vpt, P* vptl, int bh, int T, int blk, int n) {
+  return (n < D ? vpt : vptl) + ((int64_t)bh * D + (n & (D - 1))) * T + blk * 128;
+}
+
 template <int D, bool F32, bool BWD>
 __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_link_kernel(
     const bf16* __restrict__ k, Strides ks, int Hkv, int T, const float* __restrict__ rinv, float scale,
-    const float* __restrict__ pinv, const float* __restrict__ zx, float* __restrict__ y, float* __restrict__ vp32,
-    bf16* __restrict__ vpbl, bf16* __restrict__ khat, bf16* __restrict__ xt, bf16* __restrict__ link,
-    const float* __restrict__ mass, int exact_only, Lo lo) {
+    const float* __restrict__ pinv, const float* __restrict__ zx, float* __restrict__ y, bf16* __restrict__ vpt,
+    bf16* __restrict__ vptl, bf16* __restrict__ vpbl, bf16* __restrict__ khat, bf16* __restrict__ xt,
+    bf16* __restrict__ link, const float* __restrict__ mass, int exact_only, Lo lo) {
   constexpr int NKS = D / 16;
   __shared__ __attribute__((aligned(16))) union {
     float XAt[64][68];  // XAt[c][slot of a] = X_A[a][c]
@@ -732,7 +740,7 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_link_kerne
       const int n = 32 * nt + l32, m = 32 * w + 16 * hh + 8 * g;
       const int64_t row = (int64_t)bh * T + blk * 128 + n;
       const bf16x8 oh = pack_b(o, hh);
-      bf16* dh = BWD ? link + ob + n * 128 + m : reinterpret_cast<bf16*>(vp32 + row * D) + m;
+      bf16* dh = (BWD ? link + ob + n * 128 : link_row<D>(vpt, vptl, bh, T, blk, n)) + m;
       *reinterpret_cast<bf16x8*>(dh) = oh;
       if (exact) {
         bf16* dl = BWD ? dh + 16384 : (m < 64 ? vpbl : khat) + row * D + (m & 63);
@@ -1138,7 +1146,7 @@ __global__ __launch_bounds__(64 * NW) LUCID_TWO_WAVES_IF((D == 64 || NW == 8) &&
   }
   if (i2 > 0) {  // the link's rows before the wait, V'^T of the previous block after it
     const int64_t lrow = ((int64_t)bh * T + i0 + 32 * wr + l32) * D;
-    const bf16* lhi = reinterpret_cast<const bf16*>(vp32 + lrow) + 8 * g;
+    const bf16* lhi = link_row<D>(vpt, vptl, bh, T, i2, 32 * wr + l32) + 8 * g;
     bf16x8 zh[8], zl[8];
 #pragma unroll
     for (int st = 0; st < 8; ++st) {
