@@ -1706,6 +1706,7 @@ int lucid_pad_rows(int n, const void* const* src, const int64_t* strides, const 
     return fail("lucid_pad_rows: 1 to 3 tensors, dtype LUCID_DTYPE_BF16 or LUCID_DTYPE_F32");
   if (B <= 0 || T <= 0 || Tp < T || d <= 0 || dp < d || dp % 8)
     return fail("lucid_pad_rows: B, T, d positive, Tp >= T, dp >= d and a multiple of 8");
+  if (!src || !strides || !H || !dst) return fail("lucid_pad_rows: src, strides, H and dst must be non-null");
   const int es = dtype == LUCID_DTYPE_F32 ? 4 : 2;
   lucid::PadTensors p{};
   int most = 0;
