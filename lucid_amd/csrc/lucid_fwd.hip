@@ -460,14 +460,17 @@ __global__ __launch_bounds__(256) void lucid_mass_kernel(const bf16* __restrict_
 // T-perm order so that the chain can add zx V'_A straight from its bf16 V'_A tile.
 // wave -> 32x32 quadrant.  grid (T/128, B*Hkv)
 // ---------------------------------------------------------------------------
-template <int D, bool F32 = false>
-__global__ __launch_bounds__(256) void lucid_zx_kernel(const bf16* __restrict__ k, Strides ks, int Hkv, int T,
-                                                       const float* __restrict__ rinv, float scale,
-                                                       const float* __restrict__ pinv, float* __restrict__ zx, Lo lo,
-                                                       float* __restrict__ mass = nullptr) {
+struct ZxSmem {
+  float Xb[64][68];
+  float PT[64][68];  // PT[c][m] = P_BA[m][c]
+};
+template <int D, bool F32>
+__device__ __forceinline__ void zx_block(const bf16* __restrict__ k, Strides ks, int Hkv, int T,
+                                         const float* __restrict__ rinv, float scale, const float* __restrict__ pinv,
+                                         float* zx, Lo lo, ZxSmem& sm) {
   constexpr int NKS = D / 16;
-  __shared__ __attribute__((aligned(16))) float Xb[64][68];
-  __shared__ __attribute__((aligned(16))) float PT[64][68];  // PT[c][m] = P_BA[m][c]
+  auto& Xb = sm.Xb;
+  auto& PT = sm.PT;
   const int blk = blockIdx.x, bh = blockIdx.y;
   const int b = bh / Hkv, h = bh - b * Hkv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -519,12 +522,20 @@ __global__ __launch_bounds__(256) void lucid_zx_kernel(const bf16* __restrict__ 
   float* zo = zx + ((int64_t)bh * (T / 128) + blk) * 4096 + slot;
 #pragma unroll
   for (int e = 0; e < 16; ++e) zo[(tm * 32 + drow(e, g)) * 64] = -z[e];
-  if constexpr (!F32) {
-    if (mass) {  // the row masses of the two 64-row blocks (one launch less than lucid_mass_kernel)
-      row_mass_block<D>(k, ks, Hkv, T, rinv, scale, mass, 2 * blk, bh);
-      __syncthreads();
-      row_mass_block<D>(k, ks, Hkv, T, rinv, scale, mass, 2 * blk + 1, bh);
-    }
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void lucid_zx_kernel(const bf16* __restrict__ k, Strides ks, int Hkv, int T,
+                                                       const float* __restrict__ rinv, float scale,
+                                                       const float* __restrict__ pinv, float* __restrict__ zx,
+                                                       float* __restrict__ mass) {
+  __shared__ __attribute__((aligned(16))) ZxSmem sm;
+  zx_block<D, false>(k, ks, Hkv, T, rinv, scale, pinv, zx, Lo{}, sm);
+  if (mass) {  // the row masses of the two 64-row blocks (one launch less than lucid_mass_kernel)
+    const int blk = blockIdx.x, bh = blockIdx.y;
+    row_mass_block<D>(k, ks, Hkv, T, rinv, scale, mass, 2 * blk, bh);
+    __syncthreads();
+    row_mass_block<D>(k, ks, Hkv, T, rinv, scale, mass, 2 * blk + 1, bh);
   }
 }
 
@@ -560,17 +571,17 @@ __device__ __forceinline__ P* link_row(P* vpt, P* vptl, int bh, int T, int blk, 
   return (n < D ? vpt : vptl) + ((int64_t)bh * D + (n & (D - 1))) * T + blk * 128;
 }
 
+union LinkSmem {
+  float XAt[64][68];  // XAt[c][slot of a] = X_A[a][c]
+  float x[128][132];  // Xop rows n, columns k
+};
 template <int D, bool F32, bool BWD>
-__global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_link_kernel(
+__device__ __forceinline__ void link_block(
     const bf16* __restrict__ k, Strides ks, int Hkv, int T, const float* __restrict__ rinv, float scale,
-    const float* __restrict__ pinv, const float* __restrict__ zx, float* __restrict__ y, bf16* __restrict__ vpt,
+    const float* __restrict__ pinv, const float* zx, float* __restrict__ y, bf16* __restrict__ vpt,
     bf16* __restrict__ vptl, bf16* __restrict__ vpbl, bf16* __restrict__ khat, bf16* __restrict__ xt,
-    bf16* __restrict__ link, const float* __restrict__ mass, int exact_only, Lo lo) {
+    bf16* __restrict__ link, const float* __restrict__ mass, int exact_only, Lo lo, LinkSmem& sm) {
   constexpr int NKS = D / 16;
-  __shared__ __attribute__((aligned(16))) union {
-    float XAt[64][68];  // XAt[c][slot of a] = X_A[a][c]
-    float x[128][132];  // Xop rows n, columns k
-  } sm;
   const int blk = blockIdx.x, bh = blockIdx.y, nblk = T / 128;
   if (exact_only && !(mass[bh] > kExactMass)) return;
   const int b = bh / Hkv, h = bh - b * Hkv;
@@ -748,6 +759,49 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_link_kerne
       }
     }
   }
+}
+
+template <int D, bool F32, bool BWD>
+__global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_link_kernel(
+    const bf16* __restrict__ k, Strides ks, int Hkv, int T, const float* __restrict__ rinv, float scale,
+    const float* __restrict__ pinv, const float* __restrict__ zx, float* __restrict__ y, bf16* __restrict__ vpt,
+    bf16* __restrict__ vptl, bf16* __restrict__ vpbl, bf16* __restrict__ khat, bf16* __restrict__ xt,
+    bf16* __restrict__ link, const float* __restrict__ mass, int exact_only, Lo lo) {
+  __shared__ __attribute__((aligned(16))) LinkSmem sm;
+  link_block<D, F32, BWD>(k, ks, Hkv, T, rinv, scale, pinv, zx, y, vpt, vptl, vpbl, khat, xt, link, mass, exact_only,
+                          lo, sm);
+}
+
+// The in-block coupling and the forward link of a block in one launch, where no link waits for
+// the head masses: a precision that is forced (mass then holds it already; mass_out null), fp32
+// inputs, or a single block, which has no link (its mass goes to mass_out as in lucid_zx_kernel).
+// zx is read back within the workgroup that wrote it.  grid (T/128, B*Hkv)
+template <int D, bool F32>
+__global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_zx_link_kernel(
+    const bf16* __restrict__ k, Strides ks, int Hkv, int T, const float* __restrict__ rinv, float scale,
+    const float* __restrict__ pinv, float* zx, float* __restrict__ y, bf16* __restrict__ vpt,
+    bf16* __restrict__ vptl, bf16* __restrict__ vpbl, bf16* __restrict__ khat, const float* mass, float* mass_out,
+    int exact_only, Lo lo) {
+  __shared__ __attribute__((aligned(16))) union {
+    ZxSmem zx;
+    LinkSmem link;
+  } sm;
+  zx_block<D, F32>(k, ks, Hkv, T, rinv, scale, pinv, zx, lo, sm.zx);
+  if constexpr (!F32) {
+    if (mass_out) {
+      const int blk = blockIdx.x, bh = blockIdx.y;
+      row_mass_block<D>(k, ks, Hkv, T, rinv, scale, mass_out, 2 * blk, bh);
+      __syncthreads();
+      row_mass_block<D>(k, ks, Hkv, T, rinv, scale, mass_out, 2 * blk + 1, bh);
+      __builtin_amdgcn_s_waitcnt(0);  // the head's only block: its mass is final once the atomics are done
+      __syncthreads();
+      if (exact_only && !(__hip_atomic_load(mass_out + bh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > kExactMass))
+        return;
+    }
+  }
+  __syncthreads();
+  link_block<D, F32, false>(k, ks, Hkv, T, rinv, scale, pinv, zx, y, vpt, vptl, vpbl, khat, nullptr, nullptr, mass, 0,
+                            lo, sm.link);  // (a forced precision: every head that gets here)
 }
 
 // ---------------------------------------------------------------------------
