@@ -277,24 +277,27 @@ bool linked_bwd64(int64_t BH, int64_t T) { return T % 256 != 0 || BH < 16 || BH 
 // of the forward chains: of every head, or (links = false) of the exact heads alone.  One launch
 // where the links need not wait for the masses; the second one's start and first latency are
 // 1 to 3 us of a short forward (B1 H8 T128 d64 bf16 45.5 -> 42.0 us, Hq32 Hkv8 T128 d128 60.8 -> 59.7,
-// H8 d64 fp32 T128 62.5 -> 60.0, T512 116.6 -> 114).
+// H8 d64 fp32 T128 62.5 -> 60.0, T512 116.6 -> 114).  links_due: launch_links is still to come (the
+// fused forward puts it behind its own kernel: 233 us at B4 H16 T2048 d64, 240 before it).
 template <int D>
 int launch_couplings(const void* k, const int64_t* ks, const FwdWs& w, int Hkv, int T, int BH, float scale, bool links,
-                     hipStream_t st) {
+                     bool* links_due, hipStream_t st) {
   float* mass = g_precision == LUCID_PRECISION_AUTO ? w.mass : nullptr;
-  if (!mass && !links && g_precision == LUCID_PRECISION_FAST) {
+  *links_due = mass && T > 128;
+  if (*links_due || (!links && g_precision == LUCID_PRECISION_FAST)) {
     LUCID_LAUNCH("lucid_zx_kernel", lucid::lucid_zx_kernel<D>, dim3(T / 128, BH), st, (const bf16*)k, S(ks), Hkv, T,
-                 w.rinv, scale, w.pinv, w.zx, nullptr);
-    return LUCID_OK;
-  }
-  if (!mass || T == 128) {
+                 w.rinv, scale, w.pinv, w.zx, mass);
+  } else {
     LUCID_LAUNCH("lucid_zx_link_kernel", (lucid::lucid_zx_link_kernel<D, false>), dim3(T / 128, BH), st,
                  (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, w.vpt, w.vptl, w.vpbl, w.khat,
                  w.mass, mass, !links, lucid::Lo{});
-    return LUCID_OK;
   }
-  LUCID_LAUNCH("lucid_zx_kernel", lucid::lucid_zx_kernel<D>, dim3(T / 128, BH), st, (const bf16*)k, S(ks), Hkv, T,
-               w.rinv, scale, w.pinv, w.zx, mass);
+  return LUCID_OK;
+}
+
+template <int D>
+int launch_links(const void* k, const int64_t* ks, const FwdWs& w, int Hkv, int T, int BH, float scale, bool links,
+                 hipStream_t st) {
   LUCID_LAUNCH("lucid_link_kernel", (lucid::lucid_link_kernel<D, false, false>), dim3(T / 128, BH), st,
                (const bf16*)k, S(ks), Hkv, T, w.rinv, scale, w.pinv, w.zx, w.y, w.vpt, w.vptl, w.vpbl, w.khat,
                nullptr, nullptr, w.mass, !links, lucid::Lo{});
@@ -312,7 +315,10 @@ int launch_precond_fwd(const void* k, const int64_t* ks, const void* v, const in
                w.khat);
   // the 256-row chain keeps its own in-block coupling; only the exact heads read links then
   const bool wide = D == 128 && !linked_fwd128(BH, T);
-  if (int rc = launch_couplings<D>(k, ks, w, Hkv, T, BH, scale, !wide, st)) return rc;
+  bool links_due;
+  if (int rc = launch_couplings<D>(k, ks, w, Hkv, T, BH, scale, !wide, &links_due, st)) return rc;
+  if (links_due)
+    if (int rc = launch_links<D>(k, ks, w, Hkv, T, BH, scale, !wide, st)) return rc;
   // both instances of the chain: each solves the heads of its precision and returns at
   // once for the others
   if (g_precision != LUCID_PRECISION_EXACT) {
@@ -383,13 +389,16 @@ int launch_fwd(const void* q, const int64_t* qs, const void* k, const int64_t* k
       LUCID_LAUNCH("lucid_prep_kernel", lucid::lucid_prep_kernel<D>, dim3(T / 64, BH), st, (const bf16*)k, S(ks),
                    Hkv, T, eps, dn, scale, w.rinv, w.kt, w.pinv, w.counters, w.mass, mass_init, lucid::Lo{}, nullptr,
                    w.khat);
-      if (int rc = launch_couplings<D>(k, ks, w, Hkv, T, BH, scale, false, st)) return rc;
+      bool links_due;
+      if (int rc = launch_couplings<D>(k, ks, w, Hkv, T, BH, scale, false, &links_due, st)) return rc;
       if (g_precision != LUCID_PRECISION_EXACT)
         LUCID_LAUNCH("lucid_fused_fwd_kernel", lucid::lucid_fused_fwd_kernel<D>, dim3((T / 128) * BH), st,
                      (const bf16*)q, S(qs), (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH, w.rinv, scale,
                      vprime, w.vpb, w.vpt, w.pinv, w.zx, w.mass, w.counters, (bf16*)o, S(os), lse);
       if (g_precision != LUCID_PRECISION_FAST) {
-        // heads of the exact chains: their chain, then their attention (skip_fast)
+        // heads of the exact chains: their links and chain, then their attention (skip_fast)
+        if (links_due)
+          if (int rc = launch_links<D>(k, ks, w, Hkv, T, BH, scale, false, st)) return rc;
         LUCID_LAUNCH("lucid_precond_fwd_exact_kernel", (lucid::lucid_precond_fwd_kernel<D, true>),
                      dim3((T / 128) * BH), st, (const bf16*)k, S(ks), (const bf16*)v, S(vs), Hkv, T, BH, w.rinv,
                      w.khat, scale, vprime, w.vpb, w.vpt, w.vpbl, w.vptl, w.pinv, w.y, w.mass, w.counters,

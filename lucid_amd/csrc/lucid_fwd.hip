@@ -467,7 +467,7 @@ struct ZxSmem {
 template <int D, bool F32>
 __device__ __forceinline__ void zx_block(const bf16* __restrict__ k, Strides ks, int Hkv, int T,
                                          const float* __restrict__ rinv, float scale, const float* __restrict__ pinv,
-                                         float* zx, Lo lo, ZxSmem& sm) {
+                                         float* __restrict__ zx, Lo lo, ZxSmem& sm) {
   constexpr int NKS = D / 16;
   auto& Xb = sm.Xb;
   auto& PT = sm.PT;
