@@ -153,7 +153,10 @@ struct BwdWs {
 // 256 registers, from T = 1024 (B4 H8 d96 T1024 42.4 -> 39.4 us, B1 Hq32 Hkv4 d96 T8192 3657 ->
 // 3279 us a training pass; a block of 128 rows leaves half of the waves idle: 14.2 -> 17.8 us);
 // at 128 columns, where they spill, in long sweeps (training passes of B1 Hq32 Hkv8: T2048 kernel
-// 116 -> 129 us, T8192 4318 -> 4202 us, T32768 56.7 -> 55.0 ms).
+// 116 -> 129 us, T8192 4318 -> 4202 us, T32768 56.7 -> 55.0 ms).  Backwards of the attention alone,
+// four waves against eight, us: 96 columns B1 Hq32 Hkv4 T1536 168/185, T3072 376/337, B4 Hq32 Hkv8
+// T1536 469/429, B8 H16 T1024 339/302; 128 columns B1 Hq32 Hkv8 T4096 626/643, T6016 1350/1309,
+// T8192 2277/2236, B1 H16 T6016 725/755, T8192 1181/1159.
 bool dkdv_wide(int D, int T, bool f32) { return !f32 && D > 64 && T >= (D <= 96 ? 1024 : 8192); }
 
 // Shares that the dK/dV' sweep of a column block is cut into.  The blocks of a
@@ -257,21 +260,28 @@ lucid::Strides S(const int64_t* s) { return lucid::Strides{s[0], s[1], s[2]}; }
 // 10.4 us (its hand-off carries the attention's last pair) but shares its operand reads between
 // the chain and the attention, and the 256-row chains 20-25 us per 256 rows but stage a tile
 // per 256.  So the links win where a head has few others beside it, up to a length where the
-// sweeps outweigh the hand-offs.  Measured on one MI355X, us, links against the other (BH, T):
-//   forward at head dim 64, against the fused kernel: (4, 1024) 101/96, (4, 2048) 151/157, (8, 8192) 477/557,
-//     (8, 32768) 2660/3021, (16, 1024) 112/102, (16, 4096) 298/320, (16, 8192) 592/610, (16, 16384) 1494/1444,
-//     (16, 24576) 3003/3161, (16, 32768) 5094/5334, (32, 4096) 391/383, (32, 16384) 2974/2880, (64, 2048) 277/253
-//   forward at 128, against 256 rows: (8, 8192) 925/1230, (8, 32768) 10691/11285, (8, 49152) 24239/24258,
-//     (8, 65536) 41823/40999, (32, 4096) 541/629, (32, 8192) 1545/1541, (32, 16384) 5468/4985
-//   backward at 64, against 256 columns: (16, 1024) 166/188, (32, 4096) 701/843, (16, 16384) 3921/4031,
-//     (16, 32768) 14535/14460, (32, 32768) 30392/29882, (8, 65536) 29477/29962
-// (taken before the others' operands were written through: 3 % off the fused kernel at (64, 4096),
-// nothing off the 256-column chain at (16, 32768))
+// sweeps outweigh the hand-offs (the more heads, the sooner), and from a few blocks on: their
+// own launch costs more than one or two hand-offs.  Measured on one MI355X, us, links against
+// the other (BH, T):
+//   forward at head dim 64, against the fused kernel: (4, 1024) 100/94, (4, 2048) 149/153, (8, 1536) 129/125,
+//     (8, 2048) 156/157, (8, 8192) 475/539, (8, 32768) 2603/2750, (16, 2048) 167/168, (16, 8192) 594/601,
+//     (16, 12288) 960/919, (16, 16384) 1469/1438, (16, 24576) 2883/2920, (16, 32768) 4986/5413,
+//     (32, 4096) 392/371, (32, 16384) 2714/2636, (64, 2048) 274/241
+//   forward at 128, against 256 rows: (8, 256) 79/69, (8, 512) 98/96, (8, 768) 114/123, (8, 8192) 612/913,
+//     (8, 32768) 4757/4994, (16, 16384) 2575/2635, (16, 24576) 5497/5228, (32, 768) 130/136, (32, 6144) 981/1022,
+//     (32, 8192) 1522/1474, (48, 2048) 317/333, (64, 1024) 185/188, (64, 2048) 385/376, (64, 4096) 981/882, (128, 1024) 316/262
+//   backward of the solve at 64, against 256 columns: (8, 8192) 476/725, (8, 32768) 3861/4165, (16, 1024) 107/121,
+//     (16, 16384) 2065/2172, (16, 32768) 7865/7900, (32, 4096) 411/454, (32, 8192) 1172/1193, (32, 12288) 2342/2302,
+//     (64, 1536) 205/207, (64, 2048) 279/270, (64, 4096) 718/669, (128, 512) 108/94, (128, 2048) 509/422
 bool linked_fwd64(int64_t BH, int64_t T) {
   return T >= 2048 && (BH <= 8 || (BH <= 16 && T <= 8192) || T >= 1536 * BH);
 }
-bool linked_fwd128(int64_t BH, int64_t T) { return T % 256 != 0 || BH * T <= 8 * 49152; }
-bool linked_bwd64(int64_t BH, int64_t T) { return T % 256 != 0 || BH < 16 || BH * T < 16 * 32768; }
+bool linked_fwd128(int64_t BH, int64_t T) {
+  return T % 256 != 0 || (T >= 768 && BH * T <= 4096 * (84 - (BH < 16 ? 16 : BH)));
+}
+bool linked_bwd64(int64_t BH, int64_t T) {
+  return T % 256 != 0 || BH < 16 || BH * T <= (BH == 16 ? 16 * 24576 : 5120 * (84 - BH));
+}
 
 // The in-block coupling of every 128-row chain block, (AUTO) the heads' row masses, and the links
 // of the forward chains: of every head, or (links = false) of the exact heads alone.  One launch
