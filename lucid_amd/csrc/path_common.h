@@ -337,12 +337,6 @@ __device__ __forceinline__ void dl_store(float (*S)[68], const f32x16& x, int mo
     S[r][cl] = keep ? x[e] : 0.f;
   }
 }
-__device__ __forceinline__ f32x16 dl_load(const float (*S)[68]) {
-  const int cl = dl_col();
-  f32x16 x;
-  DL_FOR_E x[e] = S[dl_row(e)][cl];
-  return x;
-}
 // 64 x 64 block of an fp32 row-major matrix (row stride ld) into an LDS block, and back
 __device__ __forceinline__ void load_blk(float (*dst)[68], const float* __restrict__ src, int ld) {
   for (int idx = threadIdx.x; idx < 1024; idx += 256) {
