@@ -599,7 +599,7 @@ def main():
         "dtype": "f32" if wl in ("path_f32", "ref_f32") else "bf16",
         "data": "synthetic (seeded N(0,1)/sqrt(d) q,k,v; N(0,1) dO)" if not path_kind
                 else "synthetic (seeded N(0,1) q,k,v,w; w L2-normalised; beta=2 sigmoid(N(0,1)); N(0,1) dO)",
-        "precision": args.precision, "keys": args.keys, "fused_forward": not args.no_fused_fwd,
+        "precision": args.precision, "keys": args.keys, "fused_forward": "lucid_fused_fwd_kernel" in kernels,
         "config": {"workload": {"lucid": "lucid_attention_fwd_bwd", "c2": "lucid_attention_fwd_bwd",
                                 "c5": "lucid_attention_fwd", "gqa128": "lucid_attention_fwd_bwd",
                                 "ref_f32": "lucid_attention_fwd_bwd", "ref_bf16": "lucid_attention_fwd_bwd",
