@@ -294,7 +294,10 @@ size_t lucid_decode_tokens_workspace_bytes(int B, int Hq, int Hkv, int L, int T_
  * Each token's V' row is the exact prefill row: it is coupled to the cached rows and to
  * the earlier new tokens, v'_t = (v_t - sum_{j<t} P_tj v'_j) / P_tt, and each token
  * attends to the cache and to the new tokens up to itself.  The tokens run in passes of
- * 32 / (Hq/Hkv + 1) (the columns of one score tile), each pass reading the caches once.
+ * 32 / (g + 1), the columns of one score tile, g the query heads per kv head (of a chunk, where
+ * more than 31 are cut into equal chunks); with g = 4 or 8 and more tokens than that, of
+ * 64 / (g + 1) on two tiles.  Each pass reads the caches once.  The workspace follows the tokens
+ * of a pass, and so L.
  * Replaces LucidAttention.get_new_v_prime for L_k new tokens (modeling_lucid.py:576-598,
  * which couples a new token to the cache only) and the cached attention call
  * (:475-496).  lucid_decode is this entry with L = 1. */

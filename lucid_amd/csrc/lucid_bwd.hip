@@ -605,7 +605,8 @@ __global__ __launch_bounds__(64 * (WGR / RW)) LUCID_TWO_WAVES_IF(EXACT ? D == 64
 // Chained transposed solve dV = P^-T dV' (Lucid_Tril_Solver.backward :328-334)
 // and the column sums C_J = sum_{I >= J} M_IJ^T K^_I, M = (dV V'^T) * P.
 // Workgroup = 128 columns J0 .. J0+127 (block p).
-// id -> (p = NP-1 - id/BH, bh = id % BH): ids grow as p falls, so a workgroup
+// id -> block p = NP-1 - id / n of head number id % n of the instance's n heads
+// (InstanceHeads): ids grow as p falls, so a workgroup
 // waits only on later blocks held by lower ids.  counters[bh] = n means the
 // last n 64-blocks of dV are published.
 // wave w owns columns J0 + 32w .. +32 (one n-tile, lane <-> column) and sweeps

@@ -806,10 +806,11 @@ __global__ __launch_bounds__(256) LUCID_TWO_WAVES_IF(true) void lucid_zx_link_ke
 
 // ---------------------------------------------------------------------------
 // Chained preconditioner solve, 128 rows per workgroup (two 64-row sub-blocks A and B).
-// Workgroup id -> (i2 = id / BH, bh = id % BH): ids grow with i2, so every
-// wait is on a lower id (in-order dispatch keeps the chain deadlock free) and
-// the blocks of one head share an XCD when BH % 8 == 0.  counters[bh] = number
-// of 64-row blocks of V' already published (whole 128-row blocks at a time).
+// The n heads of the instance are numbered densely (InstanceHeads): workgroup id -> block
+// i2 = id / n of its head number id % n.  Ids grow with i2, so every wait is on a lower id
+// (in-order dispatch keeps the chain deadlock free), and the blocks of one head share an XCD
+// when n % 8 == 0.  counters[bh] = number of 64-row blocks of V' already published (whole
+// 128-row blocks at a time).
 //
 // The earlier keys but for the previous block are swept in pairs of 64-key tiles (128 keys
 // per barrier): K^ rows (bf16, the bf16 chains; raw K rows and 1/rms, the exact ones) and

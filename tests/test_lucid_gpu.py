@@ -51,7 +51,7 @@ CASES = [
     (1, 2, 2, 256, 64, 1.0),
     (2, 4, 2, 384, 64, 1.0),
     (1, 2, 1, 200, 128, 1.0),
-    (1, 4, 2, 768, 128, None),    # d = 128 chain over 256-row workgroups with earlier pairs
+    (1, 4, 2, 768, 128, None),    # d = 128, linked chain with earlier pairs, T a multiple of 256
     (1, 2, 1, 640, 128, 1.0),     # d = 128, T not a multiple of 256 (128-row workgroups)
 ]
 
@@ -210,8 +210,8 @@ def _correlated_keys(T, D, g, noise=0.1):
 def test_auto_precision_picks_exact_for_correlated_heads(D):
     """AUTO: a head whose keys share a direction (row mass ~T) runs the exact chains, a head of
     N(0,1)-like keys the bf16 ones; the sampled mass agrees with the exact row mass
-    max_i sum_{j<i} P_ij^2 of the float64 oracle, and both heads meet the parity bars.  At
-    head dim 128 the two instances are the 256-row bf16 chain and the exact chain."""
+    max_i sum_{j<i} P_ij^2 of the float64 oracle, and both heads meet the parity bars.  (The
+    256-row bf16 chain beside the exact one: test_short_launches_gpu.)"""
     from lucid_amd import lucid
     B, Hq, Hkv, T = 1, 2, 2, 1024
     g = torch.Generator().manual_seed(21)
@@ -239,7 +239,7 @@ def test_auto_precision_picks_exact_for_correlated_heads(D):
 @pytest.mark.parametrize("B,H,T,qk_std", [(1, 2, 128, None), (2, 2, 640, None), (1, 3, 1024, 1.0)])
 def test_fused_forward_matches_two_kernel_forward(B, H, T, qk_std):
     """The fused forward (chain and attention of each 128-row block in one kernel; the default
-    at head dim 64 with Hq == Hkv) against the two-kernel sequence on the same inputs: O, V'
+    at head dim 64 with Hq == Hkv at these lengths) against the two-kernel sequence on the same inputs: O, V'
     and every gradient agree to rounding order, and both meet the oracle bars.  T = 128 is a
     single block (no earlier pair), T = 640 an odd number of blocks."""
     from lucid_amd import get_fused_forward, lucid_attention, set_fused_forward
