@@ -142,7 +142,7 @@ def cpu_baseline(T=32768, H_full=16, D=64):
     One head at the full sequence length (fwd + bwd through autograd: dense P,
     solve_triangular, SDPA), times the head count -- all 16 heads at once need 64 GiB of
     fp32 P alone.  Threads: every core this process may run on, capped by OMP_NUM_THREADS
-    where the host sets it (the GPU box's CPU share).  One untimed warm-up at T=1024; the
+    where the host sets it (its share of the CPUs).  One untimed warm-up at T=1024; the
     median of three runs, or one run when it takes over 20 s.
     """
     import statistics
